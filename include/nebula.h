@@ -210,7 +210,7 @@ int nbl_material_destroy(nbl_material* m);
 
 /* gpu_driver ctor (drivers/gpu/gpu_driver.inl:51-89).  capacity = target
  * number of particles in flight; steps_per_launch = steps each particle takes
- * per kernel launch.  The driver keeps its own copies of geometry and
+ * per kernel launch (more when few are in flight, nbl_driver_set_cascade).  The driver keeps its own copies of geometry and
  * material descriptors (the objects must outlive it). */
 int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* geom,
 	const nbl_material* const* mats, int32_t n_mats, uint32_t physics_flags,
@@ -245,9 +245,10 @@ int nbl_driver_iterate(nbl_driver* d, uint32_t n_iter);
  * record per scattering event (elastic or inelastic, not a boundary) that
  * changes the electron's energy: position after the event, energy before
  * it, energy lost, tag of the primary, stream id of the electron.  Enable
- * before tracking; every iteration can write up to (K + 1) records per
- * particle in flight, so drain after every nbl_driver_iterate call (a drain
- * that finds records were dropped returns NBL_ERR_CAPACITY). */
+ * before tracking; an iteration can write up to (K + 1) records per
+ * particle in flight (half the buffer, if it is the only one since a drain
+ * and few particles are in flight), so drain after every nbl_driver_iterate
+ * call (a drain that finds records were dropped returns NBL_ERR_CAPACITY). */
 typedef struct {
 	float pos[3];
 	float energy;
@@ -264,6 +265,12 @@ int nbl_driver_drain_deposits(nbl_driver* d, nbl_deposit* out, uint64_t cap, uin
  * for (<= capacity; the reference's batch sizing, gpu_main.cu:167-175). */
 int nbl_driver_set_launch(nbl_driver* d, uint32_t steps_per_launch, uint32_t blocks_per_cu,
 	uint32_t target);
+
+/* Few particles in flight: an iteration that starts with at most
+ * `max_particles` keeps them and their secondaries in their waves for 64 to
+ * 1024 steps instead of steps_per_launch (default and maximum: 1024 per
+ * compute unit; 0: never).  Results do not depend on it. */
+int nbl_driver_set_cascade(nbl_driver* d, uint32_t max_particles);
 
 /* Replay each nbl_driver_iterate(d, n > 1) from a captured hipGraph of n
  * iterations (captured once per n and launch configuration). */

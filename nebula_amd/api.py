@@ -413,6 +413,11 @@ def to_particles(pri: np.ndarray) -> np.ndarray:
 RECORD_SINK = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint64)
 
 
+# run_tally shortens its frames to two iterations at this many particles:
+# the library then takes them 64 to 1024 steps on in each (k_cascade)
+FEW_PARTICLES = 1 << 18
+
+
 class Driver:
     """gpu_driver<scatter_physics<true>, intersect_t, octree<true>>
     (drivers/gpu/gpu_driver.h:56-178), run by libnebula.so."""
@@ -478,6 +483,11 @@ class Driver:
 
     def set_graph(self, enable: bool) -> None:
         check(lib().nbl_driver_set_graph(self._h, int(bool(enable))))
+
+    def set_cascade(self, max_particles: int) -> None:
+        """Particles in flight up to which an iteration takes them 64 to 1024
+        steps on in their waves (0: never; results do not depend on it)."""
+        check(lib().nbl_driver_set_cascade(self._h, max_particles))
 
     def autotune(self, iters_per_trial: int = 4) -> dict:
         """Measured search over the launch configuration on the queued work;
@@ -566,7 +576,8 @@ class Driver:
         """Track everything pushed to the end without keeping the records:
         counts[bin, 0] = detected electrons below `se_cutoff` eV (SE) and
         counts[bin, 1] = the others (BSE), binned by tag_bin[tag].  The
-        detected buffer is drained after every `frame` iterations; with
+        detected buffer is drained after every `frame` iterations (fewer
+        once few particles are left); with
         progress_s > 0 a progress line goes to stderr that often.
 
         adapt_k: follow the best steps per launch as the run goes on.  The
@@ -597,15 +608,19 @@ class Driver:
                     self.set_launch(k, self.launch["blocks_per_cu"], self.launch["target"])
             k_now = self.launch["steps_per_launch"]
             self.k_frames[k_now] = self.k_frames.get(k_now, 0) + 1
-            self.do_iteration(frame)
+            # with few particles left an iteration takes them many steps on
+            self.do_iteration(frame if left > FEW_PARTICLES else min(frame, 2))
             return time.perf_counter()
 
         # Each frame's records are drained as soon as it ends and the next
         # frame is enqueued before they are tallied, so the host's tally
         # overlaps the GPU's next frame.
+        running, _, queued = self.counts()
+        left = running + queued
         t0 = launch_frame()
         while True:
             running, det, queued = self.counts()
+            left = running + queued
             dt = time.perf_counter() - t0
             st = self.steps()
             if adapt_k:

@@ -74,6 +74,7 @@ struct Ctrl {
 	uint32_t target;        // particles in flight to aim for
 	uint32_t spill_n;       // secondaries parked on the spill stack
 	uint32_t spill_take, spill_src;  // refill from the spill stack
+	uint32_t few;           // the coming launch runs in k_cascade, not k_step
 	uint64_t refill_src;
 	uint64_t queue_n, queue_next;
 	// Counters that waves of the step kernels bump atomically.  Each sits on
@@ -250,7 +251,8 @@ __device__ __forceinline__ void wave_alloc2(uint64_t* ctr, bool want_a, bool wan
 // Adopt the previous launch's output and plan the refill from the queue.
 // Secondaries that found no room in the particle buffer wait on the spill
 // stack; they are taken back (newest first) before any new primary.
-__global__ void k_ctrl(Ctrl* c, uint32_t slots, uint32_t spill_cap)
+__global__ void k_ctrl(Ctrl* c, uint32_t slots, uint32_t spill_cap, uint32_t few_max, uint32_t waves,
+	uint32_t dep_half)
 {
 	if (threadIdx.x != 0 || blockIdx.x != 0)
 		return;
@@ -278,6 +280,10 @@ __global__ void k_ctrl(Ctrl* c, uint32_t slots, uint32_t spill_cap)
 	c->queue_next += m;
 	c->n_surv += take + m;
 	c->se_limit = slots - (c->n_surv + c->n_se);
+	// with deposits, k_cascade writes the first half of their buffer and
+	// needs room for a step of each of its waves
+	const uint32_t n = c->n_surv + c->n_se;
+	c->few = (few_max && n <= few_max && (uint64_t)c->dep_ctr + 64ull * min(n, waves) <= dep_half) ? 1u : 0u;
 	c->step_out = 0;
 	c->se_ctr = 0;
 	c->spill_ctr = c->spill_n;
@@ -598,6 +604,24 @@ __device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, co
 // holding another world's particle wait, unchanged, for a later launch.
 // Trajectories depend only on each particle's own stream, so which launch
 // steps a particle changes no result.
+// World `ww` (wave-uniform) through the constant address space: scalar
+// loads, so the world's geometry and materials sit in SGPRs as the plain
+// kernel's arguments do (not in VGPRs).
+__device__ __forceinline__ void load_world(const StepArgs& a, uint32_t ww, World& W)
+{
+	static_assert(sizeof(WorldDesc) % 4 == 0, "world descriptor in words");
+	using CWord = const __attribute__((address_space(4))) uint32_t;
+	CWord* src = (CWord*)(a.worlds + ww);
+	WorldDesc wd;
+	uint32_t* dst = reinterpret_cast<uint32_t*>(&wd);
+#pragma unroll
+	for (int k = 0; k < (int)(sizeof(WorldDesc) / 4); ++k)
+		dst[k] = src[k];
+	W.g = wd.g;
+	W.mats = wd.mats;
+	W.nmats = wd.nmats;
+}
+
 template <bool SC, bool MULTI, bool WUNI = false>
 __device__ __forceinline__ void step_body(const StepArgs& a)
 {
@@ -605,6 +629,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	// energy deposits are recorded by the general variants only
 	constexpr bool DEP_OK = SC || MULTI;
 	Ctrl* C = a.ctrl;
+	if (C->few)
+		return;   // k_cascade takes this launch
 	const uint32_t bi = C->buf_in;
 	const Bufs in = bi ? a.buf[1] : a.buf[0];
 	const Bufs out = bi ? a.buf[0] : a.buf[1];
@@ -673,20 +699,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 			// world, w0 < n_in): its world is the wave's, and no lane holds
 			// another world's particle
 			const uint32_t ww = __builtin_amdgcn_readfirstlane(s.flags >> FL_WORLD_SHIFT);
-			// through the constant address space: scalar loads, so the
-			// world's geometry and materials sit in SGPRs as the plain
-			// kernel's arguments do (not in VGPRs)
-			static_assert(sizeof(WorldDesc) % 4 == 0, "world descriptor in words");
-			using CWord = const __attribute__((address_space(4))) uint32_t;
-			CWord* src = (CWord*)(a.worlds + ww);
-			WorldDesc wd;
-			uint32_t* dst = reinterpret_cast<uint32_t*>(&wd);
-#pragma unroll
-			for (int k = 0; k < (int)(sizeof(WorldDesc) / 4); ++k)
-				dst[k] = src[k];
-			Wl.g = wd.g;
-			Wl.mats = wd.mats;
-			Wl.nmats = wd.nmats;
+			load_world(a, ww, Wl);
 			mine = valid && (s.flags >> FL_WORLD_SHIFT) == ww;
 		}
 		if (SID_LDS) {
@@ -941,6 +954,302 @@ __global__ __launch_bounds__(256) void k_inel(StepArgs a)
 	}
 }
 
+// Few particles in flight: their cascades, wave by wave.
+//
+// A launch of k_step + k_inel takes every particle K steps on and lasts as
+// long as its slowest wave: with few particles that is a chain of dependent
+// loads of one long walk, and the launches and their gaps come on top (36 us
+// for 4 steps of 100 electrons).  Here a wave keeps its particles for up to
+// 1024 steps and its secondaries with them: inelastic events run
+// in line, a secondary takes a free lane of its parent's wave (its state is
+// fetched across lanes), and waves do not wait for each other.  Particles
+// are spread over as many waves as the grid has, so a wave starts with few
+// lanes in use, diverges little and fills up with its own secondaries; those
+// beyond its 64 lanes go to the buffer's SE region (else the spill stack)
+// for the next launch, which spreads them over the waves again.
+//
+// Bound by the latency of one step's dependent loads and arithmetic (about
+// 4 us) times the longest chain of steps, where particles are few, and by
+// instruction issue on diverging lanes where they fill the waves.  One wave
+// a block: nothing here is shared between waves.  Measured on the launches
+// it takes over from k_step + k_inel: 100 primaries of 1 keV in a slab 5.6
+// -> 2.0 ms, 1003 of 10 keV 41 -> 9.0 ms, 4096 of 500 eV on a grating 8.2 ->
+// 2.8 ms, 96 903 of 500 eV 16.8 -> 13.0 ms.
+template <bool SC, bool MULTI, bool WUNI>
+__device__ __forceinline__ void cascade_body(const StepArgs& a)
+{
+	static_assert(!(WUNI && (SC || MULTI)), "the world-per-wave variant is the plain one");
+	constexpr bool DEP_OK = SC || MULTI;
+	constexpr bool SKIP = !MULTI;
+	Ctrl* C = a.ctrl;
+	if (!C->few || C->n_surv + C->n_se == 0u)
+		return;
+	const uint32_t bi = C->buf_in;
+	const Bufs in = bi ? a.buf[1] : a.buf[0];
+	const Bufs out = bi ? a.buf[0] : a.buf[1];
+	const uint32_t n_surv = C->n_surv, n_in = n_surv + C->n_se;
+	const int np = a.map.np;
+	World Wl = a.W;
+	const World& W = (MULTI || WUNI) ? Wl : a.W;
+	__shared__ int s_path[PATH_LEVELS * 64];
+	__shared__ int s_owner[4 * 64];   // owner table, pair queue, safeties
+	const uint32_t lane = threadIdx.x;
+	int* const path = s_path + lane;
+	const uint64_t below = (1ull << lane) - 1ull;
+	const bool ident = WUNI && a.perm_n[1] != 0u;
+	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
+	// Lanes a wave starts with: a power of two, so that a world's range of
+	// 64 indices is split evenly; half the grid's waves are used before a
+	// wave takes a second particle (all of them: 3.53 -> 3.96 ms at 4096).
+	uint32_t g = 1;
+	while (g < 64u && g * (gridDim.x / 2u) < n_loop)
+		g <<= 1;
+	// Steps of the launch, and the share of the live lanes that runs pending
+	// events at once: with few lanes in use a wave is bound by its longest
+	// chain of events, so nothing waits and the launch is long; full waves
+	// are bound by their instructions, and their finished lanes are idle
+	// until the next launch.  (64 steps and a quarter for every g: 12.3 and
+	// 2.5 ms for 1003 primaries of 10 keV and 100 of 1 keV in a slab; 1024
+	// steps and any lane: 9.0 and 2.0 ms, but 14.6 against 13.0 ms for
+	// 96 903 primaries of 500 eV.)
+	const uint32_t n_steps = max(64u, 1024u / g);
+	const int pend_share = max(4, 64 / (int)g);
+	const uint32_t groups = (n_loop + g - 1u) / g, waves = min(gridDim.x, groups);
+	// Room in the output buffer: a group that starts with m particles holds
+	// at most m + `extra` at any time, so at most n_in + groups * extra
+	// survive; the rest of the buffer is for the secondaries placed from its
+	// top (k_ctrl and the host read this launch's limit from se_limit, which
+	// no wave of it reads).
+	const uint32_t extra = (a.slots - n_in) / 2u / groups;
+	const uint32_t se_limit = a.slots - n_in - groups * extra;
+	if (blockIdx.x == 0 && lane == 0)
+		C->se_limit = se_limit;
+	uint32_t my_steps = 0;
+	for (uint32_t w0 = blockIdx.x * g; w0 < n_loop; w0 += gridDim.x * g) {
+		const uint32_t i = w0 + lane;
+		const bool have = lane < g && i < n_loop;
+		const uint32_t li = (WUNI && !ident) ? (have ? a.perm[i] : ~0u) : i;
+		bool occ = have && li != ~0u;   // this lane holds a particle
+		const uint64_t first = __ballot(occ);
+		if (first == 0ull)
+			continue;
+		const int hold = (int)min(64u, (uint32_t)__popcll(first) + extra);
+		State s = {};
+		Score sc;
+		if (occ) {
+			const uint32_t slot = in_slot(li, n_surv, a.slots);
+			s = load_state(in, slot);
+			if (SC) load_score(in, slot, np, sc);
+			if (MULTI) {
+				const WorldDesc& wd = a.worlds[s.flags >> FL_WORLD_SHIFT];
+				Wl.g = wd.g;
+				Wl.mats = wd.mats;
+				Wl.nmats = wd.nmats;
+			}
+		}
+		if (WUNI)   // one world a wave; its first particle names it
+			load_world(a, __builtin_amdgcn_readlane(s.flags >> FL_WORLD_SHIFT, __builtin_ctzll(first)), Wl);
+		bool pend = (s.flags & FL_PEND_INEL) != 0u;   // an inelastic event to run
+		bool det = (s.flags & FL_PEND_DET) != 0u;     // to be recorded
+		bool park = false;                            // waits for the next launch
+		s.flags &= FL_WORLD_MASK;
+		float rem = SKIP ? s.safe : -1.0f;
+		for (uint32_t k = 0; k < n_steps; ++k) {
+			const uint64_t live = __ballot(occ && !park);
+			if (live == 0ull)
+				break;
+			// every wave writes at most 64 deposits a step: stop while all of
+			// them still have room in the first half of the buffer
+			if (DEP_OK && a.dep && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+					+ 64ull * waves > a.dep_cap / 2u)
+				break;
+			if (pend_share * __popcll(__ballot(pend)) >= __popcll(live)) {
+				Particle se = {};
+				Particle pre = {};
+				bool made = false;
+				if (pend) {
+					pre = s.p;
+					Rng rng;
+					rng_start(rng, W.key0, W.key1, s.sid, s.step);
+					rng_seek(rng, 2);
+					step_event(W, s, rng, EV_INELASTIC, -1, se, made);
+					// a secondary that its first step would end is counted and
+					// not stored (as in k_inel)
+					if (made && (!in_domain(W.g, se.pos) || se.E < W.mats[s.mat].barrier + W.threshold)) {
+						made = false;
+						++my_steps;
+					}
+				}
+				const uint64_t mm = __ballot(made);
+				bool done = true;
+				if (mm) {
+					const uint64_t mf = __ballot(!occ);
+					// lanes that may be filled
+					const int nm = (int)__popcll(mm), nf = max(0, hold - 64 + (int)__popcll(mf));
+					const int r = (int)__popcll(mm & below), rf = (int)__popcll(mf & below);
+					if (made)
+						s_owner[r] = (int)lane;
+					__builtin_amdgcn_wave_barrier();
+					const bool take = !occ && rf < min(nm, nf);
+					const int src = take ? s_owner[rf] : (int)lane;
+					__builtin_amdgcn_wave_barrier();
+					// the secondaries beyond the free lanes
+					const bool over = made && r >= nf;
+					const uint32_t sslot = wave_alloc((uint32_t*)&C->se_ctr, over);
+					s.safe = rem;
+					if (over)
+						done = place_secondary<SC>(a, C, out, se_limit, true, sslot, se, s, sc);
+					const uint64_t csid = se_sid(s.sid, s.step);
+					const F3 cp = { __shfl(se.pos.x, src), __shfl(se.pos.y, src), __shfl(se.pos.z, src) };
+					const F3 cd = { __shfl(se.dir.x, src), __shfl(se.dir.y, src), __shfl(se.dir.z, src) };
+					const float cE = __shfl(se.E, src), crem = __shfl(rem, src);
+					const int cmat = __shfl(s.mat, src);
+					const uint32_t ctag = (uint32_t)__shfl((int)s.tag, src), cfl = (uint32_t)__shfl((int)s.flags, src);
+					const uint32_t clo = (uint32_t)__shfl((int)(uint32_t)csid, src);
+					const uint32_t chi = (uint32_t)__shfl((int)(uint32_t)(csid >> 32), src);
+					if (SC) {
+#pragma unroll
+						for (int q = 0; q < MAX_PARAMS; ++q)
+							if (q < np) {
+								const double v = __shfl(sc.v[q], src);
+								if (take) sc.v[q] = v;
+							}
+					}
+					if (take) {
+						s.p.pos = cp;
+						s.p.dir = cd;
+						s.p.E = cE;
+						s.mat = cmat;
+						s.last_tri = -1;
+						s.tag = ctag;
+						s.step = 0;
+						s.flags = cfl;
+						s.sid = ((uint64_t)chi << 32) | clo;
+						rem = crem;
+						if (MULTI) {
+							const WorldDesc& wd = a.worlds[s.flags >> FL_WORLD_SHIFT];
+							Wl.g = wd.g;
+							Wl.mats = wd.mats;
+							Wl.nmats = wd.nmats;
+						}
+						occ = true;
+					}
+				}
+				if (DEP_OK && a.dep)
+					deposit(a, C, pend && done && s.p.E != pre.E, s, pre.E);
+				if (pend) {
+					if (done) {
+						s.step++;
+						pend = false;
+					} else {
+						// no room anywhere: run the event again, from the same
+						// draws, in a later launch
+						s.p = pre;
+						park = true;
+					}
+				}
+			}
+			const bool run = occ && !pend && !park && !det;
+			const bool walk_any = __ballot(run) != 0ull;
+			if (walk_any) {
+				int oc = ALIVE, mat0 = s.mat, type = 0;
+				bool walk = false;
+				Rng rng;
+				F3 nd = { 0.0f, 0.0f, 0.0f };
+				float distance = 0.0f;
+				PathInfo pinfo;
+				if (run) {
+					rng_start(rng, W.key0, W.key1, s.sid, s.step);
+					oc = step_plan(W, s, rng, nd, distance, type, pinfo);
+					++my_steps;
+					walk = (oc == ALIVE);
+				}
+				const bool skip = SKIP && walk && distance <= rem;
+				float hd, saf = -1.0f;
+				int hit = propagate_wave<!MULTI, SKIP>(W.g, walk && !skip, s.p.pos, nd, distance, s.last_tri, s.mat,
+					hd, path, 64, s_owner, &saf);
+				if (SKIP && walk) {
+					if (skip) {
+						hit = -1;
+						hd = distance;
+					}
+					rem = (hit >= 0) ? -1.0f : ((skip ? rem : saf) - distance) - W.g.step_eps;
+				}
+				if (walk) {
+					int ev;
+					step_move(s, nd, distance, type, hit, hd, ev, pinfo);
+					if (SC)
+						score_free_path(sc, a.map, W, mat0, pinfo, ev);
+					if (ev == EV_INELASTIC) {
+						pend = true;
+					} else {
+						const float e0 = s.p.E;
+						if (SC) {
+							float gr = 0.0f;
+							int gmi = -1, gmo = -1;
+							oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &gr, &gmi, &gmo);
+							if (ev == EV_INTERSECT)
+								score_barrier(sc, a.map, gmi, gmo, gr);
+						} else {
+							oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+						}
+						if (DEP_OK && a.dep)
+							deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
+					}
+				}
+				if (run) {
+					if (oc == DETECTED)
+						det = true;
+					else if (oc == TERMINATED)
+						occ = false;
+					else if (!pend)
+						s.step++;
+				}
+			}
+			const bool rec = det && !park;
+			if (__ballot(rec)) {
+				const uint32_t dslot = wave_alloc(&C->det_ctr, rec);
+				if (rec) {
+					if (dslot < a.det_cap) {
+						nbl_detected r;
+						r.pos[0] = s.p.pos.x; r.pos[1] = s.p.pos.y; r.pos[2] = s.p.pos.z;
+						r.dir[0] = s.p.dir.x; r.dir[1] = s.p.dir.y; r.dir[2] = s.p.dir.z;
+						r.kin_energy = s.p.E;
+						r.tag = s.tag;
+						r.sid = s.sid;
+						a.det[dslot] = r;
+						if (SC) {
+#pragma unroll
+							for (int q = 0; q < MAX_PARAMS; ++q)
+								if (q < np)
+									a.det_sc[(size_t)dslot * np + q] = sc.v[q];
+						}
+						occ = false;
+						det = false;
+					} else {
+						park = true;   // no record slot: again next launch
+					}
+				}
+			}
+		}
+		uint32_t oslot, qslot;
+		wave_alloc2(&C->step_out, occ, false, oslot, qslot);
+		if (occ) {
+			s.flags |= (pend ? FL_PEND_INEL : 0u) | (det ? FL_PEND_DET : 0u);
+			s.safe = rem;
+			store_state(out, oslot, s);
+			if (SC) store_score(out, oslot, np, sc);
+		}
+	}
+	count_steps(C, my_steps);
+}
+
+template <bool SC, bool MULTI, bool WUNI = false>
+__global__ __launch_bounds__(64) void k_cascade(StepArgs a)
+{
+	cascade_body<SC, MULTI, WUNI>(a);
+}
+
 // Queue entries of one push: tag (tag_base + i, unless given), stream id
 // sid_base + i and world number.
 __global__ __launch_bounds__(256) void k_queue_ids(uint32_t* tag, uint64_t* sid, uint16_t* world, uint32_t n,
@@ -1162,9 +1471,11 @@ struct nbl_driver {
 	std::vector<Material> h_mats;   // host copy of d_mats
 	uint32_t blocks_per_cu = 64;    // k_step grid: blocks of 256 per compute unit
 	uint32_t target = 0;            // particles in flight to aim for
+	uint32_t few = 0;               // up to this many in flight a launch is k_cascade's
 	nbl_deposit* dep = nullptr;     // energy-deposit records (enabled when non-null)
 	uint64_t dep_cap = 0;
 	uint32_t dep_per_particle = 0;  // K + 1 when the buffer was sized
+	bool dep_drained = false;       // no iteration since the last drain of deposits
 	bool use_graph = false;         // replay iterations from captured graphs
 	uint64_t epoch = 0;             // bumped when a launch argument changes
 	struct Graph { uint32_t n; uint64_t epoch; hipGraph_t g; hipGraphExec_t exec; };
@@ -1182,6 +1493,15 @@ struct nbl_driver {
 };
 
 namespace {
+
+// Waves of a k_cascade launch, and the particles in flight up to which a
+// launch is k_cascade's.
+// 16 waves a compute unit are all resident (118 VGPRs); up to 1024 particles
+// a compute unit they hold every particle (512: 13.3 against 12.9 ms for
+// 96 903 primaries of 500 eV on a grating, 27.0 against 25.8 ms for 160 000
+// of 1 keV on contact holes; 1536, waves taking two turns: 13.7 and 26.0).
+uint32_t cascade_waves(const nbl_device* dev) { return 16u * (uint32_t)dev->n_cu; }
+uint32_t cascade_max(const nbl_device* dev) { return 64u * cascade_waves(dev); }
 
 int set_device(const nbl_device* dev)
 {
@@ -1663,6 +1983,7 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 	std::memset(&c, 0, sizeof(c));
 	c.target = capacity;
 	d->target = capacity;
+	d->few = cascade_max(dev);
 	if (hipMemcpy(d->ctrl, &c, sizeof(Ctrl), hipMemcpyHostToDevice) != hipSuccess)
 		return cleanup(fail(NBL_ERR_DEVICE, "control block upload failed"));
 	d->W.g = geom->g;
@@ -1829,7 +2150,7 @@ namespace {
 void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 {
 	const bool multi = d->h_worlds.size() > 1 || d->dep;
-	const dim3 grid(g), block(256);
+	const dim3 grid(g), block(256), cgrid(cascade_waves(d->dev)), cblock(64);
 	if (multi && !d->dep && !d->map.np) {
 		// several worlds, nothing but records: the launch's particles
 		// grouped by world, one world per wave
@@ -1844,18 +2165,23 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 		else
 			hipLaunchKernelGGL(k_world_place_wide, grid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1],
 				d->slots, nw, d->wgrp, d->perm);
+		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else if (d->map.np && multi) {
+		hipLaunchKernelGGL((k_cascade<true, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<true, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<true, true>), grid, block, 0, d->stream, a);
 	} else if (d->map.np) {
+		hipLaunchKernelGGL((k_cascade<true, false>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<true, false>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<true, false>), grid, block, 0, d->stream, a);
 	} else if (multi) {
+		hipLaunchKernelGGL((k_cascade<false, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else {
+		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, false>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, false>), grid, block, 0, d->stream, a);
 	}
@@ -1887,15 +2213,17 @@ StepArgs step_args(const nbl_driver* d)
 	return a;
 }
 
-// One tracking iteration: control, refill, step pair.  The step pair is
+// One tracking iteration: control, refill, and k_cascade or the step pair
+// (k_ctrl picks; never k_cascade without `cascade`).  The last two are
 // bracketed by timing events when timing is on.
-int enqueue_iteration(nbl_driver* d, const StepArgs& a)
+int enqueue_iteration(nbl_driver* d, const StepArgs& a, bool cascade)
 {
 	const uint32_t g_refill = blocks_for(d->capacity);
 	// grid-stride: blocks_per_cu x compute units blocks of 256 threads (a
 	// multiple of the resident blocks), never more than the capacity needs
 	const uint32_t g_step = std::min<uint32_t>(blocks_for(d->capacity), d->blocks_per_cu * (uint32_t)d->dev->n_cu);
-	hipLaunchKernelGGL(k_ctrl, dim3(1), dim3(64), 0, d->stream, d->ctrl, d->slots, d->spill_cap);
+	hipLaunchKernelGGL(k_ctrl, dim3(1), dim3(64), 0, d->stream, d->ctrl, d->slots, d->spill_cap,
+		cascade ? d->few : 0u, cascade_waves(d->dev), d->dep ? a.dep_cap / 2u : ~0u);
 	hipLaunchKernelGGL(k_refill, dim3(g_refill), dim3(256), 0, d->stream, d->ctrl, d->buf[0],
 		d->buf[1], d->spill, d->q_part, d->q_tag, d->q_sid, d->q_world, (uint32_t)d->map.np, 0ull);
 	std::pair<hipEvent_t, hipEvent_t> ev{};
@@ -1941,7 +2269,7 @@ int launch_graph(nbl_driver* d, const StepArgs& a, uint32_t n)
 	HIP_OK(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
 	int rc = NBL_OK;
 	for (uint32_t it = 0; it < n && rc == NBL_OK; ++it)
-		rc = enqueue_iteration(d, a);
+		rc = enqueue_iteration(d, a, !d->dep);
 	const hipError_t e = hipStreamEndCapture(d->stream, &gr.g);
 	if (rc) return rc;
 	if (e != hipSuccess)
@@ -1963,12 +2291,17 @@ int nbl_driver_iterate(nbl_driver* d, uint32_t n_iter)
 	// an error left by an earlier, unrelated runtime call is not this call's
 	(void)hipGetLastError();
 	const StepArgs a = step_args(d);
+	// Deposits are drained after every call: a call of one iteration on a
+	// drained buffer may write half of it (k_cascade), any other writes K + 1
+	// records a particle and iteration at most.
+	const bool cascade = !d->dep || (d->dep_drained && n_iter == 1);
+	d->dep_drained = false;
 	if (d->use_graph && !d->timing && n_iter > 1) {
 		if ((rc = launch_graph(d, a, n_iter)))
 			return rc;
 	} else {
 		for (uint32_t it = 0; it < n_iter; ++it)
-			if ((rc = enqueue_iteration(d, a)))
+			if ((rc = enqueue_iteration(d, a, cascade)))
 				return rc;
 	}
 	HIP_OK(hipGetLastError());
@@ -2093,6 +2426,7 @@ int nbl_driver_set_deposits(nbl_driver* d, int enable)
 		return rc;
 	const uint32_t zero = 0;
 	HIP_OK(hipMemcpy(&d->ctrl->dep_ctr, &zero, sizeof(zero), hipMemcpyHostToDevice));
+	d->dep_drained = true;
 	return NBL_OK;
 }
 
@@ -2119,6 +2453,7 @@ int nbl_driver_drain_deposits(nbl_driver* d, nbl_deposit* out, uint64_t cap, uin
 	const uint32_t zero = 0;
 	HIP_OK(hipMemcpyAsync(&d->ctrl->dep_ctr, &zero, sizeof(zero), hipMemcpyHostToDevice, d->stream));
 	HIP_OK(hipStreamSynchronize(d->stream));
+	d->dep_drained = true;
 	*n = written;
 	return NBL_OK;
 }
@@ -2155,6 +2490,18 @@ int nbl_driver_set_launch(nbl_driver* d, uint32_t steps_per_launch, uint32_t blo
 	HIP_OK(hipStreamSynchronize(d->stream));
 	HIP_OK(hipMemcpy(&d->ctrl->target, &target, sizeof(uint32_t), hipMemcpyHostToDevice));
 	d->target = target;
+	return NBL_OK;
+}
+
+int nbl_driver_set_cascade(nbl_driver* d, uint32_t max_particles)
+{
+	clear_error();
+	if (!d)
+		return fail(NBL_ERR_ARG, "null driver");
+	const uint32_t few = std::min(max_particles, cascade_max(d->dev));
+	if (d->few != few)
+		d->epoch++;
+	d->few = few;
 	return NBL_OK;
 }
 
@@ -2325,6 +2672,8 @@ int run_loop(nbl_driver* d, bool with_scores, uint32_t frame_iters, const Record
 	}
 	if (!d->stage_ev)
 		HIP_OK(hipEventCreateWithFlags(&d->stage_ev, hipEventDisableTiming));
+	// k_cascade takes particles many steps on, so a frame of few particles
+	// has few iterations
 	uint32_t frame = frame_iters ? frame_iters : 4;
 	uint64_t last_steps = ~0ull;
 	int stalled = 0;
@@ -2359,7 +2708,7 @@ int run_loop(nbl_driver* d, bool with_scores, uint32_t frame_iters, const Record
 			}
 			last_steps = total_steps(*d->h_ctrl);
 			if (!frame_iters)
-				frame = std::min<uint32_t>(frame * 2, 32);
+				frame = running + queued <= d->few ? 2 : std::min<uint32_t>(frame * 2, 32);
 			if ((rc = nbl_driver_iterate(d, frame)))
 				return rc;
 		}
@@ -2819,9 +3168,11 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 	int stalled = 0;
 	for (;;) {
 		for (uint32_t it = 0; it < frame; ++it) {
-			hipLaunchKernelGGL(k_ctrl, dim3(1), dim3(64), 0, st, ctrl, slots, NA_SPILL);
+			hipLaunchKernelGGL(k_ctrl, dim3(1), dim3(64), 0, st, ctrl, slots, NA_SPILL, cascade_max(dev), cascade_waves(dev),
+				~0u);
 			hipLaunchKernelGGL(k_refill, dim3(g_refill), dim3(256), 0, st, ctrl, a.buf[0], a.buf[1], a.spill,
 				primaries, tags, (const uint64_t*)nullptr, (const uint16_t*)nullptr, 0u, sid_base);
+			hipLaunchKernelGGL((k_cascade<false, false>), dim3(cascade_waves(dev)), dim3(64), 0, st, a);
 			hipLaunchKernelGGL((k_step<false, false>), dim3(g_step), dim3(256), 0, st, a);
 			hipLaunchKernelGGL((k_inel<false, false>), dim3(g_step), dim3(256), 0, st, a);
 		}
@@ -2849,7 +3200,8 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 		}
 		last_steps = total_steps(h);
 		last_det = h.det_ctr;
-		frame = std::min<uint32_t>(frame * 2, 32);
+		frame = active_count(h, NA_SPILL) + (h.queue_n - h.queue_next) <= cascade_max(dev) ? 2
+			: std::min<uint32_t>(frame * 2, 32);
 	}
 	return NBL_OK;
 }
