@@ -121,7 +121,16 @@ struct StepArgs {
 	// world (k_world_group); k_step's wave takes perm[i] for index i
 	const uint32_t* perm;
 	const uint32_t* perm_n;   // its padded length; perm_n[1]: one world, perm unused
+	// walks that a launch leaves unfinished, for the particles of buf[0] and
+	// buf[1] (WALK_FIELDS words a slot, [field][slot]), or null: a launch
+	// then finishes its walks
+	uint32_t* walk[2];
 };
+constexpr uint32_t WALK_FIELDS = 7;
+// Particles in flight from which a launch leaves walks unfinished: with so
+// many some steps end in every launch, which the callers' checks for a run
+// that makes no progress count on.
+constexpr uint32_t KEEP_WALKS_MIN = 65536;
 
 __device__ __forceinline__ State load_state(const Bufs& b, uint32_t i)
 {
@@ -604,6 +613,17 @@ __device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, co
 // holding another world's particle wait, unchanged, for a later launch.
 // Trajectories depend only on each particle's own stream, so which launch
 // steps a particle changes no result.
+__device__ __forceinline__ void store_detected(const StepArgs& a, uint32_t slot, const State& s)
+{
+	nbl_detected r;
+	r.pos[0] = s.p.pos.x; r.pos[1] = s.p.pos.y; r.pos[2] = s.p.pos.z;
+	r.dir[0] = s.p.dir.x; r.dir[1] = s.p.dir.y; r.dir[2] = s.p.dir.z;
+	r.kin_energy = s.p.E;
+	r.tag = s.tag;
+	r.sid = s.sid;
+	a.det[slot] = r;
+}
+
 // World `ww` (wave-uniform) through the constant address space: scalar
 // loads, so the world's geometry and materials sit in SGPRs as the plain
 // kernel's arguments do (not in VGPRs).
@@ -622,54 +642,234 @@ __device__ __forceinline__ void load_world(const StepArgs& a, uint32_t ww, World
 	W.nmats = wd.nmats;
 }
 
-template <bool SC, bool MULTI, bool WUNI = false>
+// A lane's step while it lasts: planned, and perhaps on its walk.
+struct InFlight {
+	Walk w;
+	float distance, logE;       // free path, log of the energy
+	int type;                   // its mechanism
+	uint32_t b2, b3;            // the event's first two draws (in a material)
+	float tau_el, tau_in;       // for the score
+	bool on;                    // walking
+	bool first;                 // in its start cell
+	bool planned;               // by an earlier launch
+	bool resume;                // and its walk goes on
+};
+
+__device__ __forceinline__ void load_walk(const StepArgs& a, uint32_t buf, uint32_t slot, Walk& w)
+{
+	const uint32_t* p = a.walk[buf];
+	const size_t n = a.slots;
+	w.cur = { __uint_as_float(p[slot]), __uint_as_float(p[n + slot]), __uint_as_float(p[2 * n + slot]) };
+	w.to_go = __uint_as_float(p[3 * n + slot]);
+	w.location = ((uint64_t)p[5 * n + slot] << 32) | p[4 * n + slot];
+	w.cells = p[6 * n + slot];
+}
+
+__device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const Walk& w)
+{
+	uint32_t* p = a.walk[buf];
+	const size_t n = a.slots;
+	p[slot] = __float_as_uint(w.cur.x);
+	p[n + slot] = __float_as_uint(w.cur.y);
+	p[2 * n + slot] = __float_as_uint(w.cur.z);
+	p[3 * n + slot] = __float_as_uint(w.to_go);
+	p[4 * n + slot] = (uint32_t)w.location;
+	p[5 * n + slot] = (uint32_t)(w.location >> 32);
+	p[6 * n + slot] = w.cells;
+}
+
+// One turn of a wave (every lane calls): lanes with `plan` set plan their
+// next step (domain, threshold, path sampling), walking lanes walk through
+// one cell, and lanes whose walk ends or whose free path stays inside the
+// safety ball move and take their boundary or elastic event.
+//
+// A walk takes as many turns as it has cells, while the other lanes go on
+// with their steps: about one walking lane in ten leaves its first cell, and
+// flights through the vacuum cross tens of them.  With every walk finished in
+// the step that began it, half of a wave's cell searches were made for one
+// or two lanes.
+//
+// Steps whose free path cannot reach a triangle skip the walk: after a walk
+// that found no hit, `rem` is the start point's safety (no triangle of its
+// cell and no cell wall within that distance, walk_round) less the distance
+// moved since; a later free path no longer than `rem` ends inside that ball,
+// where the walk would find no hit and return the full free path.  rem < 0:
+// the next step walks.
+//
+// Returns true in lanes whose step has ended: `oc` ALIVE (with `to_inel`: an
+// inelastic event is to follow), DETECTED or TERMINATED.
+template <bool SC>
+__device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, bool plan, State& s, uint64_t sid,
+	uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* path, int stride, int* owner_at,
+	int& oc, bool& to_inel)
+{
+	oc = ALIVE;
+	to_inel = false;
+	bool ended = false, skip = false;
+	if (plan) {
+		Rng rng;
+		rng_start(rng, W.key0, W.key1, sid, step);
+		F3 nd;
+		PathInfo pinfo;
+		oc = step_plan(W, s, rng, nd, f.distance, f.type, pinfo, f.planned);
+		if (!f.planned)
+			++my_steps;
+		if (oc == ALIVE) {
+			s.p.dir = nd;
+			f.logE = pinfo.logE;
+			f.b2 = rng.b2;
+			f.b3 = rng.b3;
+			if (SC) {
+				f.tau_el = pinfo.tau_el;
+				f.tau_in = pinfo.tau_in;
+			}
+			skip = !f.resume && f.distance <= rem;
+			f.on = !skip;
+			f.first = !f.resume;
+			if (f.resume) {
+				walk_path(W.g, f.w, path, stride);
+				((float*)owner_at)[192 + __lane_id()] = rem;
+			} else if (!skip) {
+				walk_start(f.w, s.p.pos, f.distance);
+			}
+		} else {
+			ended = true;
+		}
+		f.planned = f.resume = false;
+	}
+	int hit = -1;
+	float hd = 0.0f;
+	bool arrive = skip;
+	if (__ballot(f.on) != 0ull) {
+		float isect;
+		int target;
+		const int r = walk_round<true>(W.g, f.on, f.first, f.w, s.p.dir, s.last_tri, s.mat, path, stride, owner_at,
+			isect, target);
+		f.first = false;
+		if (f.on && r != WALK_ON) {
+			f.on = false;
+			arrive = true;
+			if (r == WALK_HIT) {
+				hit = target;
+				hd = f.distance - f.w.to_go + isect;
+				rem = -1.0f;
+			} else {
+				rem = (((float*)owner_at)[192 + __lane_id()] - f.distance) - W.g.step_eps;
+			}
+		}
+	}
+	if (skip)
+		rem = (rem - f.distance) - W.g.step_eps;
+	if (arrive) {
+		ended = true;
+		int ev;
+		PathInfo pinfo;
+		const int mat0 = s.mat;
+		pinfo.tau_el = f.tau_el;
+		pinfo.tau_in = f.tau_in;
+		step_move(s, s.p.dir, f.distance, f.type, hit, hd, ev, pinfo);
+		if (SC)
+			score_free_path(sc, a.map, W, mat0, pinfo, ev);
+		if (ev == EV_INELASTIC) {
+			to_inel = true;
+		} else {
+			Rng rng;
+			rng_start(rng, W.key0, W.key1, sid, step);
+			if (s.mat >= 0) {
+				// two draws were taken for the free paths
+				rng.b2 = f.b2;
+				rng.b3 = f.b3;
+				rng.idx = 2;
+			}
+			if (SC) {
+				float g = 0.0f;
+				int gmi = -1, gmo = -1;
+				oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, f.logE, &g, &gmi, &gmo);
+				if (ev == EV_INTERSECT)
+					score_barrier(sc, a.map, gmi, gmo, g);
+			} else {
+				oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, f.logE);
+			}
+		}
+	}
+	return ended;
+}
+
+// Write the wave's particles out: detected records, the inelastic queue and
+// the survivors, with one ballot per kind and one atomic per wave for the
+// last two together.  `f`: walks that go on in the next launch, or null.
+template <bool SC>
+__device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const Score& sc,
+	bool keep, bool det, bool to_inel, const InFlight* f)
+{
+	const Bufs out = out_buf ? a.buf[1] : a.buf[0];
+	const int np = a.map.np;
+	const uint32_t dslot = wave_alloc(&C->det_ctr, det);
+	if (det) {
+		if (dslot < a.det_cap) {
+			store_detected(a, dslot, s);
+			if (SC) {
+#pragma unroll
+				for (int q = 0; q < MAX_PARAMS; ++q)
+					if (q < np)
+						a.det_sc[(size_t)dslot * np + q] = sc.v[q];
+			}
+			keep = false;
+		} else {
+			// no record slot: wait as a survivor and retry next launch
+			s.flags |= FL_PEND_DET;
+		}
+	}
+	const bool queue = keep && to_inel;
+	const bool survive = keep && !to_inel;
+	uint32_t oslot, qslot;
+	wave_alloc2(&C->step_out, survive, queue, oslot, qslot);
+	if (queue) {
+		store_state(a.inel, qslot, s);
+		if (SC) store_score(a.inel, qslot, np, sc);
+	}
+	if (survive) {
+		if (f && f->on) {
+			s.flags |= FL_PLANNED | FL_WALK;
+			store_walk(a, out_buf, oslot, f->w);
+		}
+		store_state(out, oslot, s);
+		if (SC) store_score(out, oslot, np, sc);
+	}
+}
+
+template <bool SC, bool WUNI>
 __device__ __forceinline__ void step_body(const StepArgs& a)
 {
-	static_assert(!(WUNI && (SC || MULTI)), "the world-per-wave variant is the plain one");
-	// energy deposits are recorded by the general variants only
-	constexpr bool DEP_OK = SC || MULTI;
+	static_assert(!(WUNI && SC), "the world-per-wave variant is the plain one");
 	Ctrl* C = a.ctrl;
 	if (C->few)
 		return;   // k_cascade takes this launch
 	const uint32_t bi = C->buf_in;
 	const Bufs in = bi ? a.buf[1] : a.buf[0];
-	const Bufs out = bi ? a.buf[0] : a.buf[1];
 	const uint32_t n_surv = C->n_surv, n_in = n_surv + C->n_se;
-	const uint32_t B = a.slots, det_cap = a.det_cap, K = a.K;
+	const uint32_t K = a.K;
 	const int np = a.map.np;
+	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	World Wl = a.W;
-	const World& W = (MULTI || WUNI) ? Wl : a.W;
+	const World& W = WUNI ? Wl : a.W;
 	__shared__ int s_path[PATH_LEVELS * 256];
 	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
 	// In the plain variant a particle's stream id waits here during its steps
-	// (each step reads it once to start its Philox stream): two fewer VGPRs
-	// across the step loop, and the loop no longer spills (4 % faster).  The
-	// multi-world variant has the registers and ran 3 % slower with it.
-	constexpr bool SID_LDS = !SC && !MULTI;
+	// (each step reads it once to start its Philox stream), and with it its
+	// tag, step and flags (the walk needs none of them).
+	constexpr bool SID_LDS = !SC;
 	__shared__ uint64_t s_sid[SID_LDS ? 256 : 1];
-	// With the stream id wait the particle's tag, step and flags (the walk
-	// needs none of them): three VGPRs fewer across the step loop.
 	__shared__ uint32_t s_aux[SID_LDS ? 3 * 256 : 1];
 	uint32_t* const aux = s_aux + (SID_LDS ? threadIdx.x : 0u);
 
 	int* path = s_path + threadIdx.x;
 	int* owner_at = s_owner + 4 * (threadIdx.x & ~63u);
-	// Steps whose free path cannot reach a triangle skip the walk: after a
-	// walk that found no hit, `rem` is the start point's safety (no triangle
-	// of its cell and no cell wall within that distance, propagate_wave)
-	// less the distance moved since; a later free path no longer than `rem`
-	// ends inside that ball, where the walk would find no hit and return the
-	// full free path.  rem < 0: the next step walks.  It travels with the
-	// particle (State::safe) from launch to launch, through the inelastic
-	// queue (the event does not move it) and into its secondaries (they
-	// start where it stands).  (Single-world variants; the multi-world walk
-	// gives no safety and clears it.)
-	constexpr bool SKIP = !MULTI;
 	uint32_t my_steps = 0;
 	const uint32_t stride = gridDim.x * blockDim.x;
 	// Whole waves take consecutive particles and step in lockstep: the walk
-	// shares its triangle tests across the wave (propagate_wave), so every
-	// lane joins it each step, also lanes whose particle has stopped.
+	// shares its triangle tests across the wave (walk_round), so every
+	// lane joins it each turn, also lanes whose particle has stopped.
 	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
 	// world-per-wave: index i names particle perm[i] (~0u: padding), or
 	// particle i when the launch holds one world's particles only
@@ -681,106 +881,53 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		const bool valid = (WUNI && !ident) ? li != ~0u : i < n_in;
 		State s = {};
 		Score sc;
+		InFlight f = {};
 		if (valid) {
-			const uint32_t slot = (li < n_surv) ? li : (B - 1u - (li - n_surv));
+			const uint32_t slot = in_slot(li, n_surv, a.slots);
 			s = load_state(in, slot);
 			if (SC) load_score(in, slot, np, sc);
-			if (MULTI) {
-				const WorldDesc& wd = a.worlds[s.flags >> FL_WORLD_SHIFT];
-				Wl.g = wd.g;
-				Wl.mats = wd.mats;
-				Wl.nmats = wd.nmats;
-			}
+			f.planned = (s.flags & FL_PLANNED) != 0u;
+			f.resume = (s.flags & FL_WALK) != 0u;
+			if (f.resume)
+				load_walk(a, bi, slot, f.w);
 		}
-		bool mine = valid;
 		if (WUNI) {
 			// lane 0 holds a particle (each world's range starts at a multiple
 			// of 64 and has no padding before its last particle; with one
 			// world, w0 < n_in): its world is the wave's, and no lane holds
 			// another world's particle
-			const uint32_t ww = __builtin_amdgcn_readfirstlane(s.flags >> FL_WORLD_SHIFT);
-			load_world(a, ww, Wl);
-			mine = valid && (s.flags >> FL_WORLD_SHIFT) == ww;
+			load_world(a, __builtin_amdgcn_readfirstlane(s.flags >> FL_WORLD_SHIFT), Wl);
 		}
+		bool det = (s.flags & FL_PEND_DET) != 0u;
+		// an inelastic event that found no secondary slot earlier
+		bool to_inel = (s.flags & FL_PEND_INEL) != 0u;
+		bool run = valid && !det && !to_inel, dead = false;
 		if (SID_LDS) {
 			s_sid[threadIdx.x] = s.sid;
 			aux[0] = s.tag;
 			aux[256] = s.step;
-			aux[512] = s.flags;
+			aux[512] = s.flags & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
+		} else {
+			s.flags &= ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
 		}
-		bool run = mine, det = false, to_inel = false, dead = false;
-		float rem = SKIP ? s.safe : -1.0f;
-		for (uint32_t k = 0; k < K; ++k) {
+		float rem = s.safe;
+		// K turns, and if walks are not kept, the walks to their end
+		for (uint32_t k = 0; k < K || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
 			if (__ballot(run) == 0ull)
 				break;
-			int oc = ALIVE;
-			bool walk = false;
-			Rng rng;
-			int mat0 = s.mat, type = 0;
-			F3 nd = { 0.0f, 0.0f, 0.0f };
-			float distance = 0.0f;
-			PathInfo pinfo;
-			if (run) {
-				const uint32_t fl = SID_LDS ? aux[512] : s.flags;
-				if (fl & FL_PEND_DET) {
-					oc = DETECTED;
-				} else if (fl & FL_PEND_INEL) {
-					// an inelastic event that found no secondary slot earlier
-					if (SID_LDS)
-						aux[512] = fl & ~FL_PEND_INEL;
-					else
-						s.flags = fl & ~FL_PEND_INEL;
-					to_inel = true;
-				} else {
-					rng_start(rng, W.key0, W.key1, SID_LDS ? s_sid[threadIdx.x] : s.sid, SID_LDS ? aux[256] : s.step);
-					mat0 = s.mat;
-					oc = step_plan(W, s, rng, nd, distance, type, pinfo);
-					++my_steps;
-					walk = (oc == ALIVE);
-				}
-			}
-			const bool skip = SKIP && walk && distance <= rem;
-			float hd, saf = -1.0f;
-			int hit = propagate_wave<!MULTI, SKIP>(W.g, walk && !skip, s.p.pos, nd, distance, s.last_tri, s.mat,
-				hd, path, 256, owner_at, &saf);
-			if (SKIP && walk) {
-				if (skip) {
-					hit = -1;
-					hd = distance;
-				}
-				rem = (hit >= 0) ? -1.0f : ((skip ? rem : saf) - distance) - W.g.step_eps;
-			}
-			if (walk) {
-				int ev;
-				step_move(s, nd, distance, type, hit, hd, ev, pinfo);
-				if (SC)
-					score_free_path(sc, a.map, W, mat0, pinfo, ev);
-				if (ev == EV_INELASTIC) {
-					to_inel = true;
-				} else if (SC) {
-					float g = 0.0f;
-					int gmi = -1, gmo = -1;
-					const float e0 = s.p.E;
-					oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &g, &gmi, &gmo);
-					if (ev == EV_INTERSECT)
-						score_barrier(sc, a.map, gmi, gmo, g);
-					if (DEP_OK && a.dep)
-						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
-				} else {
-					const float e0 = s.p.E;
-					oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
-					if (DEP_OK && a.dep)
-						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
-				}
-			}
-			if (run) {
+			int oc;
+			bool inel;
+			const bool ended = step_turn<SC>(a, W, run && !f.on && k < K, s, SID_LDS ? s_sid[threadIdx.x] : s.sid,
+				SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, path, 256, owner_at, oc, inel);
+			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
 					run = false;
 				} else if (oc == TERMINATED) {
 					dead = true;
 					run = false;
-				} else if (to_inel) {
+				} else if (inel) {
+					to_inel = true;
 					run = false;
 				} else if (SID_LDS) {
 					aux[256] += 1u;
@@ -795,43 +942,113 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 			s.step = aux[256];
 			s.flags = aux[512];
 		}
-		// the multi-world kernel moves particles without a safety: clear it
-		s.safe = rem;
-		bool keep = valid && !dead;
-		const uint32_t dslot = wave_alloc(&C->det_ctr, det);
-		if (det) {
-			if (dslot < det_cap) {
-				nbl_detected r;
-				r.pos[0] = s.p.pos.x; r.pos[1] = s.p.pos.y; r.pos[2] = s.p.pos.z;
-				r.dir[0] = s.p.dir.x; r.dir[1] = s.p.dir.y; r.dir[2] = s.p.dir.z;
-				r.kin_energy = s.p.E;
-				r.tag = s.tag;
-				r.sid = s.sid;
-				a.det[dslot] = r;
-				if (SC) {
-#pragma unroll
-					for (int q = 0; q < MAX_PARAMS; ++q)
-						if (q < np)
-							a.det_sc[(size_t)dslot * np + q] = sc.v[q];
+		// a walk that goes on keeps the safety of its start point
+		s.safe = f.on ? ((float*)owner_at)[192 + __lane_id()] : rem;
+		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, &f);
+	}
+	count_steps(C, my_steps);
+}
+
+// The general variant: lanes of different worlds (flags bits 16..31), each
+// with its particle's geometry and materials from the world table, and
+// energy deposits.  Its walk gives no safety (and clears a particle's).
+template <bool SC>
+__device__ __forceinline__ void step_multi(const StepArgs& a)
+{
+	Ctrl* C = a.ctrl;
+	if (C->few)
+		return;   // k_cascade takes this launch
+	const uint32_t bi = C->buf_in;
+	const Bufs in = bi ? a.buf[1] : a.buf[0];
+	const uint32_t n_surv = C->n_surv, n_in = n_surv + C->n_se;
+	const uint32_t K = a.K;
+	const int np = a.map.np;
+	World W = a.W;
+	__shared__ int s_path[PATH_LEVELS * 256];
+	__shared__ int s_owner[4 * 64];   // per wave: owner table
+	int* path = s_path + threadIdx.x;
+	int* owner_at = s_owner + (threadIdx.x & ~63u);
+	uint32_t my_steps = 0;
+	const uint32_t stride = gridDim.x * blockDim.x;
+	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
+	for (uint32_t w0 = wave0; w0 < n_in; w0 += stride) {
+		const uint32_t i = w0 + __lane_id();
+		const bool valid = i < n_in;
+		State s = {};
+		Score sc;
+		if (valid) {
+			const uint32_t slot = in_slot(i, n_surv, a.slots);
+			s = load_state(in, slot);
+			if (SC) load_score(in, slot, np, sc);
+			const WorldDesc& wd = a.worlds[s.flags >> FL_WORLD_SHIFT];
+			W.g = wd.g;
+			W.mats = wd.mats;
+			W.nmats = wd.nmats;
+		}
+		// a step planned by another variant is walked from its start
+		bool planned = (s.flags & FL_PLANNED) != 0u;
+		bool det = (s.flags & FL_PEND_DET) != 0u, to_inel = (s.flags & FL_PEND_INEL) != 0u;
+		bool run = valid && !det && !to_inel, dead = false;
+		s.flags &= ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
+		for (uint32_t k = 0; k < K; ++k) {
+			if (__ballot(run) == 0ull)
+				break;
+			int oc = ALIVE;
+			bool walk = false;
+			Rng rng;
+			int mat0 = s.mat, type = 0;
+			F3 nd = { 0.0f, 0.0f, 0.0f };
+			float distance = 0.0f;
+			PathInfo pinfo;
+			if (run) {
+				rng_start(rng, W.key0, W.key1, s.sid, s.step);
+				oc = step_plan(W, s, rng, nd, distance, type, pinfo, planned);
+				if (!planned)
+					++my_steps;
+				planned = false;
+				walk = (oc == ALIVE);
+			}
+			float hd;
+			const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd, path, 256,
+				owner_at);
+			if (walk) {
+				int ev;
+				step_move(s, nd, distance, type, hit, hd, ev, pinfo);
+				if (SC)
+					score_free_path(sc, a.map, W, mat0, pinfo, ev);
+				if (ev == EV_INELASTIC) {
+					to_inel = true;
+				} else {
+					const float e0 = s.p.E;
+					if (SC) {
+						float g = 0.0f;
+						int gmi = -1, gmo = -1;
+						oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &g, &gmi, &gmo);
+						if (ev == EV_INTERSECT)
+							score_barrier(sc, a.map, gmi, gmo, g);
+					} else {
+						oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+					}
+					if (a.dep)
+						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
 				}
-				keep = false;
-			} else {
-				// no record slot: wait as a survivor and retry next launch
-				s.flags |= FL_PEND_DET;
+			}
+			if (run) {
+				if (oc == DETECTED) {
+					det = true;
+					run = false;
+				} else if (oc == TERMINATED) {
+					dead = true;
+					run = false;
+				} else if (to_inel) {
+					run = false;
+				} else {
+					s.step++;
+				}
 			}
 		}
-		const bool queue = keep && to_inel;
-		const bool survive = keep && !to_inel;
-		uint32_t oslot, qslot;
-		wave_alloc2(&C->step_out, survive, queue, oslot, qslot);
-		if (queue) {
-			store_state(a.inel, qslot, s);
-			if (SC) store_score(a.inel, qslot, np, sc);
-		}
-		if (survive) {
-			store_state(out, oslot, s);
-			if (SC) store_score(out, oslot, np, sc);
-		}
+		s.safe = -1.0f;
+		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, nullptr);
 	}
 	count_steps(C, my_steps);
 }
@@ -847,19 +1064,22 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 template <bool SC, bool MULTI, bool WUNI = false>
 __global__ __launch_bounds__(256) void k_step(StepArgs a)
 {
-	step_body<SC, MULTI, WUNI>(a);
+	if constexpr (MULTI)
+		step_multi<SC>(a);
+	else
+		step_body<SC, WUNI>(a);
 }
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, false>(StepArgs a)
 {
-	step_body<false, false, false>(a);
+	step_body<false, false>(a);
 }
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, true>(StepArgs a)
 {
-	step_body<false, false, true>(a);
+	step_body<false, true>(a);
 }
 
 // The inelastic events queued by k_step (drivers/gpu/gpu_driver.inl:505-540):
@@ -979,8 +1199,6 @@ template <bool SC, bool MULTI, bool WUNI>
 __device__ __forceinline__ void cascade_body(const StepArgs& a)
 {
 	static_assert(!(WUNI && (SC || MULTI)), "the world-per-wave variant is the plain one");
-	constexpr bool DEP_OK = SC || MULTI;
-	constexpr bool SKIP = !MULTI;
 	Ctrl* C = a.ctrl;
 	if (!C->few || C->n_surv + C->n_se == 0u)
 		return;
@@ -1020,6 +1238,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	// survive; the rest of the buffer is for the secondaries placed from its
 	// top (k_ctrl and the host read this launch's limit from se_limit, which
 	// no wave of it reads).
+	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	const uint32_t extra = (a.slots - n_in) / 2u / groups;
 	const uint32_t se_limit = a.slots - n_in - groups * extra;
 	if (blockIdx.x == 0 && lane == 0)
@@ -1036,15 +1255,20 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		const int hold = (int)min(64u, (uint32_t)__popcll(first) + extra);
 		State s = {};
 		Score sc;
+		InFlight f = {};
 		if (occ) {
 			const uint32_t slot = in_slot(li, n_surv, a.slots);
 			s = load_state(in, slot);
 			if (SC) load_score(in, slot, np, sc);
+			f.planned = (s.flags & FL_PLANNED) != 0u;
+			f.resume = !MULTI && (s.flags & FL_WALK) != 0u;
 			if (MULTI) {
 				const WorldDesc& wd = a.worlds[s.flags >> FL_WORLD_SHIFT];
 				Wl.g = wd.g;
 				Wl.mats = wd.mats;
 				Wl.nmats = wd.nmats;
+			} else if (f.resume) {
+				load_walk(a, bi, slot, f.w);
 			}
 		}
 		if (WUNI)   // one world a wave; its first particle names it
@@ -1053,17 +1277,18 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		bool det = (s.flags & FL_PEND_DET) != 0u;     // to be recorded
 		bool park = false;                            // waits for the next launch
 		s.flags &= FL_WORLD_MASK;
-		float rem = SKIP ? s.safe : -1.0f;
-		for (uint32_t k = 0; k < n_steps; ++k) {
+		float rem = MULTI ? -1.0f : s.safe;
+		// n_steps turns, and if walks are not kept, the walks to their end
+		for (uint32_t k = 0; k < n_steps || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
 			const uint64_t live = __ballot(occ && !park);
 			if (live == 0ull)
 				break;
 			// every wave writes at most 64 deposits a step: stop while all of
 			// them still have room in the first half of the buffer
-			if (DEP_OK && a.dep && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+			if (MULTI && a.dep && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 					+ 64ull * waves > a.dep_cap / 2u)
 				break;
-			if (pend_share * __popcll(__ballot(pend)) >= __popcll(live)) {
+			if (k < n_steps && pend_share * __popcll(__ballot(pend)) >= __popcll(live)) {
 				Particle se = {};
 				Particle pre = {};
 				bool made = false;
@@ -1135,7 +1360,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						occ = true;
 					}
 				}
-				if (DEP_OK && a.dep)
+				if (MULTI && a.dep)
 					deposit(a, C, pend && done && s.p.E != pre.E, s, pre.E);
 				if (pend) {
 					if (done) {
@@ -1150,54 +1375,57 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				}
 			}
 			const bool run = occ && !pend && !park && !det;
-			const bool walk_any = __ballot(run) != 0ull;
-			if (walk_any) {
-				int oc = ALIVE, mat0 = s.mat, type = 0;
-				bool walk = false;
-				Rng rng;
-				F3 nd = { 0.0f, 0.0f, 0.0f };
-				float distance = 0.0f;
-				PathInfo pinfo;
-				if (run) {
-					rng_start(rng, W.key0, W.key1, s.sid, s.step);
-					oc = step_plan(W, s, rng, nd, distance, type, pinfo);
-					++my_steps;
-					walk = (oc == ALIVE);
-				}
-				const bool skip = SKIP && walk && distance <= rem;
-				float hd, saf = -1.0f;
-				int hit = propagate_wave<!MULTI, SKIP>(W.g, walk && !skip, s.p.pos, nd, distance, s.last_tri, s.mat,
-					hd, path, 64, s_owner, &saf);
-				if (SKIP && walk) {
-					if (skip) {
-						hit = -1;
-						hd = distance;
+			if (__ballot(run) != 0ull) {
+				int oc = ALIVE;
+				bool ended = run;
+				if constexpr (MULTI) {
+					bool walk = false;
+					const int mat0 = s.mat;
+					int type = 0;
+					Rng rng;
+					F3 nd = { 0.0f, 0.0f, 0.0f };
+					float distance = 0.0f;
+					PathInfo pinfo;
+					if (run) {
+						rng_start(rng, W.key0, W.key1, s.sid, s.step);
+						oc = step_plan(W, s, rng, nd, distance, type, pinfo, f.planned);
+						if (!f.planned)
+							++my_steps;
+						f.planned = false;
+						walk = (oc == ALIVE);
 					}
-					rem = (hit >= 0) ? -1.0f : ((skip ? rem : saf) - distance) - W.g.step_eps;
-				}
-				if (walk) {
-					int ev;
-					step_move(s, nd, distance, type, hit, hd, ev, pinfo);
-					if (SC)
-						score_free_path(sc, a.map, W, mat0, pinfo, ev);
-					if (ev == EV_INELASTIC) {
-						pend = true;
-					} else {
-						const float e0 = s.p.E;
-						if (SC) {
-							float gr = 0.0f;
-							int gmi = -1, gmo = -1;
-							oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &gr, &gmi, &gmo);
-							if (ev == EV_INTERSECT)
-								score_barrier(sc, a.map, gmi, gmo, gr);
+					float hd;
+					const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd, path,
+						64, s_owner);
+					if (walk) {
+						int ev;
+						step_move(s, nd, distance, type, hit, hd, ev, pinfo);
+						if (SC)
+							score_free_path(sc, a.map, W, mat0, pinfo, ev);
+						if (ev == EV_INELASTIC) {
+							pend = true;
 						} else {
-							oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+							const float e0 = s.p.E;
+							if (SC) {
+								float gr = 0.0f;
+								int gmi = -1, gmo = -1;
+								oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &gr, &gmi, &gmo);
+								if (ev == EV_INTERSECT)
+									score_barrier(sc, a.map, gmi, gmo, gr);
+							} else {
+								oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+							}
+							if (a.dep)
+								deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
 						}
-						if (DEP_OK && a.dep)
-							deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
 					}
+				} else {
+					bool inel;
+					ended = step_turn<SC>(a, W, run && !f.on && k < n_steps, s, s.sid, s.step, f, rem, sc, my_steps, path,
+						64, s_owner, oc, inel);
+					pend = pend || (ended && inel);
 				}
-				if (run) {
+				if (ended) {
 					if (oc == DETECTED)
 						det = true;
 					else if (oc == TERMINATED)
@@ -1211,13 +1439,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				const uint32_t dslot = wave_alloc(&C->det_ctr, rec);
 				if (rec) {
 					if (dslot < a.det_cap) {
-						nbl_detected r;
-						r.pos[0] = s.p.pos.x; r.pos[1] = s.p.pos.y; r.pos[2] = s.p.pos.z;
-						r.dir[0] = s.p.dir.x; r.dir[1] = s.p.dir.y; r.dir[2] = s.p.dir.z;
-						r.kin_energy = s.p.E;
-						r.tag = s.tag;
-						r.sid = s.sid;
-						a.det[dslot] = r;
+						store_detected(a, dslot, s);
 						if (SC) {
 #pragma unroll
 							for (int q = 0; q < MAX_PARAMS; ++q)
@@ -1237,6 +1459,14 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		if (occ) {
 			s.flags |= (pend ? FL_PEND_INEL : 0u) | (det ? FL_PEND_DET : 0u);
 			s.safe = rem;
+			if (!MULTI && f.on) {
+				// the walk goes on in the next launch, with its start's safety
+				s.flags |= FL_PLANNED | FL_WALK;
+				s.safe = ((float*)s_owner)[192 + lane];
+				store_walk(a, bi ^ 1u, oslot, f.w);
+			} else if (MULTI && f.planned) {
+				s.flags |= FL_PLANNED;   // not taken up here
+			}
 			store_state(out, oslot, s);
 			if (SC) store_score(out, oslot, np, sc);
 		}
@@ -1261,6 +1491,14 @@ __global__ __launch_bounds__(256) void k_queue_ids(uint32_t* tag, uint64_t* sid,
 		sid[i] = sid_base + i;
 		world[i] = w;
 	}
+}
+
+// Forget the unfinished walks of a buffer's particles: their steps start
+// again, from the free path.
+__global__ __launch_bounds__(256) void k_drop_walks(Bufs b)
+{
+	for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < b.sc_stride; i += gridDim.x * blockDim.x)
+		fld_u(b, F_FLAGS)[i] &= ~FL_WALK;
 }
 
 __global__ void k_reset_det(Ctrl* c)
@@ -1297,7 +1535,7 @@ __global__ __launch_bounds__(256) void k_query(Geometry g, const float* pos, con
 	}
 	// the walk of the step kernel: whole waves, candidate tests shared
 	float od;
-	const int r = propagate_wave<true>(g, valid, p, d, dd, it, im, od, s_path + threadIdx.x, 256,
+	const int r = propagate_wave(g, valid, p, d, dd, it, im, od, s_path + threadIdx.x, 256,
 		s_owner + 4 * (threadIdx.x & ~63u));
 	if (valid) {
 		out_tri[i] = r;
@@ -1450,6 +1688,7 @@ struct nbl_driver {
 	uint32_t spill_cap;
 	Bufs inel;
 	void* inel_mem;
+	uint32_t* walk[2];      // unfinished walks of the particles of buf[0] and buf[1], or null
 	Ctrl* ctrl;
 	Ctrl* h_ctrl;
 	nbl_detected* det;
@@ -1475,6 +1714,7 @@ struct nbl_driver {
 	nbl_deposit* dep = nullptr;     // energy-deposit records (enabled when non-null)
 	uint64_t dep_cap = 0;
 	uint32_t dep_per_particle = 0;  // K + 1 when the buffer was sized
+	bool flying = false;            // particles may be in flight
 	bool dep_drained = false;       // no iteration since the last drain of deposits
 	bool use_graph = false;         // replay iterations from captured graphs
 	uint64_t epoch = 0;             // bumped when a launch argument changes
@@ -1575,20 +1815,22 @@ int collect_timing(nbl_driver* d)
 	return NBL_OK;
 }
 
-int read_ctrl(nbl_driver* d)
-{
-	HIP_OK(hipMemcpyAsync(d->h_ctrl, d->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, d->stream));
-	HIP_OK(hipStreamSynchronize(d->stream));
-	if (d->timing)
-		return collect_timing(d);
-	return NBL_OK;
-}
-
 uint32_t active_count(const Ctrl& c, uint32_t spill_cap)
 {
 	if (c.stepped)
 		return out_surv(c) + std::min(out_se(c), c.se_limit) + std::min(c.spill_ctr, spill_cap);
 	return c.n_surv + c.n_se + c.spill_n;
+}
+
+int read_ctrl(nbl_driver* d)
+{
+	HIP_OK(hipMemcpyAsync(d->h_ctrl, d->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, d->stream));
+	HIP_OK(hipStreamSynchronize(d->stream));
+	if (active_count(*d->h_ctrl, d->spill_cap) == 0)
+		d->flying = false;
+	if (d->timing)
+		return collect_timing(d);
+	return NBL_OK;
 }
 
 } // namespace
@@ -1885,6 +2127,8 @@ int nbl_driver_destroy(nbl_driver* d)
 	hipFree(d->buf_mem[1]);
 	hipFree(d->spill_mem);
 	hipFree(d->inel_mem);
+	hipFree(d->walk[0]);
+	hipFree(d->walk[1]);
 	hipFree(d->ctrl);
 	hipHostFree(d->h_ctrl);
 	hipHostFree(d->h_stage);
@@ -1953,6 +2197,11 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 	d->spill_cap = std::max<uint32_t>(1024u, std::min<uint64_t>(8ull * d->slots, 1ull << 28));
 	if ((rc = alloc_bufs(d->spill, d->spill_mem, d->spill_cap))) return cleanup(rc);
 	if ((rc = alloc_bufs(d->inel, d->inel_mem, d->slots))) return cleanup(rc);
+	// Unfinished walks, 28 bytes a slot and buffer.  Very large drivers (over
+	// 3.8 GB of them) go without: their launches finish every walk.
+	if (d->slots <= 1u << 26)
+		for (uint32_t*& w : d->walk)
+			if ((rc = dev_alloc(&w, (size_t)WALK_FIELDS * d->slots))) return cleanup(rc);
 	if ((rc = dev_alloc(&d->ctrl, 1))) return cleanup(rc);
 	if (hipHostMalloc((void**)&d->h_ctrl, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess)
 		return cleanup(fail(NBL_ERR_ALLOC, "hipHostMalloc failed"));
@@ -2198,6 +2447,8 @@ StepArgs step_args(const nbl_driver* d)
 	a.spill = d->spill;
 	a.spill_cap = d->spill_cap;
 	a.inel = d->inel;
+	a.walk[0] = d->walk[0];
+	a.walk[1] = d->walk[1];
 	a.ctrl = d->ctrl;
 	a.worlds = d->d_worlds;
 	a.perm = d->perm;
@@ -2296,6 +2547,7 @@ int nbl_driver_iterate(nbl_driver* d, uint32_t n_iter)
 	// records a particle and iteration at most.
 	const bool cascade = !d->dep || (d->dep_drained && n_iter == 1);
 	d->dep_drained = false;
+	d->flying = true;
 	if (d->use_graph && !d->timing && n_iter > 1) {
 		if ((rc = launch_graph(d, a, n_iter)))
 			return rc;
@@ -2794,6 +3046,18 @@ int nbl_driver_set_material_params(nbl_driver* d, int32_t material, float el_mfp
 	if (rc) return rc;
 	// the material arrays are read by kernels in flight: change them when idle
 	HIP_OK(hipStreamSynchronize(d->stream));
+	// steps whose walk has begun take the new parameters as well
+	if (d->flying && d->walk[0]) {
+		if ((rc = read_ctrl(d)))
+			return rc;
+		if (d->flying) {
+			for (const Bufs& b : d->buf)
+				hipLaunchKernelGGL(k_drop_walks, dim3(std::min<uint32_t>(blocks_for(d->slots), 8u * (uint32_t)d->dev->n_cu)),
+					dim3(256), 0, d->stream, b);
+			HIP_OK(hipGetLastError());
+			HIP_OK(hipStreamSynchronize(d->stream));
+		}
+	}
 	auto apply = [&](Material& m) {
 		m.el_scale = el_mfp_scale;
 		m.in_scale = in_mfp_scale;

@@ -33,6 +33,9 @@ enum { ALIVE = 0, TERMINATED = 1, DETECTED = 2 };
 enum { EV_NONE = 0, EV_INELASTIC = 1, EV_ELASTIC = 2, EV_INTERSECT = 3 };
 // Particle flags.
 constexpr uint32_t FL_PEND_INEL = 1u, FL_PEND_DET = 2u;
+// The particle's step has been planned (its direction is the normalised one,
+// the step is counted); FL_WALK: its walk has begun and is kept beside it.
+constexpr uint32_t FL_PLANNED = 4u, FL_WALK = 8u;
 // Bits 16..31 of a particle's flags: its world (geometry + material set) in
 // a driver that tracks several scans at once.
 constexpr uint32_t FL_WORLD_SHIFT = 16u, FL_WORLD_MASK = 0xffff0000u;
@@ -848,12 +851,29 @@ __device__ __forceinline__ int chunk_owner(int base, int excl, int n, int* owner
 	return v - 1;
 }
 
-// The same walk for the rays of a whole wave, with the candidate tests shared
-// out over all 64 lanes.
+// A ray on its way through the octree: where it has got to, what is left of
+// its free path, its cell (location code) and the cells it has been in.
+struct Walk {
+	F3 cur;
+	float to_go;
+	uint64_t location;
+	uint32_t cells;
+};
+__device__ __forceinline__ void walk_start(Walk& w, F3 start, float distance)
+{
+	w.cur = start;
+	w.to_go = distance;
+	w.location = 1;
+	w.cells = 0;
+}
+enum { WALK_ON = 0, WALK_END, WALK_HIT };
+
+// One cell of the same walk for the rays of a whole wave, with the candidate
+// tests shared out over all 64 lanes.
 //
 // One lane walking its own cell's triangle list leaves most of the wave idle:
 // lists differ in length, and the wave runs as long as the longest.  Here
-// every round, each walking lane enters its next cell and counts its list
+// every walking lane enters its next cell and gets its list's length
 // (g.odc); the (ray, candidate) pairs of all lists are numbered by a prefix
 // sum over lanes and screened 64 at a time, one per lane, with the owning
 // ray's origin and direction fetched across lanes (cell_may_hit: material
@@ -865,189 +885,228 @@ __device__ __forceinline__ int chunk_owner(int base, int excl, int n, int* owner
 // and tie choices are those of `propagate`.  (Testing every pair in full
 // took about 20 % more of the step kernel.)
 //
-// Every lane of the wave must call it (lanes with walk == false take part in
-// the shared tests only); a call from a partial wave falls back to
-// `propagate` lane by lane.  `owner_at` is 192 ints of LDS for this wave:
-// the owner table and the queue of pairs (triangle, owner lane).
+// Every lane of the wave must call it (lanes with active == false take part
+// in the shared tests only).  `owner_at` is 256 ints of LDS for this wave:
+// the owner table, the queue of pairs (triangle, owner lane) and safeties.
+// Returns WALK_HIT (triangle `target` at distance w.to_go - isect before the
+// end of the free path), WALK_END (no hit) or WALK_ON (moved to the next
+// cell).
 //
-// SHARED: every lane walks the same geometry.  Otherwise (lanes of different
-// scans) the candidate tests read the owning lane's triangle tables.
-//
-// SAF (with SHARED): also return in `saf` the safety of each walking lane's
-// start point (wall_safety of its first cell, and pair_safety of every
-// triangle listed there, minimised per owner in the 64 ints of LDS after
-// the owner table and queue), or -1 for a lane that does not walk.
-template <bool SHARED, bool SAF = false>
+// SAF: lanes with `first` set are in their start cell and also leave the
+// safety of their start point in owner_at[192 + lane] (as float bits):
+// wall_safety of the cell, and pair_safety of every triangle listed there,
+// minimised per owner.
+template <bool SAF>
+__device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool first, Walk& w, F3 dir,
+	int ignore_tri, int ignore_mat, int* __restrict__ path, int stride, int* owner_at, float& isect, int& target)
+{
+	const int lane = (int)__lane_id();
+	unsigned* s_saf = (unsigned*)owner_at + 192;
+	const uint64_t firsts = SAF ? __ballot(active && first) : 0ull;
+	int n = 0, off = 0;
+	target = 0;
+	isect = 0.0f;
+	if (active) {
+		float ax, ay, az, aw;
+		off = cell_find(g, w.cur, w.location, ax, ay, az, aw, path, stride, n);
+		++w.cells;
+		cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
+		if (SAF && first)
+			s_saf[lane] = __float_as_uint(fmaxf(wall_safety(g, w.cur, ax, ay, az, aw), 0.0f));
+	}
+	const int incl = wave_incl_sum(n);
+	const int excl = incl - n;
+	off -= excl;  // pair p of this lane tests od[off + p]
+	const int total = __builtin_amdgcn_readlane(incl, 63);
+	int* q_ti = owner_at + 64;
+	int* q_own = owner_at + 128;
+	int qn = 0;   // queued pairs (wave-uniform)
+	// Second stage: test the queued pairs in full and fold the results
+	// that can hit, in queue order, into their owners' running minimum.
+	auto flush = [&]() {
+		__builtin_amdgcn_wave_barrier();
+		int ti = -1, own = 0;
+		if (lane < qn) {
+			ti = q_ti[lane];
+			own = q_own[lane];
+		}
+		__builtin_amdgcn_wave_barrier();
+		const F3 oc = { __shfl(w.cur.x, own), __shfl(w.cur.y, own), __shfl(w.cur.z, own) };
+		const F3 odir = { __shfl(dir.x, own), __shfl(dir.y, own), __shfl(dir.z, own) };
+		float t = -1.0f;
+		if (lane < qn)
+			t = intersect_ray(load_tri(g.tris, ti), oc, odir);
+		uint64_t hits = __ballot(t > 0.0f);
+		while (hits) {
+			const int src = (int)__builtin_ctzll(hits);
+			hits &= hits - 1ull;
+			const float ts = __shfl(t, src);
+			const int tis = __shfl(ti, src), os = __shfl(own, src);
+			if (lane == os && ts <= isect + EPS) {
+				isect = ts;
+				target = tis;
+			}
+		}
+	};
+	for (int base = 0; base < total; base += 64) {
+		const int p = base + lane;
+		const int o = chunk_owner(base, excl, n, owner_at, lane);
+		const F3 oc = { __shfl(w.cur.x, o), __shfl(w.cur.y, o), __shfl(w.cur.z, o) };
+		const F3 odir = { __shfl(dir.x, o), __shfl(dir.y, o), __shfl(dir.z, o) };
+		const int oign_tri = __shfl(ignore_tri, o), oign_mat = __shfl(ignore_mat, o);
+		const float oto = __shfl(w.to_go, o);
+		const int ooff = __shfl(off, o);
+		bool pass = false;
+		int ti = -1;
+		if (p < total) {
+			ti = g.od[ooff + p];
+			const bool may = cell_may_hit(g, ooff + p, oc, odir, oign_mat, oto);
+			pass = may && ti != oign_tri;
+			if (SAF && ((firsts >> o) & 1ull))
+				atomicMin(s_saf + o, __float_as_uint(fmaxf(pair_safety(g, ooff + p, oc), 0.0f)));
+		}
+		const uint64_t pm = __ballot(pass);
+		const int np = (int)__popcll(pm);
+		if (qn + np > 64) {
+			flush();
+			qn = 0;
+		}
+		if (pass) {
+			const int slot = qn + (int)__popcll(pm & ((1ull << lane) - 1ull));
+			q_ti[slot] = ti;
+			q_own[slot] = o;
+		}
+		qn += np;
+	}
+	if (qn > 0)
+		flush();
+	if (!active)
+		return WALK_ON;
+	if (isect >= w.to_go)
+		return WALK_END;
+	if (target >= 0)
+		return WALK_HIT;
+	w.to_go -= isect;
+	w.cur = v_add(w.cur, v_mul(dir, isect));
+	cell_next(w.location, target, dir);
+	return (w.location > 1 && w.cells < MAX_CELLS) ? WALK_ON : WALK_END;
+}
+
+// The ancestors of a walk's cell into `path` (a walk taken up again).
+__device__ __forceinline__ void walk_path(const Geometry& g, const Walk& w, int* __restrict__ path, int stride)
+{
+	const int lev = (63 - __clzll((long long)w.location)) / 3;
+	int index = 0;
+	for (int l = 1; l < lev; ++l) {
+		index = g.odc[index + (int)((unsigned)(w.location >> (3 * (lev - l))) & 7u)].x;
+		path[(l - 1) * stride] = index;
+	}
+}
+
+// The whole walk for the rays of a wave (every lane calls; lanes with walk ==
+// false take part in the shared tests only).
 __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
-	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride, int* owner_at,
-	float* saf = nullptr)
+	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride, int* owner_at)
+{
+	Walk w;
+	walk_start(w, start, distance);
+	out_dist = distance;
+	int result = -1;
+	while (__ballot(walk) != 0ull) {
+		float isect;
+		int target;
+		const int r = walk_round<false>(g, walk, false, w, dir, ignore_tri, ignore_mat, path, stride, owner_at,
+			isect, target);
+		if (walk && r != WALK_ON) {
+			walk = false;
+			if (r == WALK_HIT) {
+				result = target;
+				out_dist = distance - w.to_go + isect;
+			}
+		}
+	}
+	return result;
+}
+
+// The walk for lanes of different geometries (the multi-world kernels, 4
+// waves per SIMD): the candidate tests read the owning lane's triangle
+// tables, and every pair is tested in full; the screen's queue and second
+// load measured slower there.
+__device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
+	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride, int* owner_at)
 {
 	out_dist = distance;
-	if (SAF)
-		*saf = -1.0f;
-	if (__ballot(1) != ~0ull) {
-		int r = -1;
-		if (walk)
-			r = propagate(g, start, dir, distance, ignore_tri, ignore_mat, out_dist, path, stride);
-		return r;
-	}
 	const int lane = (int)__lane_id();
-	F3 cur = start;
-	float to_go = distance;
-	uint64_t location = 1;
-	uint32_t cells = 0;
+	Walk w;
+	walk_start(w, start, distance);
 	int result = -1;
 	bool active = walk;
-	bool first = true;   // the walk's first round: every walking lane in its start cell
-	unsigned* s_saf = (unsigned*)owner_at + 192;
 	while (__ballot(active) != 0ull) {
 		int n = 0, off = 0, target = 0;
 		float isect = 0.0f;
 		if (active) {
 			float ax, ay, az, aw;
-			off = cell_find(g, cur, location, ax, ay, az, aw, path, stride, n);
-			++cells;
-			cell_exit(g, cur, dir, ax, ay, az, aw, isect, target);
-			if (SAF && first)
-				s_saf[lane] = __float_as_uint(fmaxf(wall_safety(g, cur, ax, ay, az, aw), 0.0f));
+			off = cell_find(g, w.cur, w.location, ax, ay, az, aw, path, stride, n);
+			++w.cells;
+			cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
 		}
 		const int incl = wave_incl_sum(n);
 		const int excl = incl - n;
 		off -= excl;  // pair p of this lane tests od[off + p]
 		const int total = __builtin_amdgcn_readlane(incl, 63);
-		if constexpr (SHARED) {
-			int* q_ti = owner_at + 64;
-			int* q_own = owner_at + 128;
-			int qn = 0;   // queued pairs (wave-uniform)
-			// Second stage: test the queued pairs in full and fold the results
-			// that can hit, in queue order, into their owners' running minimum.
-			auto flush = [&]() {
-				__builtin_amdgcn_wave_barrier();
-				int ti = -1, own = 0;
-				if (lane < qn) {
-					ti = q_ti[lane];
-					own = q_own[lane];
+		for (int base = 0; base < total; base += 64) {
+			const int p = base + lane;
+			const int o = chunk_owner(base, excl, n, owner_at, lane);
+			const F3 oc = { __shfl(w.cur.x, o), __shfl(w.cur.y, o), __shfl(w.cur.z, o) };
+			const F3 odir = { __shfl(dir.x, o), __shfl(dir.y, o), __shfl(dir.z, o) };
+			const int oign_tri = __shfl(ignore_tri, o), oign_mat = __shfl(ignore_mat, o);
+			const int ooff = __shfl(off, o);
+			Geometry og = g;
+			og.od = (const int*)shfl_ptr(g.od, o);
+			og.tris = (const float4*)shfl_ptr(g.tris, o);
+			float t = -1.0f;
+			int ti = -1;
+			if (p < total) {
+				ti = og.od[ooff + p];
+				if (ti != oign_tri)
+					t = cell_candidate(og, ti, oc, odir, oign_mat);
+			}
+			// this lane's pairs within the chunk, lanes [lo, hi)
+			uint64_t todo = 0;
+			const uint64_t can_hit = __ballot(t > 0.0f);
+			if (active) {
+				const int lo = max(excl - base, 0), hi = min(incl - base, 64);
+				if (lo < hi) {
+					const uint64_t upto = (hi == 64) ? ~0ull : ((1ull << hi) - 1ull);
+					todo = can_hit & upto & ~((1ull << lo) - 1ull);
 				}
-				__builtin_amdgcn_wave_barrier();
-				const F3 oc = { __shfl(cur.x, own), __shfl(cur.y, own), __shfl(cur.z, own) };
-				const F3 odir = { __shfl(dir.x, own), __shfl(dir.y, own), __shfl(dir.z, own) };
-				float t = -1.0f;
-				if (lane < qn)
-					t = intersect_ray(load_tri(g.tris, ti), oc, odir);
-				uint64_t hits = __ballot(t > 0.0f);
-				while (hits) {
-					const int src = (int)__builtin_ctzll(hits);
-					hits &= hits - 1ull;
-					const float ts = __shfl(t, src);
-					const int tis = __shfl(ti, src), os = __shfl(own, src);
-					if (lane == os && ts <= isect + EPS) {
+			}
+			while (__ballot(todo != 0ull) != 0ull) {
+				const int src = todo ? (int)__builtin_ctzll(todo) : lane;
+				const float ts = __shfl(t, src);
+				const int tis = __shfl(ti, src);
+				if (todo) {
+					if (ts <= isect + EPS) {
 						isect = ts;
 						target = tis;
 					}
-				}
-			};
-			for (int base = 0; base < total; base += 64) {
-				const int p = base + lane;
-				const int o = chunk_owner(base, excl, n, owner_at, lane);
-				const F3 oc = { __shfl(cur.x, o), __shfl(cur.y, o), __shfl(cur.z, o) };
-				const F3 odir = { __shfl(dir.x, o), __shfl(dir.y, o), __shfl(dir.z, o) };
-				const int oign_tri = __shfl(ignore_tri, o), oign_mat = __shfl(ignore_mat, o);
-				const float oto = __shfl(to_go, o);
-				const int ooff = __shfl(off, o);
-				bool pass = false;
-				int ti = -1;
-				if (p < total) {
-					ti = g.od[ooff + p];
-					const bool may = cell_may_hit(g, ooff + p, oc, odir, oign_mat, oto);
-					pass = may && ti != oign_tri;
-					if (SAF && first)
-						atomicMin(s_saf + o, __float_as_uint(fmaxf(pair_safety(g, ooff + p, oc), 0.0f)));
-				}
-				const uint64_t pm = __ballot(pass);
-				const int np = (int)__popcll(pm);
-				if (qn + np > 64) {
-					flush();
-					qn = 0;
-				}
-				if (pass) {
-					const int slot = qn + (int)__popcll(pm & ((1ull << lane) - 1ull));
-					q_ti[slot] = ti;
-					q_own[slot] = o;
-				}
-				qn += np;
-			}
-			if (qn > 0)
-				flush();
-			if (SAF && first) {
-				__builtin_amdgcn_wave_barrier();
-				if (walk)
-					*saf = __uint_as_float(s_saf[lane]);
-				__builtin_amdgcn_wave_barrier();
-			}
-		} else {
-			// Lanes of different worlds (the multi-world kernel, 4 waves per
-			// SIMD): every pair is tested in full; the screen's queue and
-			// second load measured slower there.
-			for (int base = 0; base < total; base += 64) {
-				const int p = base + lane;
-				const int o = chunk_owner(base, excl, n, owner_at, lane);
-				const F3 oc = { __shfl(cur.x, o), __shfl(cur.y, o), __shfl(cur.z, o) };
-				const F3 odir = { __shfl(dir.x, o), __shfl(dir.y, o), __shfl(dir.z, o) };
-				const int oign_tri = __shfl(ignore_tri, o), oign_mat = __shfl(ignore_mat, o);
-				const int ooff = __shfl(off, o);
-				Geometry og = g;
-				og.od = (const int*)shfl_ptr(g.od, o);
-				og.tris = (const float4*)shfl_ptr(g.tris, o);
-				float t = -1.0f;
-				int ti = -1;
-				if (p < total) {
-					ti = og.od[ooff + p];
-					if (ti != oign_tri)
-						t = cell_candidate(og, ti, oc, odir, oign_mat);
-				}
-				// this lane's pairs within the chunk, lanes [lo, hi)
-				uint64_t todo = 0;
-				const uint64_t can_hit = __ballot(t > 0.0f);
-				if (active) {
-					const int lo = max(excl - base, 0), hi = min(incl - base, 64);
-					if (lo < hi) {
-						const uint64_t upto = (hi == 64) ? ~0ull : ((1ull << hi) - 1ull);
-						todo = can_hit & upto & ~((1ull << lo) - 1ull);
-					}
-				}
-				while (__ballot(todo != 0ull) != 0ull) {
-					const int src = todo ? (int)__builtin_ctzll(todo) : lane;
-					const float ts = __shfl(t, src);
-					const int tis = __shfl(ti, src);
-					if (todo) {
-						if (ts <= isect + EPS) {
-							isect = ts;
-							target = tis;
-						}
-						todo &= todo - 1ull;
-					}
+					todo &= todo - 1ull;
 				}
 			}
 		}
-		first = false;
 		if (active) {
-			if (isect >= to_go) {
-				out_dist = distance;
-				result = -1;
+			if (isect >= w.to_go) {
 				active = false;
 			} else if (target >= 0) {
-				out_dist = distance - to_go + isect;
+				out_dist = distance - w.to_go + isect;
 				result = target;
 				active = false;
 			} else {
-				to_go -= isect;
-				cur = v_add(cur, v_mul(dir, isect));
-				cell_next(location, target, dir);
-				if (!(location > 1 && cells < MAX_CELLS)) {
-					out_dist = distance;
-					result = -1;
+				w.to_go -= isect;
+				w.cur = v_add(w.cur, v_mul(dir, isect));
+				cell_next(w.location, target, dir);
+				if (!(w.location > 1 && w.cells < MAX_CELLS))
 					active = false;
-				}
 			}
 		}
 	}
@@ -1390,9 +1449,10 @@ struct WorldDesc {
 //
 // step_plan: domain and energy checks and path sampling.  Returns ALIVE or
 // TERMINATED; for ALIVE, `distance` and `type` are the free path and its
-// mechanism (0 in vacuum), `nd` the normalised direction.
+// mechanism (0 in vacuum), `nd` the normalised direction (the direction
+// itself when the step was `planned` before, FL_PLANNED).
 __device__ __forceinline__ int step_plan(const World& W, const State& s, Rng& rng, F3& nd, float& distance,
-	int& type, PathInfo& pinfo)
+	int& type, PathInfo& pinfo, bool planned = false)
 {
 	pinfo.type = 0;
 	pinfo.logE = 0.0f;
@@ -1416,7 +1476,7 @@ __device__ __forceinline__ int step_plan(const World& W, const State& s, Rng& rn
 		if (pi < dist) { type = 1; dist = pi; }
 		distance = dist;
 	}
-	nd = normalised(s.p.dir);
+	nd = planned ? s.p.dir : normalised(s.p.dir);
 	pinfo.tau_el = tau_el;
 	pinfo.tau_in = tau_in;
 	return ALIVE;

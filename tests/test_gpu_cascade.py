@@ -87,3 +87,21 @@ def test_both_routes_give_the_same(world, kind, few):
         return np.sort(det, order="sid").tobytes(), more, steps
 
     assert track(few) == track(None)
+
+
+@pytest.mark.parametrize("few", [0, None])
+def test_walks_kept_between_launches(world, few):
+    """With many particles in flight a launch leaves unfinished walks to the
+    next one: records and step counts equal the oracle's."""
+    dev, mats, geoms, oracles = world
+    n = 70000
+    pri = W.raster_scan(100, 100, 7, 260.0, -140.0, 140.0, -140.0, 140.0, 37.0, seed=6)
+    d = A.Driver(dev, 1 << 18, geoms["grating"], mats, seed=21, steps_per_launch=3)
+    if few is not None:
+        d.set_cascade(few)
+    d.push(pri, np.arange(n, dtype=np.uint32), sid_base=5)
+    det = d.run(4 * n)
+    ref, steps = oracles["grating"].run_philox(pri, 21, 4 * n, threads=16, sid_base=5)
+    assert d.steps() == steps
+    assert np.sort(det, order="sid").tobytes() == np.sort(ref.astype(det.dtype), order="sid").tobytes()
+    d.close()
