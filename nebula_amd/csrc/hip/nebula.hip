@@ -126,7 +126,7 @@ struct StepArgs {
 	// then finishes its walks
 	uint32_t* walk[2];
 };
-constexpr uint32_t WALK_FIELDS = 7;
+constexpr uint32_t WALK_FIELDS = 6;
 // Particles in flight from which a launch leaves walks unfinished: with so
 // many some steps end in every launch, which the callers' checks for a run
 // that makes no progress count on.
@@ -661,8 +661,8 @@ __device__ __forceinline__ void load_walk(const StepArgs& a, uint32_t buf, uint3
 	const size_t n = a.slots;
 	w.cur = { __uint_as_float(p[slot]), __uint_as_float(p[n + slot]), __uint_as_float(p[2 * n + slot]) };
 	w.to_go = __uint_as_float(p[3 * n + slot]);
-	w.location = ((uint64_t)p[5 * n + slot] << 32) | p[4 * n + slot];
-	w.cells = p[6 * n + slot];
+	w.cell = p[4 * n + slot];
+	w.cells = p[5 * n + slot];
 }
 
 __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const Walk& w)
@@ -673,9 +673,8 @@ __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint
 	p[n + slot] = __float_as_uint(w.cur.y);
 	p[2 * n + slot] = __float_as_uint(w.cur.z);
 	p[3 * n + slot] = __float_as_uint(w.to_go);
-	p[4 * n + slot] = (uint32_t)w.location;
-	p[5 * n + slot] = (uint32_t)(w.location >> 32);
-	p[6 * n + slot] = w.cells;
+	p[4 * n + slot] = w.cell;
+	p[5 * n + slot] = w.cells;
 }
 
 // One turn of a wave (every lane calls): lanes with `plan` set plan their
@@ -700,7 +699,7 @@ __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint
 // inelastic event is to follow), DETECTED or TERMINATED.
 template <bool SC>
 __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, bool plan, State& s, uint64_t sid,
-	uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* path, int stride, int* owner_at,
+	uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* owner_at,
 	int& oc, bool& to_inel)
 {
 	oc = ALIVE;
@@ -726,12 +725,10 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 			skip = !f.resume && f.distance <= rem;
 			f.on = !skip;
 			f.first = !f.resume;
-			if (f.resume) {
-				walk_path(W.g, f.w, path, stride);
+			if (f.resume)
 				((float*)owner_at)[192 + __lane_id()] = rem;
-			} else if (!skip) {
-				walk_start(f.w, s.p.pos, f.distance);
-			}
+			else if (!skip)
+				walk_start(W.g, f.w, s.p.pos, f.distance);
 		} else {
 			ended = true;
 		}
@@ -743,7 +740,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 	if (__ballot(f.on) != 0ull) {
 		float isect;
 		int target;
-		const int r = walk_round<true>(W.g, f.on, f.first, f.w, s.p.dir, s.last_tri, s.mat, path, stride, owner_at,
+		const int r = walk_round<true>(W.g, f.on, f.first, f.w, s.p.dir, s.last_tri, s.mat, owner_at,
 			isect, target);
 		f.first = false;
 		if (f.on && r != WALK_ON) {
@@ -853,7 +850,6 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	World Wl = a.W;
 	const World& W = WUNI ? Wl : a.W;
-	__shared__ int s_path[PATH_LEVELS * 256];
 	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
 	// In the plain variant a particle's stream id waits here during its steps
 	// (each step reads it once to start its Philox stream), and with it its
@@ -863,7 +859,6 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	__shared__ uint32_t s_aux[SID_LDS ? 3 * 256 : 1];
 	uint32_t* const aux = s_aux + (SID_LDS ? threadIdx.x : 0u);
 
-	int* path = s_path + threadIdx.x;
 	int* owner_at = s_owner + 4 * (threadIdx.x & ~63u);
 	uint32_t my_steps = 0;
 	const uint32_t stride = gridDim.x * blockDim.x;
@@ -918,7 +913,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 			int oc;
 			bool inel;
 			const bool ended = step_turn<SC>(a, W, run && !f.on && k < K, s, SID_LDS ? s_sid[threadIdx.x] : s.sid,
-				SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, path, 256, owner_at, oc, inel);
+				SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, owner_at, oc, inel);
 			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
@@ -964,9 +959,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 	const uint32_t K = a.K;
 	const int np = a.map.np;
 	World W = a.W;
-	__shared__ int s_path[PATH_LEVELS * 256];
 	__shared__ int s_owner[4 * 64];   // per wave: owner table
-	int* path = s_path + threadIdx.x;
 	int* owner_at = s_owner + (threadIdx.x & ~63u);
 	uint32_t my_steps = 0;
 	const uint32_t stride = gridDim.x * blockDim.x;
@@ -1009,7 +1002,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 				walk = (oc == ALIVE);
 			}
 			float hd;
-			const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd, path, 256,
+			const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd,
 				owner_at);
 			if (walk) {
 				int ev;
@@ -1209,10 +1202,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	const int np = a.map.np;
 	World Wl = a.W;
 	const World& W = (MULTI || WUNI) ? Wl : a.W;
-	__shared__ int s_path[PATH_LEVELS * 64];
 	__shared__ int s_owner[4 * 64];   // owner table, pair queue, safeties
 	const uint32_t lane = threadIdx.x;
-	int* const path = s_path + lane;
 	const uint64_t below = (1ull << lane) - 1ull;
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
@@ -1395,8 +1386,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						walk = (oc == ALIVE);
 					}
 					float hd;
-					const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd, path,
-						64, s_owner);
+					const int hit = propagate_wave_multi(W.g, walk, s.p.pos, nd, distance, s.last_tri, s.mat, hd,
+						s_owner);
 					if (walk) {
 						int ev;
 						step_move(s, nd, distance, type, hit, hd, ev, pinfo);
@@ -1421,8 +1412,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					}
 				} else {
 					bool inel;
-					ended = step_turn<SC>(a, W, run && !f.on && k < n_steps, s, s.sid, s.step, f, rem, sc, my_steps, path,
-						64, s_owner, oc, inel);
+					ended = step_turn<SC>(a, W, run && !f.on && k < n_steps, s, s.sid, s.step, f, rem, sc, my_steps,
+						s_owner, oc, inel);
 					pend = pend || (ended && inel);
 				}
 				if (ended) {
@@ -1519,7 +1510,6 @@ __global__ __launch_bounds__(256) void k_query(Geometry g, const float* pos, con
 	const float* dist, const int* ignore_tri, const int* ignore_mat, int* out_tri,
 	float* out_dist, uint32_t n)
 {
-	__shared__ int s_path[PATH_LEVELS * 256];
 	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	const bool valid = i < n;
@@ -1535,7 +1525,7 @@ __global__ __launch_bounds__(256) void k_query(Geometry g, const float* pos, con
 	}
 	// the walk of the step kernel: whole waves, candidate tests shared
 	float od;
-	const int r = propagate_wave(g, valid, p, d, dd, it, im, od, s_path + threadIdx.x, 256,
+	const int r = propagate_wave(g, valid, p, d, dd, it, im, od,
 		s_owner + 4 * (threadIdx.x & ~63u));
 	if (valid) {
 		out_tri[i] = r;
@@ -1573,7 +1563,6 @@ __global__ __launch_bounds__(256) void k_probe(Material m, int which, int mode, 
 __global__ __launch_bounds__(256) void k_step_states(World W, nbl_step_state* st, int* event,
 	int* outcome, nbl_step_state* se_out, int* se_made_out, uint32_t n)
 {
-	__shared__ int s_path[PATH_LEVELS * 256];
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
 		return;
@@ -1589,7 +1578,7 @@ __global__ __launch_bounds__(256) void k_step_states(World W, nbl_step_state* st
 	rng_start(rng, W.key0, W.key1, s.sid, s.step);
 	int ev = EV_NONE, hit = -1;
 	PathInfo pinfo;
-	int oc = step_init(W, s, rng, ev, hit, s_path + threadIdx.x, 256, pinfo);
+	int oc = step_init(W, s, rng, ev, hit, pinfo);
 	Particle se;
 	bool made = false;
 	if (oc == ALIVE)
@@ -1664,7 +1653,9 @@ struct nbl_geometry {
 	int* od;
 	float4* tris;
 	float4* scr;
-	int2* odc;
+	float4* cells;
+	uint32_t* next;
+	uint32_t* start;
 	Geometry g;
 	int max_material;   // largest physical material index named by a triangle
 };
@@ -1803,6 +1794,115 @@ int alloc_bufs(Bufs& b, void*& mem, uint32_t slots)
 	return NBL_OK;
 }
 
+// The tables of an octree's cells (Geometry: cells, next, start), built from
+// the root down.
+struct Cells {
+	std::vector<float4> rec;
+	std::vector<uint32_t> next, start;
+	std::vector<uint32_t> inner;      // the inner cells, in the order they are split in
+	std::vector<uint8_t> inner_depth;
+	float half[3], lo[3], inv[3];
+	float start_eps = 0.0f;
+	uint32_t start_bits = 0;
+
+	static float bits(int32_t v)
+	{
+		float f;
+		std::memcpy(&f, &v, 4);
+		return f;
+	}
+	static int32_t word(float f)
+	{
+		int32_t v;
+		std::memcpy(&v, &f, 4);
+		return v;
+	}
+
+	void root(const float center[3], const float halfsize[3])
+	{
+		std::memcpy(half, halfsize, sizeof(half));
+		rec = { make_float4(center[0], center[1], center[2], 1.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f) };
+		next.assign(8, 0u);
+		inner = { 0u };
+		inner_depth = { 0 };
+	}
+
+	// The children of the k-th inner cell: inner cells, or leaves with
+	// list[o] (the negative start in the table) and length[o].
+	void split(size_t k, const bool inner_child[8], const int32_t list[8], const int32_t length[8])
+	{
+		const uint32_t up = inner[k], first = (uint32_t)(rec.size() / 2);
+		const float4 c = rec[2 * (size_t)up];
+		// octree.inl: centre +- halfsize times the scale; the product with
+		// +-0.5 is exact, and scaling by a power of two commutes with rounding
+		// (halfsize >= 1 nm and scale >= 2^-21 stay far from underflow)
+		const float hw = 0.5f * c.w;
+		const float h[3] = { hw * half[0], hw * half[1], hw * half[2] };
+		rec[2 * (size_t)up + 1].x = bits((int32_t)first);
+		rec.resize(rec.size() + 16);
+		next.resize(next.size() + 64, 0u);
+		for (uint32_t o = 0; o < 8; ++o) {
+			const uint32_t i = first + o;
+			rec[2 * (size_t)i] = make_float4(c.x + ((o & 1u) ? h[0] : -h[0]), c.y + ((o & 2u) ? h[1] : -h[1]),
+				c.z + ((o & 4u) ? h[2] : -h[2]), hw);
+			rec[2 * (size_t)i + 1] = make_float4(bits(list[o]), bits(length[o]), 0.0f, 0.0f);
+			// the deepest level at which the move stays inside the parent
+			for (uint32_t axis = 0; axis < 3; ++axis)
+				for (uint32_t low = 0; low < 2; ++low) {
+					const uint32_t m = 1u << axis;
+					const bool inside = (o & m) == (low ? m : 0u);
+					next[8 * (size_t)i + 2 * axis + low] = inside ? first + (o ^ m) : next[8 * (size_t)up + 2 * axis + low];
+				}
+			if (inner_child[o]) {
+				inner.push_back(i);
+				inner_depth.push_back((uint8_t)(inner_depth[k] + 1));
+			}
+		}
+	}
+
+	// Fill level `depth` of the start grid below cell i.
+	void fill(uint32_t i, uint32_t depth, uint32_t x, uint32_t y, uint32_t z)
+	{
+		const int32_t child = word(rec[2 * (size_t)i + 1].x);
+		const uint32_t b = start_bits;
+		if (depth == b || child < 0) {
+			const uint32_t n = 1u << (b - depth);
+			for (uint32_t u = z * n; u < (z + 1) * n; ++u)
+				for (uint32_t v = y * n; v < (y + 1) * n; ++v)
+					std::fill_n(start.begin() + (((size_t)u << b | v) << b) + (size_t)x * n, n, i);
+			return;
+		}
+		for (uint32_t o = 0; o < 8; ++o)
+			fill((uint32_t)child + o, depth + 1, 2 * x + (o & 1u), 2 * y + ((o >> 1) & 1u), 2 * z + (o >> 2));
+	}
+
+	// The start grid: a level with about as many cells as the tree has leaves,
+	// 2^18 at most (1 MB), as long as its walls are far enough apart.
+	void make_start()
+	{
+		const size_t leaves = rec.size() / 2;
+		for (start_bits = 0; start_bits < 6u && (8ull << (3 * start_bits)) <= leaves;)
+			++start_bits;
+		for (;; --start_bits) {
+			// rounding of t in cell_start and of the walls (a sum of one term a
+			// level), in widths of the grid's cells, with a factor of four
+			start_eps = 0.0f;
+			for (int a = 0; a < 3; ++a) {
+				const float c = a == 0 ? rec[0].x : a == 1 ? rec[0].y : rec[0].z;
+				lo[a] = c - half[a];
+				inv[a] = std::ldexp(0.5f, (int)start_bits) / half[a];
+				const float far = (std::fabs(c) + half[a]) / (2.0f * half[a]);
+				start_eps = std::max(start_eps,
+					std::ldexp(8.0f + ((float)start_bits + 1.0f) * far, (int)start_bits - 22));
+			}
+			if (start_bits == 0 || start_eps < 0.03f)
+				break;
+		}
+		start.assign((size_t)1 << (3 * start_bits), 0u);
+		fill(0u, 0u, 0u, 0u, 0u);
+	}
+};
+
 int collect_timing(nbl_driver* d)
 {
 	for (auto& pr : d->ev_used) {
@@ -1899,33 +1999,38 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 		return fail(NBL_ERR_ARG, "invalid geometry arguments");
 	// Walk the whole table once: every child offset must point at a node
 	// inside it and every leaf entry at a triangle, so that the traversal
-	// kernel cannot read out of bounds.
+	// kernel cannot read out of bounds.  The cells are numbered on the way
+	// (Cells below), level by level.
+	Cells cells;
 	{
-		// (node offset, depth); leaves may sit at depth 21 at most (the
-		// builder's limit, which the 64-bit location code and the per-level
-		// path cache of the walk rely on)
+		// leaves may sit at depth 21 at most (the builder's limit)
 		std::vector<uint8_t> seen((size_t)n_od, 0);
-		std::vector<std::pair<int64_t, int>> stack{ { 0, 0 } };
 		seen[0] = 1;
-		while (!stack.empty()) {
-			const int64_t node = stack.back().first;
-			const int depth = stack.back().second;
-			stack.pop_back();
+		cells.root(center, halfsize);
+		// nodes[k]: offset in the table of the k-th inner cell
+		std::vector<int64_t> nodes{ 0 };
+		for (size_t k = 0; k < nodes.size(); ++k) {
+			const int64_t node = nodes[k];
+			const int depth = cells.inner_depth[k];
 			if (node + 8 > n_od)
 				return fail(NBL_ERR_FORMAT, "octree node out of range at " + std::to_string(node));
-			if (depth + 1 > PATH_LEVELS)
+			if (depth + 1 > MAX_DEPTH)
 				return fail(NBL_ERR_FORMAT, "octree deeper than 21 levels");
+			bool inner[8] = {};
+			int32_t list[8] = {}, length[8] = {};
 			for (int o = 0; o < 8; ++o) {
 				const int64_t v = od[node + o];
 				if (v > 0) {
 					if (v >= n_od || seen[v])
 						return fail(NBL_ERR_FORMAT, "bad octree child offset at " + std::to_string(node + o));
 					seen[v] = 1;
-					stack.push_back({ v, depth + 1 });
+					nodes.push_back(v);
+					inner[o] = true;
 				} else {
 					int64_t p = -v;
 					if (p <= 0 || p >= n_od)
 						return fail(NBL_ERR_FORMAT, "bad octree leaf offset at " + std::to_string(node + o));
+					list[o] = (int32_t)v;
 					for (;; ++p) {
 						if (p >= n_od)
 							return fail(NBL_ERR_FORMAT, "unterminated octree leaf");
@@ -1934,9 +2039,12 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 						if (od[p] >= ntri)
 							return fail(NBL_ERR_FORMAT, "octree leaf names triangle " + std::to_string(od[p]));
 					}
+					length[o] = (int32_t)(p + v);
 				}
 			}
+			cells.split(k, inner, list, length);
 		}
+		cells.make_start();
 	}
 	int rc = set_device(dev);
 	if (rc) return rc;
@@ -1949,18 +2057,16 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 			return fail(NBL_ERR_ARG, "triangle " + std::to_string(i) + ": material id outside the 16-bit range");
 		}
 	if ((rc = dev_alloc(&g->od, (size_t)n_od)) || (rc = dev_alloc(&g->tris, (size_t)ntri * 3))
-		|| (rc = dev_alloc(&g->scr, (size_t)n_od * 2)) || (rc = dev_alloc(&g->odc, (size_t)n_od))) {
+		|| (rc = dev_alloc(&g->scr, (size_t)n_od * 2)) || (rc = dev_alloc(&g->cells, cells.rec.size()))
+		|| (rc = dev_alloc(&g->next, cells.next.size())) || (rc = dev_alloc(&g->start, cells.start.size()))) {
 		hipFree(g->od);
 		hipFree(g->tris);
 		hipFree(g->scr);
+		hipFree(g->cells);
+		hipFree(g->next);
 		delete g;
 		return rc;
 	}
-	// cnt[i]: number of triangle entries from od[i] up to the next negative
-	// entry (the length of a leaf list when i is its start)
-	std::vector<int32_t> cnt((size_t)n_od, 0);
-	for (int64_t i = n_od - 1; i >= 0; --i)
-		cnt[i] = (od[i] < 0 || i + 1 == n_od) ? 0 : cnt[i + 1] + 1;
 	std::vector<float4> packed((size_t)ntri * 3), tscr((size_t)ntri * 2);
 	for (int64_t i = 0; i < ntri; ++i) {
 		const nbl_triangle44& t = tris[i];
@@ -1995,18 +2101,20 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 	HIP_OK(hipMemcpy(g->od, od, sizeof(int32_t) * n_od, hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->tris, packed.data(), sizeof(float4) * packed.size(), hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->scr, scr.data(), sizeof(float4) * scr.size(), hipMemcpyHostToDevice));
-	// child entries with their list lengths (leaf offsets are checked above
-	// to lie in (0, n_od))
-	std::vector<int2> odc((size_t)n_od);
-	for (int64_t i = 0; i < n_od; ++i) {
-		const int32_t v = od[i];
-		odc[i] = make_int2(v, (v < 0 && (int64_t)-(int64_t)v < n_od) ? cnt[(size_t)-(int64_t)v] : 0);
-	}
-	HIP_OK(hipMemcpy(g->odc, odc.data(), sizeof(int2) * n_od, hipMemcpyHostToDevice));
+	HIP_OK(hipMemcpy(g->cells, cells.rec.data(), sizeof(float4) * cells.rec.size(), hipMemcpyHostToDevice));
+	HIP_OK(hipMemcpy(g->next, cells.next.data(), sizeof(uint32_t) * cells.next.size(), hipMemcpyHostToDevice));
+	HIP_OK(hipMemcpy(g->start, cells.start.data(), sizeof(uint32_t) * cells.start.size(), hipMemcpyHostToDevice));
 	g->g.od = g->od;
 	g->g.tris = g->tris;
 	g->g.scr = g->scr;
-	g->g.odc = g->odc;
+	g->g.cells = g->cells;
+	g->g.next = g->next;
+	g->g.start = g->start;
+	g->g.lo = { cells.lo[0], cells.lo[1], cells.lo[2] };
+	g->g.inv = { cells.inv[0], cells.inv[1], cells.inv[2] };
+	g->g.start_eps = cells.start_eps;
+	g->g.start_bits = cells.start_bits;
+	g->g.start_n = std::ldexp(1.0f, (int)cells.start_bits);
 	g->g.center = { center[0], center[1], center[2] };
 	g->g.halfsize = { halfsize[0], halfsize[1], halfsize[2] };
 	// octree.inl:298-300: 2 |halfsize|, CPU expression order
@@ -2031,7 +2139,9 @@ int nbl_geometry_destroy(nbl_geometry* g)
 	hipFree(g->od);
 	hipFree(g->tris);
 	hipFree(g->scr);
-	hipFree(g->odc);
+	hipFree(g->cells);
+	hipFree(g->next);
+	hipFree(g->start);
 	delete g;
 	return NBL_OK;
 }
@@ -2197,8 +2307,8 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 	d->spill_cap = std::max<uint32_t>(1024u, std::min<uint64_t>(8ull * d->slots, 1ull << 28));
 	if ((rc = alloc_bufs(d->spill, d->spill_mem, d->spill_cap))) return cleanup(rc);
 	if ((rc = alloc_bufs(d->inel, d->inel_mem, d->slots))) return cleanup(rc);
-	// Unfinished walks, 28 bytes a slot and buffer.  Very large drivers (over
-	// 3.8 GB of them) go without: their launches finish every walk.
+	// Unfinished walks, 24 bytes a slot and buffer.  Very large drivers (over
+	// 3.2 GB of them) go without: their launches finish every walk.
 	if (d->slots <= 1u << 26)
 		for (uint32_t*& w : d->walk)
 			if ((rc = dev_alloc(&w, (size_t)WALK_FIELDS * d->slots))) return cleanup(rc);

@@ -497,10 +497,25 @@ struct Geometry {
 	// neighbouring records for neighbouring pairs, without waiting for the
 	// triangle index.
 	const float4* scr;
-	// odc[i] = (od[i], length of the leaf list at -od[i] when od[i] < 0
-	// names one): the walk reads a child entry and its list length in one
-	// load.
-	const int2* odc;
+	// The octree's cells, inner ones and leaves, numbered from 1 with the
+	// eight children of a cell in a row (0: the root).  cells[2 i]: centre and
+	// scale (half extents over the root's) of cell i, with the roundings of
+	// the reference's descent; cells[2 i + 1] in integer bits: for an inner
+	// cell its first child, for a leaf the negative start of its list in `od`
+	// and the list's length.
+	const float4* cells;
+	// next[8 i + 2 axis + (0 or 1)]: the cell that a ray leaving leaf i
+	// through its upper (0) or lower (1) wall of that axis enters, or an inner
+	// cell that holds it; 0: none, the ray leaves the octree
+	const uint32_t* next;
+	// The cells of one level of the tree by position: start[(z << 2 b) + (y <<
+	// b) + x], b = start_bits, with x = (pos - lo) * inv rounded down; a leaf
+	// above that level fills its part.  A position closer than start_eps (in
+	// these cells' widths) to one of their walls starts at the root instead.
+	const uint32_t* start;
+	F3 lo, inv;
+	float start_eps, start_n;   // start_n: 2^b
+	uint32_t start_bits;
 	F3 center, halfsize;
 	float max_extent;
 	int ntri;
@@ -540,72 +555,52 @@ __device__ __forceinline__ bool in_domain(const Geometry& g, F3 p)
 		&& (p.z > c.z - h.z) && (p.z < c.z + h.z);
 }
 
-// Levels of the octree table cached per thread: path[(l - 1) * stride] holds
-// the node index at level l (1..21) of the current cell.
-constexpr int PATH_LEVELS = 21;
+// Levels of the octree at most (the builder's limit).
+constexpr int MAX_DEPTH = 21;
 
 // The pieces of the cell walk of geometry/octree.inl:32-192.
 //
-// The reference re-descends from the root for every cell.  Here the node
-// indices of the current cell's ancestors are kept in LDS (`path`, one int
-// per level, lane-strided), so moving to a neighbour loads only the flipped
-// level and whatever lies below it.  The cell-centre arithmetic still runs
-// from the root in the reference's order, so every value is unchanged.
+// The reference finds every cell by a descent from the root, adding up the
+// centre on the way, and its neighbour by flipping bits of a location code.
+// Both depend on the cell alone, so they are tables here: a cell's centre and
+// scale as that descent rounds them, and the cell a location code with its
+// bits flipped names.  A walk starts from the cell that one level's grid names
+// for its position and goes down the few levels that are left (comparing with
+// the centres as the reference does), and a move to the next cell reads one
+// entry.  (With descents of seven levels from the root for every walk and
+// the centre added up again for every further cell: 6 553 600 primaries of
+// 300 eV on a grating 294 ms, now 288; 160 000 of 1 keV on contact holes 21.5
+// and 21.0; 2046 of 300 eV 1.72 and 1.68.)
 //
-// cell_find: centre (ax, ay, az) and scale aw of the leaf holding `cur`,
-// extending `location` down to it; returns the start of its triangle list
-// and its length in `count`.
-__device__ __forceinline__ int cell_find(const Geometry& g, F3 cur, uint64_t& location,
-	float& ax, float& ay, float& az, float& aw, int* __restrict__ path, int stride, int& count)
+// cell_start: the cell in which a walk from `p` begins its descent.
+__device__ __forceinline__ uint32_t cell_start(const Geometry& g, F3 p)
 {
-	const int2* __restrict__ odc = g.odc;
-	const F3 hs = g.halfsize;
-	// The reference adds aw * hs * (bit - 0.5) per level.  The product with
-	// +-0.5 is exact, and scaling by a power of two commutes with rounding
-	// (aw >= 2^-21 and hs >= 1 nm keep every product far from underflow), so
-	// it equals +-(hw * hs) with hw = aw / 2: the same bits in three
-	// operations per axis instead of six.
-	ax = g.center.x; ay = g.center.y; az = g.center.z;
-	float hw = 0.5f;
-	const int clz = __clzll((long long)location);
-	for (int i = 60 - clz; i >= 0; i -= 3) {
-		const unsigned oct = (unsigned)(location >> i) & 7u;
-		const float hx = hw * hs.x, hy = hw * hs.y, hz = hw * hs.z;
-		ax += (oct & 1u) ? hx : -hx;
-		ay += (oct & 2u) ? hy : -hy;
-		az += (oct & 4u) ? hz : -hz;
-		hw *= 0.5f;
+	const float tx = (p.x - g.lo.x) * g.inv.x, ty = (p.y - g.lo.y) * g.inv.y, tz = (p.z - g.lo.z) * g.inv.z;
+	const float fx = __builtin_amdgcn_fractf(tx), fy = __builtin_amdgcn_fractf(ty), fz = __builtin_amdgcn_fractf(tz);
+	// near a wall, where the rounding of t could name the other side, and
+	// outside the domain (also for a NaN): from the root
+	if (!(tx >= 0.0f && ty >= 0.0f && tz >= 0.0f && fmaxf(fmaxf(tx, ty), tz) < g.start_n
+			&& fminf(fminf(fx, fy), fz) >= g.start_eps && fmaxf(fmaxf(fx, fy), fz) <= 1.0f - g.start_eps))
+		return 0u;
+	return g.start[((((uint32_t)tz << g.start_bits) | (uint32_t)ty) << g.start_bits) | (uint32_t)tx];
+}
+
+// cell_find: the leaf that holds `cur`, from `cell` downwards, with its centre
+// (ax, ay, az) and scale aw; returns the start of its triangle list and its
+// length in `count`.
+__device__ __forceinline__ int cell_find(const Geometry& g, F3 cur, uint32_t& cell,
+	float& ax, float& ay, float& az, float& aw, int& count)
+{
+	for (;;) {
+		const float4 a = g.cells[2 * (size_t)cell];
+		const int2 e = *(const int2*)(g.cells + 2 * (size_t)cell + 1);
+		if (e.x < 0) {
+			ax = a.x; ay = a.y; az = a.z; aw = a.w;
+			count = e.y;
+			return -e.x;
+		}
+		cell = (uint32_t)e.x + ((cur.x > a.x) ? 1u : 0u) + ((cur.y > a.y) ? 2u : 0u) + ((cur.z > a.z) ? 4u : 0u);
 	}
-	// levels 1..L-1 are unchanged ancestors; level L holds the new octant
-	int lev = (63 - clz) / 3;
-	int index = 0;
-	count = 0;
-	if (lev > 0) {
-		const int parent = (lev >= 2) ? path[(lev - 2) * stride] : 0;
-		const int2 e = odc[parent + (int)((unsigned)location & 7u)];
-		index = e.x;
-		count = e.y;
-		path[(lev - 1) * stride] = index;
-	}
-	while (index >= 0) {
-		unsigned oct = 0;
-		oct ^= (cur.x > ax) ? 1u : 0u;
-		oct ^= (cur.y > ay) ? 2u : 0u;
-		oct ^= (cur.z > az) ? 4u : 0u;
-		location = (location << 3) | oct;
-		const int2 e = odc[index + (int)oct];
-		index = e.x;
-		count = e.y;
-		path[lev * stride] = index;   // level lev + 1
-		++lev;
-		const float hx = hw * hs.x, hy = hw * hs.y, hz = hw * hs.z;
-		ax += (oct & 1u) ? hx : -hx;
-		ay += (oct & 2u) ? hy : -hy;
-		az += (oct & 4u) ? hz : -hz;
-		hw *= 0.5f;
-	}
-	aw = 2.0f * hw;
-	return -index;
 }
 
 // Distance to the cell wall the ray leaves through (target -1/-2/-4 for the
@@ -736,39 +731,28 @@ __device__ __forceinline__ float wall_safety(const Geometry& g, F3 cur, float ax
 	return w - (1e-3f + 4e-6f * mag);
 }
 
-// The neighbour across wall `target` (-1/-2/-4): flip that axis' bit at the
-// deepest level where the move stays inside the parent; location 1 (or 0)
-// means the ray left the octree.
-__device__ __forceinline__ void cell_next(uint64_t& location, int target, F3 dir)
+// The cell across wall `target` (-1/-2/-4); 0 means the ray left the octree.
+__device__ __forceinline__ uint32_t cell_next(const Geometry& g, uint32_t cell, int target, F3 dir)
 {
-	const unsigned mask = (unsigned)(-target);
-	unsigned value;
-	if (mask == 1u) value = (dir.x >= 0.0f) ? 0u : 1u;
-	else if (mask == 2u) value = (dir.y >= 0.0f) ? 0u : 2u;
-	else value = (dir.z >= 0.0f) ? 0u : 4u;
-	while (location > 1) {
-		if ((location & (uint64_t)mask) == (uint64_t)value) {
-			location ^= (uint64_t)mask;
-			break;
-		}
-		location >>= 3;
-	}
+	const float d = target == -1 ? dir.x : target == -2 ? dir.y : dir.z;
+	const uint32_t axis = (uint32_t)(-target) >> 1;   // 0, 1, 2
+	return g.next[8 * (size_t)cell + 2u * axis + ((d >= 0.0f) ? 0u : 1u)];
 }
 
-// geometry/octree.inl:32-192: walk leaf cells by location code; returns the
+// geometry/octree.inl:32-192: walk from leaf to leaf; returns the
 // hit triangle (or -1) and the distance.  One lane, one ray.
 __device__ inline int propagate(const Geometry& g, F3 start, F3 dir, float distance,
-	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride)
+	int ignore_tri, int ignore_mat, float& out_dist)
 {
 	const int* __restrict__ od = g.od;
 	F3 cur = start;
 	float to_go = distance;
-	uint64_t location = 1;
+	uint32_t cell = cell_start(g, start);
 	uint32_t cells = 0;
 	do {
 		float ax, ay, az, aw;
 		int count;
-		int index = cell_find(g, cur, location, ax, ay, az, aw, path, stride, count);
+		int index = cell_find(g, cur, cell, ax, ay, az, aw, count);
 		++cells;
 		float isect;
 		int target;
@@ -794,8 +778,8 @@ __device__ inline int propagate(const Geometry& g, F3 start, F3 dir, float dista
 		}
 		to_go -= isect;
 		cur = v_add(cur, v_mul(dir, isect));
-		cell_next(location, target, dir);
-	} while (location > 1 && cells < MAX_CELLS);
+		cell = cell_next(g, cell, target, dir);
+	} while (cell != 0u && cells < MAX_CELLS);
 	out_dist = distance;
 	return -1;
 }
@@ -852,18 +836,19 @@ __device__ __forceinline__ int chunk_owner(int base, int excl, int n, int* owner
 }
 
 // A ray on its way through the octree: where it has got to, what is left of
-// its free path, its cell (location code) and the cells it has been in.
+// its free path, its cell (or an inner one that holds it) and the cells it
+// has been in.
 struct Walk {
 	F3 cur;
 	float to_go;
-	uint64_t location;
+	uint32_t cell;
 	uint32_t cells;
 };
-__device__ __forceinline__ void walk_start(Walk& w, F3 start, float distance)
+__device__ __forceinline__ void walk_start(const Geometry& g, Walk& w, F3 start, float distance)
 {
 	w.cur = start;
 	w.to_go = distance;
-	w.location = 1;
+	w.cell = cell_start(g, start);
 	w.cells = 0;
 }
 enum { WALK_ON = 0, WALK_END, WALK_HIT };
@@ -874,7 +859,7 @@ enum { WALK_ON = 0, WALK_END, WALK_HIT };
 // One lane walking its own cell's triangle list leaves most of the wave idle:
 // lists differ in length, and the wave runs as long as the longest.  Here
 // every walking lane enters its next cell and gets its list's length
-// (g.odc); the (ray, candidate) pairs of all lists are numbered by a prefix
+// (cell_find); the (ray, candidate) pairs of all lists are numbered by a prefix
 // sum over lanes and screened 64 at a time, one per lane, with the owning
 // ray's origin and direction fetched across lanes (cell_may_hit: material
 // test and a conservative plane test; about 2 % of the pairs pass on a
@@ -898,7 +883,7 @@ enum { WALK_ON = 0, WALK_END, WALK_HIT };
 // minimised per owner.
 template <bool SAF>
 __device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool first, Walk& w, F3 dir,
-	int ignore_tri, int ignore_mat, int* __restrict__ path, int stride, int* owner_at, float& isect, int& target)
+	int ignore_tri, int ignore_mat, int* owner_at, float& isect, int& target)
 {
 	const int lane = (int)__lane_id();
 	unsigned* s_saf = (unsigned*)owner_at + 192;
@@ -908,7 +893,7 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool f
 	isect = 0.0f;
 	if (active) {
 		float ax, ay, az, aw;
-		off = cell_find(g, w.cur, w.location, ax, ay, az, aw, path, stride, n);
+		off = cell_find(g, w.cur, w.cell, ax, ay, az, aw, n);
 		++w.cells;
 		cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
 		if (SAF && first)
@@ -988,35 +973,24 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool f
 		return WALK_HIT;
 	w.to_go -= isect;
 	w.cur = v_add(w.cur, v_mul(dir, isect));
-	cell_next(w.location, target, dir);
-	return (w.location > 1 && w.cells < MAX_CELLS) ? WALK_ON : WALK_END;
-}
-
-// The ancestors of a walk's cell into `path` (a walk taken up again).
-__device__ __forceinline__ void walk_path(const Geometry& g, const Walk& w, int* __restrict__ path, int stride)
-{
-	const int lev = (63 - __clzll((long long)w.location)) / 3;
-	int index = 0;
-	for (int l = 1; l < lev; ++l) {
-		index = g.odc[index + (int)((unsigned)(w.location >> (3 * (lev - l))) & 7u)].x;
-		path[(l - 1) * stride] = index;
-	}
+	w.cell = cell_next(g, w.cell, target, dir);
+	return (w.cell != 0u && w.cells < MAX_CELLS) ? WALK_ON : WALK_END;
 }
 
 // The whole walk for the rays of a wave (every lane calls; lanes with walk ==
 // false take part in the shared tests only).
 __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
-	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride, int* owner_at)
+	int ignore_tri, int ignore_mat, float& out_dist, int* owner_at)
 {
-	Walk w;
-	walk_start(w, start, distance);
+	Walk w = {};
+	if (walk)
+		walk_start(g, w, start, distance);
 	out_dist = distance;
 	int result = -1;
 	while (__ballot(walk) != 0ull) {
 		float isect;
 		int target;
-		const int r = walk_round<false>(g, walk, false, w, dir, ignore_tri, ignore_mat, path, stride, owner_at,
-			isect, target);
+		const int r = walk_round<false>(g, walk, false, w, dir, ignore_tri, ignore_mat, owner_at, isect, target);
 		if (walk && r != WALK_ON) {
 			walk = false;
 			if (r == WALK_HIT) {
@@ -1033,12 +1007,13 @@ __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 
 // tables, and every pair is tested in full; the screen's queue and second
 // load measured slower there.
 __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
-	int ignore_tri, int ignore_mat, float& out_dist, int* __restrict__ path, int stride, int* owner_at)
+	int ignore_tri, int ignore_mat, float& out_dist, int* owner_at)
 {
 	out_dist = distance;
 	const int lane = (int)__lane_id();
-	Walk w;
-	walk_start(w, start, distance);
+	Walk w = {};
+	if (walk)
+		walk_start(g, w, start, distance);
 	int result = -1;
 	bool active = walk;
 	while (__ballot(active) != 0ull) {
@@ -1046,7 +1021,7 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 		float isect = 0.0f;
 		if (active) {
 			float ax, ay, az, aw;
-			off = cell_find(g, w.cur, w.location, ax, ay, az, aw, path, stride, n);
+			off = cell_find(g, w.cur, w.cell, ax, ay, az, aw, n);
 			++w.cells;
 			cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
 		}
@@ -1104,8 +1079,8 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 			} else {
 				w.to_go -= isect;
 				w.cur = v_add(w.cur, v_mul(dir, isect));
-				cell_next(w.location, target, dir);
-				if (!(w.location > 1 && w.cells < MAX_CELLS))
+				w.cell = cell_next(g, w.cell, target, dir);
+				if (!(w.cell != 0u && w.cells < MAX_CELLS))
 					active = false;
 			}
 		}
@@ -1503,8 +1478,7 @@ __device__ __forceinline__ void step_move(State& s, F3 nd, float distance, int t
 // The whole init for one lane: domain and energy checks, path sampling,
 // propagate, move.  Returns ALIVE or TERMINATED and the event; `hit` is the
 // intersected triangle.
-__device__ inline int step_init(const World& W, State& s, Rng& rng, int& event, int& hit,
-	int* path, int stride, PathInfo& pinfo)
+__device__ inline int step_init(const World& W, State& s, Rng& rng, int& event, int& hit, PathInfo& pinfo)
 {
 	event = EV_NONE;
 	hit = -1;
@@ -1514,7 +1488,7 @@ __device__ inline int step_init(const World& W, State& s, Rng& rng, int& event, 
 	if (step_plan(W, s, rng, nd, distance, type, pinfo) != ALIVE)
 		return TERMINATED;
 	float hd;
-	hit = propagate(W.g, s.p.pos, nd, distance, s.last_tri, s.mat, hd, path, stride);
+	hit = propagate(W.g, s.p.pos, nd, distance, s.last_tri, s.mat, hd);
 	step_move(s, nd, distance, type, hit, hd, event, pinfo);
 	return ALIVE;
 }
