@@ -647,7 +647,7 @@ struct InFlight {
 	Walk w;
 	float distance, logE;       // free path, log of the energy
 	int type;                   // its mechanism
-	uint32_t b2, b3;            // the event's first two draws (in a material)
+	uint32_t b0, b1;            // the event's draws
 	float tau_el, tau_in;       // for the score
 	bool on;                    // walking
 	bool first;                 // in its start cell
@@ -706,8 +706,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 	to_inel = false;
 	bool ended = false, skip = false;
 	if (plan) {
-		Rng rng;
-		rng_start(rng, W.key0, W.key1, sid, step);
+		Draws rng = step_draws(W.key0, W.key1, sid, step);
 		F3 nd;
 		PathInfo pinfo;
 		oc = step_plan(W, s, rng, nd, f.distance, f.type, pinfo, f.planned);
@@ -716,8 +715,8 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 		if (oc == ALIVE) {
 			s.p.dir = nd;
 			f.logE = pinfo.logE;
-			f.b2 = rng.b2;
-			f.b3 = rng.b3;
+			f.b0 = rng.b0;
+			f.b1 = rng.b1;
 			if (SC) {
 				f.tau_el = pinfo.tau_el;
 				f.tau_in = pinfo.tau_in;
@@ -770,14 +769,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 		if (ev == EV_INELASTIC) {
 			to_inel = true;
 		} else {
-			Rng rng;
-			rng_start(rng, W.key0, W.key1, sid, step);
-			if (s.mat >= 0) {
-				// two draws were taken for the free paths
-				rng.b2 = f.b2;
-				rng.b3 = f.b3;
-				rng.idx = 2;
-			}
+			Draws rng = { f.b0, f.b1, 0u, 0u };
 			if (SC) {
 				float g = 0.0f;
 				int gmi = -1, gmo = -1;
@@ -988,13 +980,13 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 				break;
 			int oc = ALIVE;
 			bool walk = false;
-			Rng rng;
+			Draws rng = {};
 			int mat0 = s.mat, type = 0;
 			F3 nd = { 0.0f, 0.0f, 0.0f };
 			float distance = 0.0f;
 			PathInfo pinfo;
 			if (run) {
-				rng_start(rng, W.key0, W.key1, s.sid, s.step);
+				rng = step_draws(W.key0, W.key1, s.sid, s.step);
 				oc = step_plan(W, s, rng, nd, distance, type, pinfo, planned);
 				if (!planned)
 					++my_steps;
@@ -1373,12 +1365,12 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					bool walk = false;
 					const int mat0 = s.mat;
 					int type = 0;
-					Rng rng;
+					Draws rng = {};
 					F3 nd = { 0.0f, 0.0f, 0.0f };
 					float distance = 0.0f;
 					PathInfo pinfo;
 					if (run) {
-						rng_start(rng, W.key0, W.key1, s.sid, s.step);
+						rng = step_draws(W.key0, W.key1, s.sid, s.step);
 						oc = step_plan(W, s, rng, nd, distance, type, pinfo, f.planned);
 						if (!f.planned)
 							++my_steps;
@@ -1754,10 +1746,14 @@ int dev_alloc(T** p, size_t count)
 	return NBL_OK;
 }
 
-Table1 tab1(const nbl_table& t, const float* d) { return { d, t.dims[0], t.min[0], t.step[0] }; }
+Table1 tab1(const nbl_table& t, const float* d)
+{
+	return { d, t.dims[0], t.min[0], t.step[0], (float)(t.dims[0] - 2) };
+}
 Table2 tab2(const nbl_table& t, const float* d)
 {
-	return { d, t.dims[0], t.dims[1], t.min[0], t.step[0], t.min[1], t.step[1] };
+	return { d, t.dims[0], t.dims[1], t.min[0], t.step[0], t.min[1], t.step[1], (float)(t.dims[0] - 2),
+		(float)(t.dims[1] - 2) };
 }
 Table3 tab3(const nbl_table& t, const float* d)
 {
