@@ -297,6 +297,17 @@ int nbl_driver_counts(nbl_driver* d, uint32_t* running, uint32_t* detected, uint
  * copy out up to cap detected electrons and remove them from the device. */
 int nbl_driver_drain_detected(nbl_driver* d, nbl_detected* out, uint32_t cap, uint32_t* n);
 
+/* Counts of detected electrons instead of their records, kept on the device:
+ * electron i belongs to bin tag_bin[tag] (n_tags entries, copied by the call),
+ * column 0 below an energy of the caller's and 1 above.  nbl_driver_tally
+ * counts the records detected so far and removes them from the device, without
+ * waiting; nbl_driver_tally_read waits and copies out counts[2 * n_bins] and
+ * *bad: 0, or 1 if a tag was outside the table plus 2 if a bin was outside
+ * [0, n_bins) (such records are not counted). */
+int nbl_driver_tally_begin(nbl_driver* d, const int64_t* tag_bin, uint64_t n_tags, uint64_t n_bins);
+int nbl_driver_tally(nbl_driver* d, double se_cutoff);
+int nbl_driver_tally_read(nbl_driver* d, int64_t* counts, uint32_t* bad);
+
 /* Total particle-steps taken so far (init calls on active particles). */
 int nbl_driver_steps(nbl_driver* d, uint64_t* steps);
 

@@ -158,6 +158,9 @@ _SIGS = {
                                         C.c_int32, _p(C.c_uint32)]),
     "nbl_driver_counts": (C.c_int, [C.c_void_p, _p(C.c_uint32), _p(C.c_uint32), _p(C.c_uint64)]),
     "nbl_driver_drain_detected": (C.c_int, [C.c_void_p, C.c_void_p, C.c_uint32, _p(C.c_uint32)]),
+    "nbl_driver_tally_begin": (C.c_int, [C.c_void_p, C.c_void_p, C.c_uint64, C.c_uint64]),
+    "nbl_driver_tally": (C.c_int, [C.c_void_p, C.c_double]),
+    "nbl_driver_tally_read": (C.c_int, [C.c_void_p, C.c_void_p, _p(C.c_uint32)]),
     "nbl_driver_steps": (C.c_int, [C.c_void_p, _p(C.c_uint64)]),
     "nbl_driver_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_uint64, _p(C.c_uint64)]),
     "nbl_driver_stream": (C.c_void_p, [C.c_void_p]),

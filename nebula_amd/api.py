@@ -576,8 +576,10 @@ class Driver:
         """Track everything pushed to the end without keeping the records:
         counts[bin, 0] = detected electrons below `se_cutoff` eV (SE) and
         counts[bin, 1] = the others (BSE), binned by tag_bin[tag].  The
-        detected buffer is drained after every `frame` iterations (fewer
-        once few particles are left); with
+        detected buffer is tallied after every `frame` iterations (fewer
+        once few particles are left), on the GPU (k_tally) unless `tag_bin`
+        is no plain array of integers or far longer than what is to be
+        tracked: then the records are copied out and tallied here.  With
         progress_s > 0 a progress line goes to stderr that often.
 
         adapt_k: follow the best steps per launch as the run goes on.  The
@@ -591,7 +593,7 @@ class Driver:
         import time
         t_last = time.perf_counter()
         counts = np.zeros((n_bins, 2), np.int64)
-        buf = np.zeros(max(1, self.capacity), dtype=DET_DTYPE)
+        buf = None
         n = C.c_uint32()
         last_steps, stalled = -1, 0
         ks = tuple(k_choices)
@@ -612,12 +614,21 @@ class Driver:
             self.do_iteration(frame if left > FEW_PARTICLES else min(frame, 2))
             return time.perf_counter()
 
-        # Each frame's records are drained as soon as it ends and the next
-        # frame is enqueued before they are tallied, so the host's tally
-        # overlaps the GPU's next frame.
+        # Each frame's records are tallied on the GPU before the next frame;
+        # or they are drained as soon as it ends and the next frame is enqueued
+        # before they are tallied, so that the host's tally overlaps it.
         running, _, queued = self.counts()
         left = running + queued
         t0 = launch_frame()
+        on_gpu = (isinstance(tag_bin, np.ndarray) and tag_bin.ndim == 1 and tag_bin.dtype.kind in "iu"
+                  and tag_bin.dtype != np.uint64 and len(tag_bin) <= 4 * left + 65536)
+        if on_gpu:
+            # while the first frame runs
+            bins = np.ascontiguousarray(tag_bin, np.int64)
+            check(lib().nbl_driver_tally_begin(self._h, ptr(bins), len(bins), n_bins))
+            # a Python number is compared as float32, like the records' energies
+            cutoff = float(np.float32(se_cutoff)) if type(se_cutoff) in (int, float) else float(se_cutoff)
+            bad = C.c_uint32()
         while True:
             running, det, queued = self.counts()
             left = running + queued
@@ -644,7 +655,11 @@ class Driver:
                         probe = nxt
             steps_prev = st
             got = None
-            if det:
+            if det and on_gpu:
+                check(lib().nbl_driver_tally(self._h, cutoff))
+            elif det:
+                if buf is None:
+                    buf = np.zeros(max(1, self.capacity), dtype=DET_DTYPE)
                 check(lib().nbl_driver_drain_detected(self._h, ptr(buf), len(buf), C.byref(n)))
                 got = buf[: n.value]
             finished = running == 0 and queued == 0
@@ -659,6 +674,12 @@ class Driver:
                 se = got["E"] < se_cutoff
                 counts[:, 0] += np.bincount(b[se], minlength=n_bins)
                 counts[:, 1] += np.bincount(b[~se], minlength=n_bins)
+            if finished and on_gpu:
+                check(lib().nbl_driver_tally_read(self._h, ptr(counts), C.byref(bad)))
+                if bad.value & 1:
+                    raise IndexError(f"an electron's tag is outside tag_bin ({len(tag_bin)} entries)")
+                if bad.value:
+                    raise ValueError(f"an electron's bin is outside the {n_bins} of the tally")
             if finished:
                 return counts
             if progress_s > 0 and time.perf_counter() - t_last > progress_s:
