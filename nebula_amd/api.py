@@ -452,30 +452,48 @@ class Driver:
         self.deposits = bool(enable)
 
     def drain_deposits(self) -> np.ndarray:
+        n = self._deposits_waiting()
+        out = np.zeros(n, dtype=_lib.DEP_DTYPE)
+        if n:
+            self._drain_deposits_into(out)
+        return out
+
+    def _deposits_waiting(self) -> int:
         n = C.c_uint64()
         rc = lib().nbl_driver_drain_deposits(self._h, None, 0, C.byref(n))
-        if rc == _lib.NBL_OK:
-            return np.zeros(0, dtype=_lib.DEP_DTYPE)
-        if rc != _lib.NBL_ERR_CAPACITY or n.value == 0:
+        if rc != _lib.NBL_OK and (rc != _lib.NBL_ERR_CAPACITY or n.value == 0):
             check(rc)
-        out = np.zeros(n.value, dtype=_lib.DEP_DTYPE)
+        return 0 if rc == _lib.NBL_OK else n.value
+
+    def _drain_deposits_into(self, out: np.ndarray) -> None:
+        n = C.c_uint64()
         check(lib().nbl_driver_drain_deposits(self._h, ptr(out), len(out), C.byref(n)))
-        return out[: n.value]
+        assert n.value == len(out)
 
     def run_with_deposits(self, cap: int):
         """Track everything pushed to the end, one iteration at a time,
         draining deposits after each: (detected, deposits)."""
-        dets, deps = [], []
+        dets = []
+        # One array for all deposits, grown by doubling: room that is not used
+        # yet is not committed, and joining an array per iteration at the end
+        # took as long as the tracking and the drains together.
+        dep, n_dep = np.empty(0, _lib.DEP_DTYPE), 0
         while True:
             self.do_iteration(1)
-            deps.append(self.drain_deposits())
+            n = self._deposits_waiting()
+            if n_dep + n > len(dep):
+                bigger = np.empty(max(2 * len(dep), n_dep + 8 * n), _lib.DEP_DTYPE)
+                bigger[:n_dep] = dep[:n_dep]
+                dep = bigger
+            if n:
+                self._drain_deposits_into(dep[n_dep:n_dep + n])
+                n_dep += n
             running, det, queued = self.counts()
             if det:
                 dets.append(self.flush_detected())
             if running == 0 and queued == 0:
                 break
-        return (np.concatenate(dets) if dets else np.zeros(0, DET_DTYPE),
-                np.concatenate(deps) if deps else np.zeros(0, _lib.DEP_DTYPE))
+        return np.concatenate(dets) if dets else np.zeros(0, DET_DTYPE), dep[:n_dep]
 
     def set_launch(self, steps_per_launch: int, blocks_per_cu: int, target: int) -> None:
         check(lib().nbl_driver_set_launch(self._h, steps_per_launch, blocks_per_cu, target))

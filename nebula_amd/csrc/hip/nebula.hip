@@ -594,16 +594,17 @@ __device__ __forceinline__ bool place_secondary(const StepArgs& a, Ctrl* C, cons
 // takes its particle's geometry and materials from the world table.
 // An energy-deposit record (energydeposit_cpu_driver.h:55-66): position
 // after the event, energy before, energy lost; slots by ballot + atomic.
-__device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, const State& s, float e0)
+__device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, const Particle& p, uint32_t tag,
+	uint64_t sid, float e0)
 {
 	const uint32_t slot = wave_alloc(&C->dep_ctr, rec);
 	if (rec && slot < a.dep_cap) {
 		nbl_deposit r;
-		r.pos[0] = s.p.pos.x; r.pos[1] = s.p.pos.y; r.pos[2] = s.p.pos.z;
+		r.pos[0] = p.pos.x; r.pos[1] = p.pos.y; r.pos[2] = p.pos.z;
 		r.energy = e0;
-		r.deposit = e0 - s.p.E;
-		r.tag = s.tag;
-		r.sid = s.sid;
+		r.deposit = e0 - p.E;
+		r.tag = tag;
+		r.sid = sid;
 		a.dep[slot] = r;
 	}
 }
@@ -698,9 +699,11 @@ __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint
 //
 // Returns true in lanes whose step has ended: `oc` ALIVE (with `to_inel`: an
 // inelastic event is to follow), DETECTED or TERMINATED.
-template <bool SC>
+//
+// DEP: energy-deposit records of the elastic events, under `tag`.
+template <bool SC, bool DEP>
 __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, bool plan, State& s, uint64_t sid,
-	uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* owner_at,
+	uint32_t tag, uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* owner_at,
 	int& oc, bool& to_inel)
 {
 	oc = ALIVE;
@@ -770,6 +773,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 		if (ev == EV_INELASTIC) {
 			to_inel = true;
 		} else {
+			const float e0 = s.p.E;
 			Draws rng = { f.b0, f.b1, 0u, 0u };
 			if (SC) {
 				float g = 0.0f;
@@ -780,6 +784,8 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 			} else {
 				oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, f.logE);
 			}
+			if (DEP)
+				deposit(a, a.ctrl, ev == EV_ELASTIC && s.p.E != e0, s.p, tag, sid, e0);
 		}
 	}
 	return ended;
@@ -828,7 +834,7 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 	}
 }
 
-template <bool SC, bool WUNI>
+template <bool SC, bool WUNI, bool DEP>
 __device__ __forceinline__ void step_body(const StepArgs& a)
 {
 	static_assert(!(WUNI && SC), "the world-per-wave variant is the plain one");
@@ -905,8 +911,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 				break;
 			int oc;
 			bool inel;
-			const bool ended = step_turn<SC>(a, W, run && !f.on && k < K, s, SID_LDS ? s_sid[threadIdx.x] : s.sid,
-				SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, owner_at, oc, inel);
+			const bool ended = step_turn<SC, DEP>(a, W, run && !f.on && k < K, s,
+				SID_LDS ? s_sid[threadIdx.x] : s.sid, SID_LDS ? aux[0] : s.tag, SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, owner_at, oc, inel);
 			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
@@ -938,8 +944,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 }
 
 // The general variant: lanes of different worlds (flags bits 16..31), each
-// with its particle's geometry and materials from the world table, and
-// energy deposits.  Its walk gives no safety (and clears a particle's).
+// with its particle's geometry and materials from the world table, with
+// scores or energy deposits.  Its walk gives no safety (and clears a particle's).
 template <bool SC>
 __device__ __forceinline__ void step_multi(const StepArgs& a)
 {
@@ -1016,7 +1022,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 						oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
 					}
 					if (a.dep)
-						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
+						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s.p, s.tag, s.sid, e0);
 				}
 			}
 			if (run) {
@@ -1047,25 +1053,25 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 #ifndef NBL_PLAIN_WAVES
 #define NBL_PLAIN_WAVES 5
 #endif
-template <bool SC, bool MULTI, bool WUNI = false>
+template <bool SC, bool MULTI, bool WUNI = false, bool DEP = false>
 __global__ __launch_bounds__(256) void k_step(StepArgs a)
 {
 	if constexpr (MULTI)
 		step_multi<SC>(a);
 	else
-		step_body<SC, WUNI>(a);
+		step_body<SC, WUNI, DEP>(a);
 }
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
-void k_step<false, false, false>(StepArgs a)
+void k_step<false, false, false, false>(StepArgs a)
 {
-	step_body<false, false>(a);
+	step_body<false, false, false>(a);
 }
 template <>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
-void k_step<false, false, true>(StepArgs a)
+void k_step<false, false, true, false>(StepArgs a)
 {
-	step_body<false, true>(a);
+	step_body<false, true, false>(a);
 }
 
 // The inelastic events queued by k_step (drivers/gpu/gpu_driver.inl:505-540):
@@ -1153,7 +1159,7 @@ __global__ __launch_bounds__(256) void k_inel(StepArgs a)
 				done = false;
 			}
 			if ((SC || MULTI) && a.dep)
-				deposit(a, C, done && s.p.E != pre.p.E, s, pre.p.E);
+				deposit(a, C, done && s.p.E != pre.p.E, s.p, s.tag, s.sid, pre.p.E);
 			store_state(out, surv0 + i, s);
 			if (SC) store_score(out, surv0 + i, np, sc);
 		}
@@ -1181,10 +1187,12 @@ __global__ __launch_bounds__(256) void k_inel(StepArgs a)
 // it takes over from k_step + k_inel: 100 primaries of 1 keV in a slab 5.6
 // -> 2.0 ms, 1003 of 10 keV 41 -> 9.0 ms, 4096 of 500 eV on a grating 8.2 ->
 // 2.8 ms, 96 903 of 500 eV 16.8 -> 13.0 ms.
-template <bool SC, bool MULTI, bool WUNI>
+// DEP: one world with deposit records (MULTI writes them if a.dep is given).
+template <bool SC, bool MULTI, bool WUNI, bool DEP>
 __device__ __forceinline__ void cascade_body(const StepArgs& a)
 {
 	static_assert(!(WUNI && (SC || MULTI)), "the world-per-wave variant is the plain one");
+	static_assert(!(DEP && (SC || MULTI || WUNI)), "deposits of one world: the plain variant");
 	Ctrl* C = a.ctrl;
 	if (!C->few || C->n_surv + C->n_se == 0u)
 		return;
@@ -1269,7 +1277,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				break;
 			// every wave writes at most 64 deposits a step: stop while all of
 			// them still have room in the first half of the buffer
-			if (MULTI && a.dep && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+			if (((MULTI && a.dep) || DEP) && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 					+ 64ull * waves > a.dep_cap / 2u)
 				break;
 			if (k < n_steps && pend_share * __popcll(__ballot(pend)) >= __popcll(live)) {
@@ -1344,8 +1352,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						occ = true;
 					}
 				}
-				if (MULTI && a.dep)
-					deposit(a, C, pend && done && s.p.E != pre.E, s, pre.E);
+				if ((MULTI && a.dep) || DEP)
+					deposit(a, C, pend && done && s.p.E != pre.E, s.p, s.tag, s.sid, pre.E);
 				if (pend) {
 					if (done) {
 						s.step++;
@@ -1400,12 +1408,12 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 								oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
 							}
 							if (a.dep)
-								deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s, e0);
+								deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s.p, s.tag, s.sid, e0);
 						}
 					}
 				} else {
 					bool inel;
-					ended = step_turn<SC>(a, W, run && !f.on && k < n_steps, s, s.sid, s.step, f, rem, sc, my_steps,
+					ended = step_turn<SC, DEP>(a, W, run && !f.on && k < n_steps, s, s.sid, s.tag, s.step, f, rem, sc, my_steps,
 						s_owner, oc, inel);
 					pend = pend || (ended && inel);
 				}
@@ -1458,10 +1466,10 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	count_steps(C, my_steps);
 }
 
-template <bool SC, bool MULTI, bool WUNI = false>
+template <bool SC, bool MULTI, bool WUNI = false, bool DEP = false>
 __global__ __launch_bounds__(64) void k_cascade(StepArgs a)
 {
-	cascade_body<SC, MULTI, WUNI>(a);
+	cascade_body<SC, MULTI, WUNI, DEP>(a);
 }
 
 // Queue entries of one push: tag (tag_base + i, unless given), stream id
@@ -2564,7 +2572,9 @@ namespace {
 // k_step + k_inel in the variant the driver needs (scores, several worlds).
 void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 {
-	const bool multi = d->h_worlds.size() > 1 || d->dep;
+	// the general variants: several worlds with deposits or scores, and both
+	// of these
+	const bool multi = d->h_worlds.size() > 1 || (d->dep && d->map.np);
 	const dim3 grid(g), block(256), cgrid(cascade_waves(d->dev)), cblock(64);
 	if (multi && !d->dep && !d->map.np) {
 		// several worlds, nothing but records: the launch's particles
@@ -2594,6 +2604,10 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 	} else if (multi) {
 		hipLaunchKernelGGL((k_cascade<false, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
+	} else if (d->dep) {
+		hipLaunchKernelGGL((k_cascade<false, false, false, true>), cgrid, cblock, 0, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, false, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else {
 		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, 0, d->stream, a);
