@@ -57,6 +57,13 @@ __device__ __forceinline__ uint32_t* fld_u(const Bufs& b, int f)
 constexpr int MAX_PARAMS = 8;
 constexpr int MAX_SCORED_MATERIALS = 16;
 struct Score { double v[MAX_PARAMS]; };
+// A lane's score in LDS, [parameter][lane]: the step kernels add to one or two
+// parameters a step, chosen by the particle's material, which in registers
+// takes a compare, two selects and an addition for each of the eight, and 16
+// of the registers that set their occupancy (k_step 132 -> 95 VGPRs, 3 -> 5
+// waves per SIMD; k_cascade 148 and scratch -> 118, 3 -> 4).  Yield and Jacobian
+// of 249 856 primaries of 300 eV 42.5 -> 38.7 ms.
+struct ScoreLds { double* at; int stride; };
 
 // Parameter index of (material, kind) or -1; kinds 0 elastic MFP scale,
 // 1 inelastic MFP scale, 2 barrier.
@@ -178,13 +185,21 @@ __device__ __forceinline__ void store_score(const Bufs& b, uint32_t i, int np, c
 			b.sc[(size_t)q * b.sc_stride + i] = sc.v[q];
 }
 
-// score[q] += inc for a runtime q, without indexing registers dynamically
-__device__ __forceinline__ void score_add(Score& sc, int q, float inc)
+__device__ __forceinline__ void load_score(const Bufs& b, uint32_t i, int np, ScoreLds& sc)
 {
-#pragma unroll
-	for (int j = 0; j < MAX_PARAMS; ++j)
-		if (j == q)
-			sc.v[j] += (double)inc;
+	for (int q = 0; q < np; ++q)
+		sc.at[q * sc.stride] = b.sc[(size_t)q * b.sc_stride + i];
+}
+
+__device__ __forceinline__ void store_score(const Bufs& b, uint32_t i, int np, const ScoreLds& sc)
+{
+	for (int q = 0; q < np; ++q)
+		b.sc[(size_t)q * b.sc_stride + i] = sc.at[q * sc.stride];
+}
+
+__device__ __forceinline__ void score_add(ScoreLds& sc, int q, float inc)
+{
+	sc.at[q * sc.stride] += (double)inc;
 }
 
 __device__ __forceinline__ int score_index(const ScoreMap& m, int mat, int kind)
@@ -194,7 +209,7 @@ __device__ __forceinline__ int score_index(const ScoreMap& m, int mat, int kind)
 
 // d log p / d theta of a step's free-path race in material `mat`: rates
 // 1/tau, travelled distance d, winner `event` (or a boundary first).
-__device__ __forceinline__ void score_free_path(Score& sc, const ScoreMap& map, const World& W,
+__device__ __forceinline__ void score_free_path(ScoreLds& sc, const ScoreMap& map, const World& W,
 	int mat, const PathInfo& pi, int event)
 {
 	if (pi.type == 0)
@@ -208,7 +223,7 @@ __device__ __forceinline__ void score_free_path(Score& sc, const ScoreMap& map, 
 }
 
 // d log p / d b for the barriers on either side of a boundary (dU = b_mo - b_mi)
-__device__ __forceinline__ void score_barrier(Score& sc, const ScoreMap& map, int mi, int mo, float g)
+__device__ __forceinline__ void score_barrier(ScoreLds& sc, const ScoreMap& map, int mi, int mo, float g)
 {
 	if (g == 0.0f)
 		return;
@@ -539,9 +554,9 @@ __device__ __forceinline__ void count_steps(Ctrl* C, uint32_t my_steps)
 // Place a new secondary: the output buffer's SE region, else the spill
 // stack; returns false when both are full.  With scores, the secondary
 // starts from its parent's score.
-template <bool SC>
+template <bool SC, class S>
 __device__ __forceinline__ bool place_secondary(const StepArgs& a, Ctrl* C, const Bufs& out,
-	uint32_t se_limit, bool made, uint32_t sslot, const Particle& se, const State& parent, const Score& psc)
+	uint32_t se_limit, bool made, uint32_t sslot, const Particle& se, const State& parent, const S& psc)
 {
 	bool ok = true;
 	if (made) {
@@ -703,7 +718,7 @@ __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint
 // DEP: energy-deposit records of the elastic events, under `tag`.
 template <bool SC, bool DEP>
 __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, bool plan, State& s, uint64_t sid,
-	uint32_t tag, uint32_t step, InFlight& f, float& rem, Score& sc, uint32_t& my_steps, int* owner_at,
+	uint32_t tag, uint32_t step, InFlight& f, float& rem, ScoreLds& sc, uint32_t& my_steps, int* owner_at,
 	int& oc, bool& to_inel)
 {
 	oc = ALIVE;
@@ -795,7 +810,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, boo
 // the survivors, with one ballot per kind and one atomic per wave for the
 // last two together.  `f`: walks that go on in the next launch, or null.
 template <bool SC>
-__device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const Score& sc,
+__device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
 	bool keep, bool det, bool to_inel, const InFlight* f)
 {
 	const Bufs out = out_buf ? a.buf[1] : a.buf[0];
@@ -805,10 +820,8 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 		if (dslot < a.det_cap) {
 			store_detected(a, dslot, s);
 			if (SC) {
-#pragma unroll
-				for (int q = 0; q < MAX_PARAMS; ++q)
-					if (q < np)
-						a.det_sc[(size_t)dslot * np + q] = sc.v[q];
+				for (int q = 0; q < np; ++q)
+					a.det_sc[(size_t)dslot * np + q] = sc.at[q * sc.stride];
 			}
 			keep = false;
 		} else {
@@ -850,13 +863,14 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	World Wl = a.W;
 	const World& W = WUNI ? Wl : a.W;
 	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
-	// In the plain variant a particle's stream id waits here during its steps
-	// (each step reads it once to start its Philox stream), and with it its
-	// tag, step and flags (the walk needs none of them).
-	constexpr bool SID_LDS = !SC;
-	__shared__ uint64_t s_sid[SID_LDS ? 256 : 1];
-	__shared__ uint32_t s_aux[SID_LDS ? 3 * 256 : 1];
-	uint32_t* const aux = s_aux + (SID_LDS ? threadIdx.x : 0u);
+	// A particle's stream id waits here during its steps (each reads it once
+	// to start its Philox stream), and with it its tag, step and flags (the
+	// walk needs none of them).
+	__shared__ uint64_t s_sid[256];
+	__shared__ uint32_t s_aux[3 * 256];
+	__shared__ double s_score[SC ? MAX_PARAMS * 256 : 1];
+	uint32_t* const aux = s_aux + threadIdx.x;
+	ScoreLds sc = { s_score + (SC ? threadIdx.x : 0u), 256 };
 
 	int* owner_at = s_owner + 4 * (threadIdx.x & ~63u);
 	uint32_t my_steps = 0;
@@ -874,7 +888,6 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		const uint32_t li = (WUNI && !ident) ? ((i < n_loop) ? a.perm[i] : ~0u) : i;
 		const bool valid = (WUNI && !ident) ? li != ~0u : i < n_in;
 		State s = {};
-		Score sc;
 		InFlight f = {};
 		if (valid) {
 			const uint32_t slot = in_slot(li, n_surv, a.slots);
@@ -896,14 +909,10 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		// an inelastic event that found no secondary slot earlier
 		bool to_inel = (s.flags & FL_PEND_INEL) != 0u;
 		bool run = valid && !det && !to_inel, dead = false;
-		if (SID_LDS) {
-			s_sid[threadIdx.x] = s.sid;
-			aux[0] = s.tag;
-			aux[256] = s.step;
-			aux[512] = s.flags & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
-		} else {
-			s.flags &= ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
-		}
+		s_sid[threadIdx.x] = s.sid;
+		aux[0] = s.tag;
+		aux[256] = s.step;
+		aux[512] = s.flags & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
 		float rem = s.safe;
 		// K turns, and if walks are not kept, the walks to their end
 		for (uint32_t k = 0; k < K || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
@@ -912,7 +921,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 			int oc;
 			bool inel;
 			const bool ended = step_turn<SC, DEP>(a, W, run && !f.on && k < K, s,
-				SID_LDS ? s_sid[threadIdx.x] : s.sid, SID_LDS ? aux[0] : s.tag, SID_LDS ? aux[256] : s.step, f, rem, sc, my_steps, owner_at, oc, inel);
+				s_sid[threadIdx.x], aux[0], aux[256], f, rem, sc, my_steps, owner_at, oc, inel);
 			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
@@ -923,19 +932,15 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 				} else if (inel) {
 					to_inel = true;
 					run = false;
-				} else if (SID_LDS) {
-					aux[256] += 1u;
 				} else {
-					s.step++;
+					aux[256] += 1u;
 				}
 			}
 		}
-		if (SID_LDS) {
-			s.sid = s_sid[threadIdx.x];
-			s.tag = aux[0];
-			s.step = aux[256];
-			s.flags = aux[512];
-		}
+		s.sid = s_sid[threadIdx.x];
+		s.tag = aux[0];
+		s.step = aux[256];
+		s.flags = aux[512];
 		// a walk that goes on keeps the safety of its start point
 		s.safe = f.on ? ((float*)owner_at)[192 + __lane_id()] : rem;
 		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, &f);
@@ -960,6 +965,8 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 	World W = a.W;
 	__shared__ int s_owner[4 * 64];   // per wave: owner table
 	int* owner_at = s_owner + (threadIdx.x & ~63u);
+	__shared__ double s_score[SC ? MAX_PARAMS * 256 : 1];
+	ScoreLds sc = { s_score + (SC ? threadIdx.x : 0u), 256 };
 	uint32_t my_steps = 0;
 	const uint32_t stride = gridDim.x * blockDim.x;
 	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
@@ -967,7 +974,6 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 		const uint32_t i = w0 + __lane_id();
 		const bool valid = i < n_in;
 		State s = {};
-		Score sc;
 		if (valid) {
 			const uint32_t slot = in_slot(i, n_surv, a.slots);
 			s = load_state(in, slot);
@@ -1205,6 +1211,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	const World& W = (MULTI || WUNI) ? Wl : a.W;
 	__shared__ int s_owner[4 * 64];   // owner table, pair queue, safeties
 	const uint32_t lane = threadIdx.x;
+	__shared__ double s_score[SC ? MAX_PARAMS * 64 : 1];
+	ScoreLds sc = { s_score + (SC ? lane : 0u), 64 };
 	const uint64_t below = (1ull << lane) - 1ull;
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
@@ -1246,7 +1254,6 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			continue;
 		const int hold = (int)min(64u, (uint32_t)__popcll(first) + extra);
 		State s = {};
-		Score sc;
 		InFlight f = {};
 		if (occ) {
 			const uint32_t slot = in_slot(li, n_surv, a.slots);
@@ -1325,12 +1332,11 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					const uint32_t clo = (uint32_t)__shfl((int)(uint32_t)csid, src);
 					const uint32_t chi = (uint32_t)__shfl((int)(uint32_t)(csid >> 32), src);
 					if (SC) {
-#pragma unroll
-						for (int q = 0; q < MAX_PARAMS; ++q)
-							if (q < np) {
-								const double v = __shfl(sc.v[q], src);
-								if (take) sc.v[q] = v;
-							}
+						// (a parent keeps its lane; the lanes filled were free)
+						if (take)
+							for (int q = 0; q < np; ++q)
+								sc.at[q * 64] = s_score[q * 64 + src];
+						__builtin_amdgcn_wave_barrier();
 					}
 					if (take) {
 						s.p.pos = cp;
@@ -1433,10 +1439,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					if (dslot < a.det_cap) {
 						store_detected(a, dslot, s);
 						if (SC) {
-#pragma unroll
-							for (int q = 0; q < MAX_PARAMS; ++q)
-								if (q < np)
-									a.det_sc[(size_t)dslot * np + q] = sc.v[q];
+							for (int q = 0; q < np; ++q)
+								a.det_sc[(size_t)dslot * np + q] = sc.at[q * sc.stride];
 						}
 						occ = false;
 						det = false;
