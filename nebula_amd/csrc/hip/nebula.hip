@@ -133,6 +133,7 @@ struct StepArgs {
 	// buf[1] (WALK_FIELDS words a slot, [field][slot]), or null: a launch
 	// then finishes its walks
 	uint32_t* walk[2];
+	uint32_t max_mats;      // most materials of a world
 };
 constexpr uint32_t WALK_FIELDS = 6;
 // Particles in flight from which a launch leaves walks unfinished: with so
@@ -209,12 +210,13 @@ __device__ __forceinline__ int score_index(const ScoreMap& m, int mat, int kind)
 
 // d log p / d theta of a step's free-path race in material `mat`: rates
 // 1/tau, travelled distance d, winner `event` (or a boundary first).
-__device__ __forceinline__ void score_free_path(ScoreLds& sc, const ScoreMap& map, const World& W,
+template <class M>
+__device__ __forceinline__ void score_free_path(ScoreLds& sc, const ScoreMap& map, const M* mats,
 	int mat, const PathInfo& pi, int event)
 {
 	if (pi.type == 0)
 		return;
-	const Material& m = W.mats[mat];
+	const M& m = mats[mat];
 	const int pe = score_index(map, mat, 0), pn = score_index(map, mat, 1);
 	if (pe >= 0)
 		score_add(sc, pe, (pi.dist / pi.tau_el - ((event == EV_ELASTIC) ? 1.0f : 0.0f)) / m.el_scale);
@@ -659,12 +661,11 @@ __device__ __forceinline__ void load_world(const StepArgs& a, uint32_t ww, World
 	W.nmats = wd.nmats;
 }
 
-// A lane's step while it lasts: planned, and perhaps on its walk.
+// A lane's step while it lasts: planned, and perhaps on its walk (the rest of
+// it is in WaveMem).
 struct InFlight {
-	Walk w;
-	float distance, logE;       // free path, log of the energy
-	int type;                   // its mechanism
-	uint32_t b0, b1;            // the event's draws
+	uint32_t cells;             // cells its walk has been in
+	int type;                   // the free path's mechanism
 	float tau_el, tau_in;       // for the score
 	bool on;                    // walking
 	bool first;                 // in its start cell
@@ -672,26 +673,51 @@ struct InFlight {
 	bool resume;                // and its walk goes on
 };
 
-__device__ __forceinline__ void load_walk(const StepArgs& a, uint32_t buf, uint32_t slot, Walk& w)
+// A particle between global memory and WaveMem.  Its tag and flags stay where
+// they were read from.
+__device__ __forceinline__ void put_state(WaveMem& m, uint32_t lane, const State& s)
+{
+	m.pos[lane] = { s.p.pos.x, s.p.pos.y, s.p.pos.z, s.p.E };
+	m.dir[lane] = { s.p.dir.x, s.p.dir.y, s.p.dir.z, __int_as_float(s.mat) };
+	m.last[lane].x = s.last_tri;
+	m.sid[lane] = s.sid;
+	m.step[lane] = s.step;
+}
+__device__ __forceinline__ void get_state(const WaveMem& m, uint32_t lane, State& s)
+{
+	const float4 p = m.pos[lane], d = m.dir[lane];
+	s.p.pos = xyz(p);
+	s.p.E = p.w;
+	s.p.dir = xyz(d);
+	s.mat = __float_as_int(d.w);
+	s.last_tri = m.last[lane].x;
+	s.sid = m.sid[lane];
+	s.step = m.step[lane];
+}
+
+__device__ __forceinline__ void load_walk(const StepArgs& a, uint32_t buf, uint32_t slot, WaveMem& m, uint32_t lane,
+	InFlight& f)
 {
 	const uint32_t* p = a.walk[buf];
 	const size_t n = a.slots;
-	w.cur = { __uint_as_float(p[slot]), __uint_as_float(p[n + slot]), __uint_as_float(p[2 * n + slot]) };
-	w.to_go = __uint_as_float(p[3 * n + slot]);
-	w.cell = p[4 * n + slot];
-	w.cells = p[5 * n + slot];
+	m.cur[lane] = { __uint_as_float(p[slot]), __uint_as_float(p[n + slot]), __uint_as_float(p[2 * n + slot]),
+		__uint_as_float(p[3 * n + slot]) };
+	m.cell[lane] = p[4 * n + slot];
+	f.cells = p[5 * n + slot];
 }
 
-__device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const Walk& w)
+__device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const WaveMem& m,
+	uint32_t lane, const InFlight& f)
 {
 	uint32_t* p = a.walk[buf];
 	const size_t n = a.slots;
-	p[slot] = __float_as_uint(w.cur.x);
-	p[n + slot] = __float_as_uint(w.cur.y);
-	p[2 * n + slot] = __float_as_uint(w.cur.z);
-	p[3 * n + slot] = __float_as_uint(w.to_go);
-	p[4 * n + slot] = w.cell;
-	p[5 * n + slot] = w.cells;
+	const float4 c = m.cur[lane];
+	p[slot] = __float_as_uint(c.x);
+	p[n + slot] = __float_as_uint(c.y);
+	p[2 * n + slot] = __float_as_uint(c.z);
+	p[3 * n + slot] = __float_as_uint(c.w);
+	p[4 * n + slot] = m.cell[lane];
+	p[5 * n + slot] = f.cells;
 }
 
 // One turn of a wave (every lane calls): lanes with `plan` set plan their
@@ -717,101 +743,117 @@ __device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint
 //
 // DEP: energy-deposit records of the elastic events, under `tag`.
 template <bool SC, bool DEP>
-__device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, bool plan, State& s, uint64_t sid,
-	uint32_t tag, uint32_t step, InFlight& f, float& rem, ScoreLds& sc, uint32_t& my_steps, int* owner_at,
-	int& oc, bool& to_inel)
+__device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, const StepMat* mats, bool plan,
+	WaveMem& m, uint32_t tag,
+	InFlight& f, float& rem, ScoreLds& sc, uint32_t& wave_steps, int& oc, bool& to_inel)
 {
+	const uint32_t lane = __lane_id();
 	oc = ALIVE;
 	to_inel = false;
 	bool ended = false, skip = false;
+	wave_steps += (uint32_t)__popcll(__ballot(plan && !f.planned));
 	if (plan) {
-		Draws rng = step_draws(W.key0, W.key1, sid, step);
+		State s;
+		const float4 p = m.pos[lane], d = m.dir[lane];
+		s.p.pos = xyz(p);
+		s.p.E = p.w;
+		s.p.dir = xyz(d);
+		s.mat = __float_as_int(d.w);
+		Draws rng = step_draws(W.key0, W.key1, m.sid[lane], m.step[lane]);
 		F3 nd;
 		PathInfo pinfo;
-		oc = step_plan(W, s, rng, nd, f.distance, f.type, pinfo, f.planned);
-		if (!f.planned)
-			++my_steps;
+		float distance;
+		oc = step_plan(W, mats, s, rng, nd, distance, f.type, pinfo, f.planned);
 		if (oc == ALIVE) {
-			s.p.dir = nd;
-			f.logE = pinfo.logE;
-			f.b0 = rng.b0;
-			f.b1 = rng.b1;
+			m.dir[lane] = { nd.x, nd.y, nd.z, d.w };
+			m.evt[lane] = { distance, pinfo.logE, __uint_as_float(rng.b0), __uint_as_float(rng.b1) };
 			if (SC) {
 				f.tau_el = pinfo.tau_el;
 				f.tau_in = pinfo.tau_in;
 			}
-			skip = !f.resume && f.distance <= rem;
+			skip = !f.resume && distance <= rem;
 			f.on = !skip;
 			f.first = !f.resume;
-			if (f.resume)
-				((float*)owner_at)[192 + __lane_id()] = rem;
-			else if (!skip)
-				walk_start(W.g, f.w, s.p.pos, f.distance);
+			if (f.on && f.first) {
+				m.cur[lane] = { p.x, p.y, p.z, distance };
+				m.cell[lane] = cell_start(W.g, s.p.pos);
+				f.cells = 0;
+			}
 		} else {
 			ended = true;
 		}
 		f.planned = f.resume = false;
 	}
+	lds_again();
 	int hit = -1;
 	float hd = 0.0f;
 	bool arrive = skip;
 	if (__ballot(f.on) != 0ull) {
-		float isect;
+		float isect, safety;
 		int target;
-		const int r = walk_round<true>(W.g, f.on, f.first, f.w, s.p.dir, s.last_tri, s.mat, owner_at,
-			isect, target);
+		const int r = walk_round<true>(W.g, f.on, m, f.cells, safety, isect, target);
+		// while a walk lasts, rem is the safety of its start point
+		if (f.on && f.first)
+			rem = safety;
 		f.first = false;
 		if (f.on && r != WALK_ON) {
 			f.on = false;
 			arrive = true;
 			if (r == WALK_HIT) {
 				hit = target;
-				hd = f.distance - f.w.to_go + isect;
-				rem = -1.0f;
-			} else {
-				rem = (((float*)owner_at)[192 + __lane_id()] - f.distance) - W.g.step_eps;
+				hd = m.evt[lane].x - m.cur[lane].w + isect;
 			}
 		}
 	}
-	if (skip)
-		rem = (rem - f.distance) - W.g.step_eps;
 	if (arrive) {
 		ended = true;
 		int ev;
+		State s;
+		const float4 p = m.pos[lane], d = m.dir[lane], e = m.evt[lane];
+		s.p.pos = xyz(p);
+		s.p.E = p.w;
+		s.p.dir = xyz(d);
+		s.mat = __float_as_int(d.w);
+		s.last_tri = m.last[lane].x;
+		rem = (hit >= 0) ? -1.0f : (rem - e.x) - W.g.step_eps;
 		PathInfo pinfo;
 		const int mat0 = s.mat;
 		pinfo.tau_el = f.tau_el;
 		pinfo.tau_in = f.tau_in;
-		step_move(s, s.p.dir, f.distance, f.type, hit, hd, ev, pinfo);
+		step_move(s, s.p.dir, e.x, f.type, hit, hd, ev, pinfo);
 		if (SC)
-			score_free_path(sc, a.map, W, mat0, pinfo, ev);
+			score_free_path(sc, a.map, mats, mat0, pinfo, ev);
 		if (ev == EV_INELASTIC) {
 			to_inel = true;
 		} else {
 			const float e0 = s.p.E;
-			Draws rng = { f.b0, f.b1, 0u, 0u };
+			Draws rng = { __float_as_uint(e.z), __float_as_uint(e.w), 0u, 0u };
 			if (SC) {
 				float g = 0.0f;
 				int gmi = -1, gmo = -1;
-				oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, f.logE, &g, &gmi, &gmo);
+				oc = step_event_elastic_or_boundary(W, mats, s, rng, ev, hit, e.y, &g, &gmi, &gmo);
 				if (ev == EV_INTERSECT)
 					score_barrier(sc, a.map, gmi, gmo, g);
 			} else {
-				oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, f.logE);
+				oc = step_event_elastic_or_boundary(W, mats, s, rng, ev, hit, e.y);
 			}
 			if (DEP)
-				deposit(a, a.ctrl, ev == EV_ELASTIC && s.p.E != e0, s.p, tag, sid, e0);
+				deposit(a, a.ctrl, ev == EV_ELASTIC && s.p.E != e0, s.p, tag, m.sid[lane], e0);
 		}
+		m.pos[lane] = { s.p.pos.x, s.p.pos.y, s.p.pos.z, s.p.E };
+		m.dir[lane] = { s.p.dir.x, s.p.dir.y, s.p.dir.z, __int_as_float(s.mat) };
+		m.last[lane].x = s.last_tri;
 	}
+	lds_again();
 	return ended;
 }
 
 // Write the wave's particles out: detected records, the inelastic queue and
 // the survivors, with one ballot per kind and one atomic per wave for the
-// last two together.  `f`: walks that go on in the next launch, or null.
+// last two together.  `m`: with walks that go on in the next launch, or null.
 template <bool SC>
 __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
-	bool keep, bool det, bool to_inel, const InFlight* f)
+	bool keep, bool det, bool to_inel, const WaveMem* m, const InFlight& f)
 {
 	const Bufs out = out_buf ? a.buf[1] : a.buf[0];
 	const int np = a.map.np;
@@ -838,9 +880,9 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 		if (SC) store_score(a.inel, qslot, np, sc);
 	}
 	if (survive) {
-		if (f && f->on) {
+		if (m && f.on) {
 			s.flags |= FL_PLANNED | FL_WALK;
-			store_walk(a, out_buf, oslot, f->w);
+			store_walk(a, out_buf, oslot, *m, __lane_id(), f);
 		}
 		store_state(out, oslot, s);
 		if (SC) store_score(out, oslot, np, sc);
@@ -862,18 +904,21 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	World Wl = a.W;
 	const World& W = WUNI ? Wl : a.W;
-	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
-	// A particle's stream id waits here during its steps (each reads it once
-	// to start its Philox stream), and with it its tag, step and flags (the
-	// walk needs none of them).
-	__shared__ uint64_t s_sid[256];
-	__shared__ uint32_t s_aux[3 * 256];
-	__shared__ double s_score[SC ? MAX_PARAMS * 256 : 1];
-	uint32_t* const aux = s_aux + threadIdx.x;
-	ScoreLds sc = { s_score + (SC ? threadIdx.x : 0u), 256 };
+	__shared__ WaveMem s_mem[4];
+	WaveMem& m = s_mem[threadIdx.x >> 6];
+	const uint32_t lane = __lane_id();
+	// scores, then the materials (the block's, or with several worlds each
+	// wave's); step_lds is their size
+	extern __shared__ double s_dyn[];
+	ScoreLds sc = { s_dyn + threadIdx.x, 256 };
+	StepMat* const mats = (StepMat*)(s_dyn + (SC ? np * 256 : 0)) + (WUNI ? (threadIdx.x >> 6) * a.max_mats : 0u);
+	if (!WUNI) {
+		if (threadIdx.x < (uint32_t)a.W.nmats)
+			load_step_mat(mats[threadIdx.x], a.W.mats[threadIdx.x]);
+		__syncthreads();
+	}
 
-	int* owner_at = s_owner + 4 * (threadIdx.x & ~63u);
-	uint32_t my_steps = 0;
+	uint32_t wave_steps = 0;
 	const uint32_t stride = gridDim.x * blockDim.x;
 	// Whole waves take consecutive particles and step in lockstep: the walk
 	// shares its triangle tests across the wave (walk_round), so every
@@ -884,44 +929,47 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
 	for (uint32_t w0 = wave0; w0 < n_loop; w0 += stride) {
-		const uint32_t i = w0 + __lane_id();
+		const uint32_t i = w0 + lane;
 		const uint32_t li = (WUNI && !ident) ? ((i < n_loop) ? a.perm[i] : ~0u) : i;
 		const bool valid = (WUNI && !ident) ? li != ~0u : i < n_in;
-		State s = {};
+		const uint32_t slot = valid ? in_slot(li, n_surv, a.slots) : 0u;
 		InFlight f = {};
+		float rem = -1.0f;
+		uint32_t flags = 0, tag = 0;
 		if (valid) {
-			const uint32_t slot = in_slot(li, n_surv, a.slots);
-			s = load_state(in, slot);
+			const State s = load_state(in, slot);
 			if (SC) load_score(in, slot, np, sc);
 			f.planned = (s.flags & FL_PLANNED) != 0u;
 			f.resume = (s.flags & FL_WALK) != 0u;
 			if (f.resume)
-				load_walk(a, bi, slot, f.w);
+				load_walk(a, bi, slot, m, lane, f);
+			put_state(m, lane, s);
+			rem = s.safe;
+			flags = s.flags;
+			tag = s.tag;
 		}
 		if (WUNI) {
 			// lane 0 holds a particle (each world's range starts at a multiple
 			// of 64 and has no padding before its last particle; with one
 			// world, w0 < n_in): its world is the wave's, and no lane holds
 			// another world's particle
-			load_world(a, __builtin_amdgcn_readfirstlane(s.flags >> FL_WORLD_SHIFT), Wl);
+			load_world(a, __builtin_amdgcn_readfirstlane(flags >> FL_WORLD_SHIFT), Wl);
+			if (lane < (uint32_t)Wl.nmats)
+				load_step_mat(mats[lane], Wl.mats[lane]);
+			lds_again();
 		}
-		bool det = (s.flags & FL_PEND_DET) != 0u;
+		bool det = (flags & FL_PEND_DET) != 0u;
 		// an inelastic event that found no secondary slot earlier
-		bool to_inel = (s.flags & FL_PEND_INEL) != 0u;
+		bool to_inel = (flags & FL_PEND_INEL) != 0u;
 		bool run = valid && !det && !to_inel, dead = false;
-		s_sid[threadIdx.x] = s.sid;
-		aux[0] = s.tag;
-		aux[256] = s.step;
-		aux[512] = s.flags & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
-		float rem = s.safe;
 		// K turns, and if walks are not kept, the walks to their end
 		for (uint32_t k = 0; k < K || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
 			if (__ballot(run) == 0ull)
 				break;
 			int oc;
 			bool inel;
-			const bool ended = step_turn<SC, DEP>(a, W, run && !f.on && k < K, s,
-				s_sid[threadIdx.x], aux[0], aux[256], f, rem, sc, my_steps, owner_at, oc, inel);
+			const bool ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < K, m, DEP ? tag : 0u, f, rem, sc, wave_steps,
+				oc, inel);
 			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
@@ -933,19 +981,23 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 					to_inel = true;
 					run = false;
 				} else {
-					aux[256] += 1u;
+					m.step[lane] += 1u;
 				}
 			}
 		}
-		s.sid = s_sid[threadIdx.x];
-		s.tag = aux[0];
-		s.step = aux[256];
-		s.flags = aux[512];
-		// a walk that goes on keeps the safety of its start point
-		s.safe = f.on ? ((float*)owner_at)[192 + __lane_id()] : rem;
-		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, &f);
+		State s = {};
+		if (valid) {
+			get_state(m, lane, s);
+			// (read again rather than kept: two registers less in the loop)
+			s.tag = fld_u(in, F_TAG)[slot];
+			s.flags = fld_u(in, F_FLAGS)[slot] & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
+		}
+		// of a walk that goes on: the safety of its start point
+		s.safe = rem;
+		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, &m, f);
 	}
-	count_steps(C, my_steps);
+	if (lane == 0 && wave_steps)
+		atomicAdd((unsigned long long*)&C->steps, (unsigned long long)wave_steps);
 }
 
 // The general variant: lanes of different worlds (flags bits 16..31), each
@@ -1000,7 +1052,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 			PathInfo pinfo;
 			if (run) {
 				rng = step_draws(W.key0, W.key1, s.sid, s.step);
-				oc = step_plan(W, s, rng, nd, distance, type, pinfo, planned);
+				oc = step_plan(W, W.mats, s, rng, nd, distance, type, pinfo, planned);
 				if (!planned)
 					++my_steps;
 				planned = false;
@@ -1013,7 +1065,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 				int ev;
 				step_move(s, nd, distance, type, hit, hd, ev, pinfo);
 				if (SC)
-					score_free_path(sc, a.map, W, mat0, pinfo, ev);
+					score_free_path(sc, a.map, W.mats, mat0, pinfo, ev);
 				if (ev == EV_INELASTIC) {
 					to_inel = true;
 				} else {
@@ -1021,11 +1073,11 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 					if (SC) {
 						float g = 0.0f;
 						int gmi = -1, gmo = -1;
-						oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &g, &gmi, &gmo);
+						oc = step_event_elastic_or_boundary(W, W.mats, s, rng, ev, hit, pinfo.logE, &g, &gmi, &gmo);
 						if (ev == EV_INTERSECT)
 							score_barrier(sc, a.map, gmi, gmo, g);
 					} else {
-						oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+						oc = step_event_elastic_or_boundary(W, W.mats, s, rng, ev, hit, pinfo.logE);
 					}
 					if (a.dep)
 						deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s.p, s.tag, s.sid, e0);
@@ -1046,16 +1098,15 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 			}
 		}
 		s.safe = -1.0f;
-		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, nullptr);
+		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, nullptr, InFlight());
 	}
 	count_steps(C, my_steps);
 }
 
-// The plain variant runs at 5 waves per SIMD (96 VGPRs, 6 of them spilled,
-// 28 bytes of scratch per lane, hipcc -Rpass-analysis=kernel-resource-usage):
-// measured faster than 6 waves (80 VGPRs, 2 % slower with the tag, step and
-// flags in LDS, 11 % before) or 7.  The scored and multi-world variants
-// would spill, so they are left free.
+// The plain variant runs at 6 waves per SIMD: 74 VGPRs, and 25.9 KB of LDS a
+// block with the materials beside it (6 blocks of a compute unit's 160 KB).
+// With its state in registers (93 VGPRs, 5 waves) the full image took 254 ms,
+// 273 at 4 waves and 316 at 3.
 #ifndef NBL_PLAIN_WAVES
 #define NBL_PLAIN_WAVES 5
 #endif
@@ -1209,10 +1260,15 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	const int np = a.map.np;
 	World Wl = a.W;
 	const World& W = (MULTI || WUNI) ? Wl : a.W;
-	__shared__ int s_owner[4 * 64];   // owner table, pair queue, safeties
+	__shared__ WaveMem m;
+	int* const s_owner = m.owner;
 	const uint32_t lane = threadIdx.x;
 	__shared__ double s_score[SC ? MAX_PARAMS * 64 : 1];
 	ScoreLds sc = { s_score + (SC ? lane : 0u), 64 };
+	extern __shared__ double s_dyn[];
+	StepMat* const mats = (StepMat*)s_dyn;
+	if (!MULTI && !WUNI && lane < (uint32_t)W.nmats)
+		load_step_mat(mats[lane], W.mats[lane]);
 	const uint64_t below = (1ull << lane) - 1ull;
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
@@ -1243,7 +1299,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	const uint32_t se_limit = a.slots - n_in - groups * extra;
 	if (blockIdx.x == 0 && lane == 0)
 		C->se_limit = se_limit;
-	uint32_t my_steps = 0;
+	uint32_t my_steps = 0, wave_steps = 0;   // of this lane, of the wave
 	for (uint32_t w0 = blockIdx.x * g; w0 < n_loop; w0 += gridDim.x * g) {
 		const uint32_t i = w0 + lane;
 		const bool have = lane < g && i < n_loop;
@@ -1266,12 +1322,17 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				Wl.g = wd.g;
 				Wl.mats = wd.mats;
 				Wl.nmats = wd.nmats;
-			} else if (f.resume) {
-				load_walk(a, bi, slot, f.w);
+			} else {
+				if (f.resume)
+					load_walk(a, bi, slot, m, lane, f);
+				put_state(m, lane, s);
 			}
 		}
 		if (WUNI)   // one world a wave; its first particle names it
 			load_world(a, __builtin_amdgcn_readlane(s.flags >> FL_WORLD_SHIFT, __builtin_ctzll(first)), Wl);
+		if (WUNI && lane < (uint32_t)Wl.nmats)
+			load_step_mat(mats[lane], Wl.mats[lane]);
+		lds_again();
 		bool pend = (s.flags & FL_PEND_INEL) != 0u;   // an inelastic event to run
 		bool det = (s.flags & FL_PEND_DET) != 0u;     // to be recorded
 		bool park = false;                            // waits for the next launch
@@ -1291,6 +1352,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				Particle se = {};
 				Particle pre = {};
 				bool made = false;
+				if (!MULTI)
+					get_state(m, lane, s);
 				if (pend) {
 					pre = s.p;
 					Rng rng;
@@ -1371,6 +1434,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						park = true;
 					}
 				}
+				if (!MULTI)
+					put_state(m, lane, s);
 			}
 			const bool run = occ && !pend && !park && !det;
 			if (__ballot(run) != 0ull) {
@@ -1386,7 +1451,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					PathInfo pinfo;
 					if (run) {
 						rng = step_draws(W.key0, W.key1, s.sid, s.step);
-						oc = step_plan(W, s, rng, nd, distance, type, pinfo, f.planned);
+						oc = step_plan(W, W.mats, s, rng, nd, distance, type, pinfo, f.planned);
 						if (!f.planned)
 							++my_steps;
 						f.planned = false;
@@ -1399,7 +1464,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						int ev;
 						step_move(s, nd, distance, type, hit, hd, ev, pinfo);
 						if (SC)
-							score_free_path(sc, a.map, W, mat0, pinfo, ev);
+							score_free_path(sc, a.map, W.mats, mat0, pinfo, ev);
 						if (ev == EV_INELASTIC) {
 							pend = true;
 						} else {
@@ -1407,11 +1472,11 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 							if (SC) {
 								float gr = 0.0f;
 								int gmi = -1, gmo = -1;
-								oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE, &gr, &gmi, &gmo);
+								oc = step_event_elastic_or_boundary(W, W.mats, s, rng, ev, hit, pinfo.logE, &gr, &gmi, &gmo);
 								if (ev == EV_INTERSECT)
 									score_barrier(sc, a.map, gmi, gmo, gr);
 							} else {
-								oc = step_event_elastic_or_boundary(W, s, rng, ev, hit, pinfo.logE);
+								oc = step_event_elastic_or_boundary(W, W.mats, s, rng, ev, hit, pinfo.logE);
 							}
 							if (a.dep)
 								deposit(a, C, ev == EV_ELASTIC && s.p.E != e0, s.p, s.tag, s.sid, e0);
@@ -1419,8 +1484,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					}
 				} else {
 					bool inel;
-					ended = step_turn<SC, DEP>(a, W, run && !f.on && k < n_steps, s, s.sid, s.tag, s.step, f, rem, sc, my_steps,
-						s_owner, oc, inel);
+					ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < n_steps, m, s.tag, f, rem, sc, wave_steps, oc, inel);
 					pend = pend || (ended && inel);
 				}
 				if (ended) {
@@ -1428,14 +1492,18 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						det = true;
 					else if (oc == TERMINATED)
 						occ = false;
-					else if (!pend)
+					else if (!pend && MULTI)
 						s.step++;
+					else if (!pend)
+						m.step[lane] += 1u;
 				}
 			}
 			const bool rec = det && !park;
 			if (__ballot(rec)) {
 				const uint32_t dslot = wave_alloc(&C->det_ctr, rec);
 				if (rec) {
+					if (!MULTI)
+						get_state(m, lane, s);
 					if (dslot < a.det_cap) {
 						store_detected(a, dslot, s);
 						if (SC) {
@@ -1453,13 +1521,14 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		uint32_t oslot, qslot;
 		wave_alloc2(&C->step_out, occ, false, oslot, qslot);
 		if (occ) {
+			if (!MULTI)
+				get_state(m, lane, s);
 			s.flags |= (pend ? FL_PEND_INEL : 0u) | (det ? FL_PEND_DET : 0u);
 			s.safe = rem;
 			if (!MULTI && f.on) {
 				// the walk goes on in the next launch, with its start's safety
 				s.flags |= FL_PLANNED | FL_WALK;
-				s.safe = ((float*)s_owner)[192 + lane];
-				store_walk(a, bi ^ 1u, oslot, f.w);
+				store_walk(a, bi ^ 1u, oslot, m, lane, f);
 			} else if (MULTI && f.planned) {
 				s.flags |= FL_PLANNED;   // not taken up here
 			}
@@ -1467,7 +1536,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			if (SC) store_score(out, oslot, np, sc);
 		}
 	}
-	count_steps(C, my_steps);
+	count_steps(C, my_steps + ((lane == 0) ? wave_steps : 0u));
 }
 
 template <bool SC, bool MULTI, bool WUNI = false, bool DEP = false>
@@ -1566,7 +1635,7 @@ __global__ __launch_bounds__(256) void k_query(Geometry g, const float* pos, con
 	const float* dist, const int* ignore_tri, const int* ignore_mat, int* out_tri,
 	float* out_dist, uint32_t n)
 {
-	__shared__ int s_owner[4 * 256];   // per wave: owner table, pair queue, safeties
+	__shared__ WaveMem s_mem[4];
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	const bool valid = i < n;
 	F3 p = { 0.0f, 0.0f, 0.0f }, d = { 1.0f, 0.0f, 0.0f };
@@ -1581,8 +1650,7 @@ __global__ __launch_bounds__(256) void k_query(Geometry g, const float* pos, con
 	}
 	// the walk of the step kernel: whole waves, candidate tests shared
 	float od;
-	const int r = propagate_wave(g, valid, p, d, dd, it, im, od,
-		s_owner + 4 * (threadIdx.x & ~63u));
+	const int r = propagate_wave(g, valid, p, d, dd, it, im, od, s_mem[threadIdx.x >> 6]);
 	if (valid) {
 		out_tri[i] = r;
 		out_dist[i] = od;
@@ -1718,7 +1786,7 @@ struct nbl_geometry {
 
 struct nbl_material {
 	nbl_device* dev;
-	float* tables[7];
+	float* tables[9];   // the seven of the host's, and those of StepMat
 	Material m;
 };
 
@@ -1886,7 +1954,7 @@ struct Cells {
 	void root(const float center[3], const float halfsize[3])
 	{
 		std::memcpy(half, halfsize, sizeof(half));
-		rec = { make_float4(center[0], center[1], center[2], 1.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f) };
+		rec = { make_float4(center[0], center[1], center[2], 0.0f), make_float4(1.0f, 0.0f, 0.0f, 0.0f) };
 		next.assign(8, 0u);
 		inner = { 0u };
 		inner_depth = { 0 };
@@ -1901,16 +1969,16 @@ struct Cells {
 		// octree.inl: centre +- halfsize times the scale; the product with
 		// +-0.5 is exact, and scaling by a power of two commutes with rounding
 		// (halfsize >= 1 nm and scale >= 2^-21 stay far from underflow)
-		const float hw = 0.5f * c.w;
+		const float hw = 0.5f * rec[2 * (size_t)up + 1].x;
 		const float h[3] = { hw * half[0], hw * half[1], hw * half[2] };
-		rec[2 * (size_t)up + 1].x = bits((int32_t)first);
+		rec[2 * (size_t)up].w = bits((int32_t)first);
 		rec.resize(rec.size() + 16);
 		next.resize(next.size() + 64, 0u);
 		for (uint32_t o = 0; o < 8; ++o) {
 			const uint32_t i = first + o;
 			rec[2 * (size_t)i] = make_float4(c.x + ((o & 1u) ? h[0] : -h[0]), c.y + ((o & 2u) ? h[1] : -h[1]),
-				c.z + ((o & 4u) ? h[2] : -h[2]), hw);
-			rec[2 * (size_t)i + 1] = make_float4(bits(list[o]), bits(length[o]), 0.0f, 0.0f);
+				c.z + ((o & 4u) ? h[2] : -h[2]), 0.0f);
+			rec[2 * (size_t)i + 1] = make_float4(hw, bits(-list[o]), bits(length[o]), 0.0f);
 			// the deepest level at which the move stays inside the parent
 			for (uint32_t axis = 0; axis < 3; ++axis)
 				for (uint32_t low = 0; low < 2; ++low) {
@@ -1928,9 +1996,9 @@ struct Cells {
 	// Fill level `depth` of the start grid below cell i.
 	void fill(uint32_t i, uint32_t depth, uint32_t x, uint32_t y, uint32_t z)
 	{
-		const int32_t child = word(rec[2 * (size_t)i + 1].x);
+		const int32_t child = word(rec[2 * (size_t)i].w);
 		const uint32_t b = start_bits;
-		if (depth == b || child < 0) {
+		if (depth == b || child == 0) {
 			const uint32_t n = 1u << (b - depth);
 			for (uint32_t u = z * n; u < (z + 1) * n; ++u)
 				for (uint32_t v = y * n; v < (y + 1) * n; ++v)
@@ -2057,6 +2125,26 @@ int nbl_device_synchronize(nbl_device* d)
 	return NBL_OK;
 }
 
+// |e1|_1 |e2|_1 in the upper 16 bits of a float, rounded up, and the safety
+// bound's factor (pair_safety) in those of another, rounded down; 0, no
+// safety, where it is no ordinary number.
+static float screen_word(float ee, float nx, float ny, float nz)
+{
+	uint32_t e, r;
+	std::memcpy(&e, &ee, 4);
+	e = (ee == ee && e < 0x7f7f0000u) ? (e + 0xffffu) & 0xffff0000u : 0x7f800000u;
+	std::memcpy(&ee, &e, 4);
+	const double norm = std::sqrt((double)nx * nx + (double)ny * ny + (double)nz * nz);
+	const float rden = (float)(0.9998 / (norm * 1.0001 + 1e-5 * (double)ee));
+	std::memcpy(&r, &rden, 4);
+	if (!(rden > 1e-30f && rden < 1e30f))
+		r = 0;
+	const uint32_t w = e | (r >> 16);
+	float f;
+	std::memcpy(&f, &w, 4);
+	return f;
+}
+
 int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const nbl_triangle44* tris,
 	int64_t ntri, const float center[3], const float halfsize[3], nbl_geometry** out)
 {
@@ -2152,7 +2240,7 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 		const uint32_t mats = ((uint32_t)t.material_in & 0xffffu) | ((uint32_t)t.material_out << 16);
 		float mf;
 		std::memcpy(&mf, &mats, 4);
-		tscr[2 * i] = make_float4(t.r0[0], t.r0[1], t.r0[2], l1 * l2);
+		tscr[2 * i] = make_float4(t.r0[0], t.r0[1], t.r0[2], screen_word(l1 * l2, nx, ny, nz));
 		tscr[2 * i + 1] = make_float4(nx, ny, nz, mf);
 	}
 	// the screening records in table order: every entry that names a
@@ -2258,7 +2346,40 @@ int nbl_material_upload(nbl_device* dev, const nbl_material_host* m, nbl_materia
 		if (e != hipSuccess)
 			return release(fail(NBL_ERR_DEVICE, std::string("material table upload: ") + hipGetErrorString(e)));
 	}
+	mm->tables[7] = mm->tables[8] = nullptr;
+	std::vector<float> pairs;
+	auto upload_pairs = [&](int k) {
+		if ((rc = dev_alloc(&mm->tables[k], pairs.size())))
+			return false;
+		const hipError_t e = hipMemcpy(mm->tables[k], pairs.data(), sizeof(float) * pairs.size(), hipMemcpyHostToDevice);
+		if (e != hipSuccess)
+			rc = fail(NBL_ERR_DEVICE, std::string("material table upload: ") + hipGetErrorString(e));
+		return rc == NBL_OK;
+	};
+	{
+		const nbl_table& el = m->el_imfp;
+		const nbl_table& in = m->in_imfp;
+		if (el.dims[0] == in.dims[0] && el.min[0] == in.min[0] && el.step[0] == in.step[0]) {
+			for (int i = 0; i < el.dims[0]; ++i) {
+				pairs.push_back(el.data[i]);
+				pairs.push_back(in.data[i]);
+			}
+			if (!upload_pairs(7))
+				return release(rc);
+		}
+		const nbl_table& c = m->el_icdf;
+		const size_t row = (size_t)c.dims[1], cells = row * (size_t)(c.dims[0] - 1);
+		pairs.resize(2 * cells);
+		for (size_t i = 0; i < cells; ++i) {
+			pairs[2 * i] = c.data[i];
+			pairs[2 * i + 1] = c.data[i + row];
+		}
+		if (!upload_pairs(8))
+			return release(rc);
+	}
 	Material& d = mm->m;
+	d.imfp2 = (const float2*)mm->tables[7];
+	d.el_icdf2 = (const float2*)mm->tables[8];
 	d.barrier = m->barrier;
 	d.phonon_loss = m->phonon_loss;
 	d.recoil_const = m->recoil_const;
@@ -2576,11 +2697,12 @@ namespace {
 // k_step + k_inel in the variant the driver needs (scores, several worlds).
 void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 {
-	// the general variants: several worlds with deposits or scores, and both
-	// of these
-	const bool multi = d->h_worlds.size() > 1 || (d->dep && d->map.np);
+	// the general variants: several worlds with deposits or scores, both of
+	// these, and more materials than LDS is to hold
+	const bool multi = d->h_worlds.size() > 1 || (d->dep && d->map.np) || a.max_mats > STEP_MATS;
+	const size_t mats = sizeof(StepMat) * a.max_mats;
 	const dim3 grid(g), block(256), cgrid(cascade_waves(d->dev)), cblock(64);
-	if (multi && !d->dep && !d->map.np) {
+	if (multi && !d->dep && !d->map.np && a.max_mats <= STEP_MATS) {
 		// several worlds, nothing but records: the launch's particles
 		// grouped by world, one world per wave
 		const uint32_t nw = (uint32_t)d->h_worlds.size();
@@ -2594,28 +2716,28 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 		else
 			hipLaunchKernelGGL(k_world_place_wide, grid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1],
 				d->slots, nw, d->wgrp, d->perm);
-		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, 0, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 4 * mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else if (d->map.np && multi) {
 		hipLaunchKernelGGL((k_cascade<true, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<true, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<true, true>), grid, block, 0, d->stream, a);
 	} else if (d->map.np) {
-		hipLaunchKernelGGL((k_cascade<true, false>), cgrid, cblock, 0, d->stream, a);
-		hipLaunchKernelGGL((k_step<true, false>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_cascade<true, false>), cgrid, cblock, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<true, false>), grid, block, mats + 256 * sizeof(double) * d->map.np, d->stream, a);
 		hipLaunchKernelGGL((k_inel<true, false>), grid, block, 0, d->stream, a);
 	} else if (multi) {
 		hipLaunchKernelGGL((k_cascade<false, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, true>), grid, block, 0, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else if (d->dep) {
-		hipLaunchKernelGGL((k_cascade<false, false, false, true>), cgrid, cblock, 0, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_cascade<false, false, false, true>), cgrid, cblock, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, false, true>), grid, block, mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else {
-		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, 0, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false>), grid, block, mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, false>), grid, block, 0, d->stream, a);
 	}
 }
@@ -2645,6 +2767,9 @@ StepArgs step_args(const nbl_driver* d)
 	a.det_cap = d->det_cap;
 	a.slots = d->slots;
 	a.K = d->K;
+	a.max_mats = 0;
+	for (const WorldDesc& w : d->h_worlds)
+		a.max_mats = std::max<uint32_t>(a.max_mats, (uint32_t)w.nmats);
 	return a;
 }
 
@@ -3680,6 +3805,9 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 	a.det_cap = out_cap;
 	a.slots = slots;
 	a.K = steps_per_launch;
+	a.max_mats = (uint32_t)n_mats;
+	static_assert(NA_MAX_MATERIALS <= STEP_MATS, "materials in LDS");
+	const size_t lds_mats = sizeof(StepMat) * a.max_mats;
 	const uint32_t g_refill = blocks_for(capacity);
 	const uint32_t g_step = std::min<uint32_t>(blocks_for(capacity), 64u * (uint32_t)dev->n_cu);
 	(void)hipGetLastError();   // not this call's
@@ -3695,8 +3823,8 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 				~0u);
 			hipLaunchKernelGGL(k_refill, dim3(g_refill), dim3(256), 0, st, ctrl, a.buf[0], a.buf[1], a.spill,
 				primaries, tags, (const uint64_t*)nullptr, (const uint16_t*)nullptr, 0u, sid_base);
-			hipLaunchKernelGGL((k_cascade<false, false>), dim3(cascade_waves(dev)), dim3(64), 0, st, a);
-			hipLaunchKernelGGL((k_step<false, false>), dim3(g_step), dim3(256), 0, st, a);
+			hipLaunchKernelGGL((k_cascade<false, false>), dim3(cascade_waves(dev)), dim3(64), lds_mats, st, a);
+			hipLaunchKernelGGL((k_step<false, false>), dim3(g_step), dim3(256), lds_mats, st, a);
 			hipLaunchKernelGGL((k_inel<false, false>), dim3(g_step), dim3(256), 0, st, a);
 		}
 		HIP_OK(hipGetLastError());

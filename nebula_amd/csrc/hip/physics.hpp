@@ -497,6 +497,9 @@ __device__ __forceinline__ float t_index(float xi, float top)
 // otherwise be loaded from as a flat one).
 using GFloat = const __attribute__((address_space(1))) float;
 
+// a float4 at a multiple of 8 bytes
+typedef float float4a8 __attribute__((ext_vector_type(4), aligned(8)));
+
 // common/util/table_1D.inl:66-81
 __device__ __forceinline__ float t1_get(const Table1& t, float x)
 {
@@ -587,7 +590,91 @@ struct Material {
 	Table1 el_imfp, in_imfp;
 	Table2 el_icdf, in_icdf, ki_ion;
 	Table3 pn_q, pn_ion;
+	// For the step kernels (StepMat): (elastic, inelastic) of each entry of the
+	// two mean-free-path tables where they share their energies, or null; and
+	// rows lx and lx + 1 of el_icdf side by side.
+	const float2* imfp2;
+	const float2* el_icdf2;
 };
+
+// What a step other than an inelastic event needs of a material.  The step
+// kernels keep it in LDS: a step read some 17 of these constants from global
+// memory, and a load takes the texture unit as long when all lanes want one
+// word as when they want 64 (16 cycles and more; the units of the CUs were
+// busy 78 % of the step kernel's time).  At 104 bytes each, 64 of them take
+// 6.7 KB; drivers with more run the general variants, which read global memory.
+struct StepMat {
+	float barrier, phonon_loss, recoil_const, el_scale, in_scale;
+	struct { float xmin, xstep, topx; } el, in;
+	struct { float xmin, xstep, ymin, ystep, topx, topy; } cdf;
+	int ny;
+	const float2* imfp2;        // or null: the two tables below
+	const float2* icdf2;
+	const float* el_imfp;
+	const float* in_imfp;
+};
+constexpr int STEP_MATS = 64;   // materials a step kernel keeps in LDS
+__device__ __forceinline__ void load_step_mat(StepMat& d, const Material& m)
+{
+	d.barrier = m.barrier;
+	d.phonon_loss = m.phonon_loss;
+	d.recoil_const = m.recoil_const;
+	d.el_scale = m.el_scale;
+	d.in_scale = m.in_scale;
+	d.el = { m.el_imfp.xmin, m.el_imfp.xstep, m.el_imfp.topx };
+	d.in = { m.in_imfp.xmin, m.in_imfp.xstep, m.in_imfp.topx };
+	d.cdf = { m.el_icdf.xmin, m.el_icdf.xstep, m.el_icdf.ymin, m.el_icdf.ystep, m.el_icdf.topx, m.el_icdf.topy };
+	d.ny = m.el_icdf.ny;
+	d.imfp2 = m.imfp2;
+	d.icdf2 = m.el_icdf2;
+	d.el_imfp = m.el_imfp.d;
+	d.in_imfp = m.in_imfp.d;
+}
+using GFloat2 = const __attribute__((address_space(1))) float2;
+
+// Both logarithms of the inverse mean free paths at log energy x (t1_get)
+__device__ __forceinline__ void log_imfps(const Material& m, float x, float& el, float& in)
+{
+	el = t1_get(m.el_imfp, x);
+	in = t1_get(m.in_imfp, x);
+}
+__device__ __forceinline__ void log_imfps(const StepMat& m, float x, float& el, float& in)
+{
+	const float xe = (x - m.el.xmin) * m.el.xstep;
+	const float le = t_index(xe, m.el.topx), fe = xe - le;
+	float e0, e1, i0, i1, fi;
+	if (m.imfp2) {
+		const float4a8 v = *(const __attribute__((address_space(1))) float4a8*)((GFloat2*)m.imfp2 + (int)le);
+		e0 = v.x; i0 = v.y; e1 = v.z; i1 = v.w;
+		fi = fe;
+	} else {
+		const float xn = (x - m.in.xmin) * m.in.xstep;
+		const float ln = t_index(xn, m.in.topx);
+		GFloat* p = (GFloat*)m.el_imfp + (int)le;
+		GFloat* q = (GFloat*)m.in_imfp + (int)ln;
+		e0 = p[0]; e1 = p[1]; i0 = q[0]; i1 = q[1];
+		fi = xn - ln;
+	}
+	el = (1.0f - fe) * e0 + fe * e1;
+	in = (1.0f - fi) * i0 + fi * i1;
+}
+
+// The elastic event's cosine (t2_get)
+__device__ __forceinline__ float el_cosine(const Material& m, float x, float y) { return t2_get(m.el_icdf, x, y); }
+__device__ __forceinline__ float el_cosine(const StepMat& m, float x, float y)
+{
+	const float xi = (x - m.cdf.xmin) * m.cdf.xstep;
+	const float yi = (y - m.cdf.ymin) * m.cdf.ystep;
+	const float lx = t_index(xi, m.cdf.topx), ly = t_index(yi, m.cdf.topy);
+	// v00, v10, v01, v11
+	const float4a8 v = *(const __attribute__((address_space(1))) float4a8*)((GFloat2*)m.icdf2
+		+ ((size_t)(uint32_t)(int)lx * (uint32_t)m.ny + (uint32_t)(int)ly));
+	const float fx = xi - lx, fy = yi - ly;
+	return (1.0f - fx) * (1.0f - fy) * v.x
+		+ fx * (1.0f - fy) * v.y
+		+ (1.0f - fx) * fy * v.z
+		+ fx * fy * v.w;
+}
 
 // -------------------------------------------------------------- geometry --
 // Triangle as three float4: (r0.xyz, e1.x), (e1.yz, e2.xy), (e2.z, mat_in,
@@ -612,18 +699,19 @@ struct Geometry {
 	const int* od;
 	const float4* tris;
 	// Screening record per entry of the octree table, two float4, filled at
-	// every position that names a triangle: (r0, |e1|_1 |e2|_1) and (e1 x e2
-	// as the triangle test computes it, material_in | material_out as two
-	// int16 in the bits of w).  Stored in list order, so the screen reads
+	// every position that names a triangle: (r0, in 16 bits each |e1|_1 |e2|_1
+	// rounded up and the safety's 0.9999 / (1.0001 |n| + 1e-5 |e1|_1 |e2|_1)
+	// rounded down) and (n = e1 x e2 as the triangle test computes it,
+	// material_in | material_out as two int16 in the bits of w).  Stored in list order, so the screen reads
 	// neighbouring records for neighbouring pairs, without waiting for the
 	// triangle index.
 	const float4* scr;
 	// The octree's cells, inner ones and leaves, numbered from 1 with the
-	// eight children of a cell in a row (0: the root).  cells[2 i]: centre and
-	// scale (half extents over the root's) of cell i, with the roundings of
-	// the reference's descent; cells[2 i + 1] in integer bits: for an inner
-	// cell its first child, for a leaf the negative start of its list in `od`
-	// and the list's length.
+	// eight children of a cell in a row (0: the root).  cells[2 i]: centre of
+	// cell i, with the roundings of the reference's descent, and its first
+	// child in integer bits (0: a leaf); cells[2 i + 1], of a leaf: its scale
+	// (half extents over the root's) and in integer bits the start of its list
+	// in `od` and the list's length.
 	const float4* cells;
 	// next[8 i + 2 axis + (0 or 1)]: the cell that a ray leaving leaf i
 	// through its upper (0) or lower (1) wall of that axis enters, or an inner
@@ -716,13 +804,14 @@ __device__ __forceinline__ int cell_find(const Geometry& g, F3 cur, uint32_t& ce
 {
 	for (;;) {
 		const float4 a = g.cells[2 * (size_t)cell];
-		const int2 e = *(const int2*)(g.cells + 2 * (size_t)cell + 1);
-		if (e.x < 0) {
-			ax = a.x; ay = a.y; az = a.z; aw = a.w;
-			count = e.y;
-			return -e.x;
+		const uint32_t child = __float_as_uint(a.w);
+		if (child == 0u) {
+			const float4 e = g.cells[2 * (size_t)cell + 1];
+			ax = a.x; ay = a.y; az = a.z; aw = e.x;
+			count = __float_as_int(e.z);
+			return __float_as_int(e.y);
 		}
-		cell = (uint32_t)e.x + ((cur.x > a.x) ? 1u : 0u) + ((cur.y > a.y) ? 2u : 0u) + ((cur.z > a.z) ? 4u : 0u);
+		cell = child + ((cur.x > a.x) ? 1u : 0u) + ((cur.y > a.y) ? 2u : 0u) + ((cur.z > a.z) ? 4u : 0u);
 	}
 }
 
@@ -791,15 +880,17 @@ __device__ __forceinline__ float cell_candidate(const Geometry& g, int ti, F3 cu
 // Pairs that pass are tested in full (intersect_ray) in the second stage.
 __device__ __forceinline__ float dot_fma(F3 a, F3 b) { return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x)); }
 __device__ __forceinline__ float norm1(F3 a) { return fabsf(a.x) + fabsf(a.y) + fabsf(a.z); }
-// What both bounds need of a pair: e1 x e2, the materials, |e1|_1 |e2|_1,
-// |s|_1 and s . n.
-struct Screen { F3 nrm; uint32_t mats; float ee, slen, d0; };
+// What both bounds need of a pair: e1 x e2, the materials, |e1|_1 |e2|_1 and
+// the safety's factor, |s|_1 and s . n.
+struct Screen { F3 nrm; uint32_t mats; float ee, rden, slen, d0; };
 __device__ __forceinline__ Screen load_screen(const Geometry& g, uint32_t entry, F3 cur)
 {
 	const float4 a = g.scr[2 * (size_t)entry], b = g.scr[2 * (size_t)entry + 1];
 	const F3 nrm = { b.x, b.y, b.z };
 	const F3 sv = { cur.x - a.x, cur.y - a.y, cur.z - a.z };
-	return { nrm, __float_as_uint(b.w), a.w, norm1(sv), dot_fma(sv, nrm) };
+	const uint32_t w = __float_as_uint(a.w);
+	return { nrm, __float_as_uint(b.w), __uint_as_float(w & 0xffff0000u), __uint_as_float(w << 16), norm1(sv),
+		dot_fma(sv, nrm) };
 }
 __device__ __forceinline__ bool cell_may_hit(const Screen& s, F3 dir, int ignore_mat, float to_go)
 {
@@ -834,16 +925,14 @@ __device__ __forceinline__ bool cell_may_hit(const Screen& s, F3 dir, int ignore
 // r <= S).  A computed t >= d (= the remaining free path) is never taken as
 // a hit: the walk keeps the nearest t <= (cell exit + EPS) and reports a hit
 // only below the free path.  The bound below keeps a further 1e-4 relative
-// slack for its own rounding (reciprocal and square root within 1 ulp).
+// slack for its own rounding; its denominator is made at upload, rounded down.
 // Fused multiply-adds: their roundings are a part of those allowed for, here
 // and in cell_may_hit's plane test; the material test keeps dot()'s order.
 // Triangles skipped by the material or last-triangle tests count too: the
 // direction and the last triangle change between steps.
 __device__ __forceinline__ float pair_safety(const Screen& s)
 {
-	const float num = __builtin_fmaf(-2e-6f * s.slen, s.ee, fabsf(s.d0));
-	const float den = __builtin_fmaf(__builtin_amdgcn_sqrtf(dot_fma(s.nrm, s.nrm)), 1.0001f, 1e-5f * s.ee);
-	return num * __builtin_amdgcn_rcpf(den) * 0.9999f;
+	return __builtin_fmaf(-2e-6f * s.slen, s.ee, fabsf(s.d0)) * s.rden;
 }
 
 // Wall part: distance from `cur` to the walls of its leaf cell (centre
@@ -989,6 +1078,33 @@ __device__ __forceinline__ void walk_start(const Geometry& g, Walk& w, F3 start,
 }
 enum { WALK_ON = 0, WALK_END, WALK_HIT };
 
+// A wave's particles and walks, a lane each, in LDS: a walk's candidate tests
+// read other lanes' rays (three wide reads of LDS a pair, where fetching ten
+// values across lanes takes ten narrow ones), and what a phase of a step does
+// not need leaves its registers to the phase.
+//
+// This alone, with 6 waves per SIMD instead of 5 and 8 % fewer VALU
+// instructions, changed nothing (254 -> 257 ms for 6 553 600 primaries of
+// 300 eV): the step kernel then waited for its loads.  With the materials in
+// LDS as well (StepMat), 35 % fewer loads: 244.
+struct WaveMem {
+	float4 cur[64];       // walk: position, what is left of the free path
+	float4 dir[64];       // direction (normalised once the step is planned), material
+	float4 pos[64];       // position, energy
+	float4 evt[64];       // free path, log of the energy, the event's draws
+	int2 last[64];        // last triangle; walk: first entry of the list less the lane's first pair
+	uint64_t sid[64];
+	uint32_t step[64];
+	uint32_t cell[64];    // walk: its cell
+	int owner[64];        // owner table
+	int q_ti[64];         // queue of pairs: triangle, owner lane
+	unsigned saf[64];     // safeties
+	uint8_t q_own[64];
+};
+__device__ __forceinline__ F3 xyz(const float4& v) { return { v.x, v.y, v.z }; }
+// Reads of LDS are not carried over this point in registers.
+__device__ __forceinline__ void lds_again() { asm volatile("" ::: "memory"); }
+
 // One cell of the same walk for the rays of a whole wave, with the candidate
 // tests shared out over all 64 lanes.
 //
@@ -997,8 +1113,8 @@ enum { WALK_ON = 0, WALK_END, WALK_HIT };
 // every walking lane enters its next cell and gets its list's length
 // (cell_find); the (ray, candidate) pairs of all lists are numbered by a prefix
 // sum over lanes and screened 64 at a time, one per lane, with the owning
-// ray's origin and direction fetched across lanes (cell_may_hit: material
-// test and a conservative plane test; about 2 % of the pairs pass on a
+// ray's origin and direction read from LDS (cell_may_hit: material
+// test and a conservative plane test; about 9 % of the pairs pass on a
 // grating scan).  The pairs that pass are queued in LDS in pair order and
 // tested in full 64 at a time.  The results that can hit (t > 0) are then
 // taken in queue order, which is each owner's list order, and each owner
@@ -1007,57 +1123,50 @@ enum { WALK_ON = 0, WALK_END, WALK_HIT };
 // took about 20 % more of the step kernel.)
 //
 // Every lane of the wave must call it (lanes with active == false take part
-// in the shared tests only).  `owner_at` is 256 ints of LDS for this wave:
-// the owner table, the queue of pairs (triangle, owner lane) and safeties.
-// Returns WALK_HIT (triangle `target` at distance w.to_go - isect before the
+// in the shared tests only).  The rays are m.cur, m.dir, m.last and m.cell.
+// Returns WALK_HIT (triangle `target` at distance m.cur.w - isect before the
 // end of the free path), WALK_END (no hit) or WALK_ON (moved to the next
 // cell).
 //
-// SAF: lanes with `first` set are in their start cell and also leave the
-// safety of their start point in owner_at[192 + lane] (as float bits):
-// wall_safety of the cell, and pair_safety of every triangle listed there,
-// minimised per owner.
+// SAF: `safety` receives, from a walk's start cell, the safety of its start
+// point: wall_safety of the cell, and pair_safety of every triangle listed
+// there, minimised per owner (in other cells a value without meaning).
 template <bool SAF>
-__device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool first, Walk& w, F3 dir,
-	int ignore_tri, int ignore_mat, int* owner_at, float& isect, int& target)
+__device__ __forceinline__ int walk_round(const Geometry& g, bool active, WaveMem& m, uint32_t& cells,
+	float& safety, float& isect, int& target)
 {
 	const int lane = (int)__lane_id();
-	unsigned* s_saf = (unsigned*)owner_at + 192;
-	const uint64_t firsts = SAF ? __ballot(active && first) : 0ull;
 	int n = 0, off = 0;
 	target = 0;
 	isect = 0.0f;
 	if (active) {
 		float ax, ay, az, aw;
-		off = cell_find(g, w.cur, w.cell, ax, ay, az, aw, n);
-		++w.cells;
-		cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
-		if (SAF && first)
-			s_saf[lane] = __float_as_uint(fmaxf(wall_safety(g, w.cur, ax, ay, az, aw), 0.0f));
+		const F3 cur = xyz(m.cur[lane]), dir = xyz(m.dir[lane]);
+		uint32_t cell = m.cell[lane];
+		off = cell_find(g, cur, cell, ax, ay, az, aw, n);
+		m.cell[lane] = cell;
+		++cells;
+		cell_exit(g, cur, dir, ax, ay, az, aw, isect, target);
+		if (SAF)
+			m.saf[lane] = __float_as_uint(fmaxf(wall_safety(g, cur, ax, ay, az, aw), 0.0f));
 	}
 	const int incl = wave_incl_sum(n);
 	const int excl = incl - n;
-	off -= excl;  // pair p of this lane tests od[off + p]
+	m.last[lane].y = off - excl;  // pair p of this lane tests od[off - excl + p]
 	const int total = __builtin_amdgcn_readlane(incl, 63);
-	int* q_ti = owner_at + 64;
-	int* q_own = owner_at + 128;
 	int qn = 0;   // queued pairs (wave-uniform)
 	// Second stage: test the queued pairs in full and fold the results
 	// that can hit, in queue order, into their owners' running minimum.
 	auto flush = [&]() {
 		__builtin_amdgcn_wave_barrier();
 		int ti = -1, own = 0;
+		float t = -1.0f;
 		if (lane < qn) {
-			ti = q_ti[lane];
-			own = q_own[lane];
+			ti = m.q_ti[lane];
+			own = m.q_own[lane];
+			t = intersect_ray(load_tri(g.tris, ti), xyz(m.cur[own]), xyz(m.dir[own]));
 		}
 		__builtin_amdgcn_wave_barrier();
-		const int at = own << 2;
-		const F3 oc = { lane_float(at, w.cur.x), lane_float(at, w.cur.y), lane_float(at, w.cur.z) };
-		const F3 odir = { lane_float(at, dir.x), lane_float(at, dir.y), lane_float(at, dir.z) };
-		float t = -1.0f;
-		if (lane < qn)
-			t = intersect_ray(load_tri(g.tris, ti), oc, odir);
 		uint64_t hits = __ballot(t > 0.0f);
 		while (hits) {
 			const int src = (int)__builtin_ctzll(hits);
@@ -1071,24 +1180,18 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool f
 		}
 	};
 	for (int base = 0; base < total; base += 64) {
-		const int p = base + lane;
-		const int o = chunk_owner(base, excl, n, owner_at, lane);
-		const int at = o << 2;
-		const F3 oc = { lane_float(at, w.cur.x), lane_float(at, w.cur.y), lane_float(at, w.cur.z) };
-		const F3 odir = { lane_float(at, dir.x), lane_float(at, dir.y), lane_float(at, dir.z) };
-		const int oign_tri = lane_int(at, ignore_tri), oign_mat = lane_int(at, ignore_mat);
-		const float oto = lane_float(at, w.to_go);
-		const int ooff = lane_int(at, off);
-		bool pass = false;
-		int ti = -1;
-		if (p < total) {
-			const uint32_t entry = (uint32_t)(ooff + p);
-			ti = g.od[entry];
-			const Screen sc = load_screen(g, entry, oc);
-			pass = cell_may_hit(sc, odir, oign_mat, oto) && ti != oign_tri;
-			if (SAF && ((firsts >> o) & 1ull))
-				atomicMin(s_saf + o, __float_as_uint(fmaxf(pair_safety(sc), 0.0f)));
-		}
+		lds_again();
+		const int o = chunk_owner(base, excl, n, m.owner, lane);
+		// (the lanes behind the last pair repeat it)
+		const bool valid = base + lane < total;
+		const float4 oc = m.cur[o], od = m.dir[o];
+		const int2 ol = m.last[o];
+		const uint32_t entry = (uint32_t)(ol.y + min(base + lane, total - 1));
+		const int ti = g.od[entry];
+		const Screen sc = load_screen(g, entry, xyz(oc));
+		const bool pass = valid && ti != ol.x && cell_may_hit(sc, xyz(od), __float_as_int(od.w), oc.w);
+		if (SAF && valid)
+			atomicMin(&m.saf[o], __float_as_uint(fmaxf(pair_safety(sc), 0.0f)));
 		const uint64_t pm = __ballot(pass);
 		const int np = (int)__popcll(pm);
 		if (qn + np > 64) {
@@ -1097,44 +1200,54 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, bool f
 		}
 		if (pass) {
 			const int slot = qn + (int)__popcll(pm & ((1ull << lane) - 1ull));
-			q_ti[slot] = ti;
-			q_own[slot] = o;
+			m.q_ti[slot] = ti;
+			m.q_own[slot] = (uint8_t)o;
 		}
 		qn += np;
 	}
 	if (qn > 0)
 		flush();
+	lds_again();
+	if (SAF)
+		safety = __uint_as_float(m.saf[lane]);
 	if (!active)
 		return WALK_ON;
-	if (isect >= w.to_go)
+	const float4 c = m.cur[lane];
+	if (isect >= c.w)
 		return WALK_END;
 	if (target >= 0)
 		return WALK_HIT;
-	w.to_go -= isect;
-	w.cur = v_add(w.cur, v_mul(dir, isect));
-	w.cell = cell_next(g, w.cell, target, dir);
-	return (w.cell != 0u && w.cells < MAX_CELLS) ? WALK_ON : WALK_END;
+	const F3 dir = xyz(m.dir[lane]);
+	const F3 cur = v_add(xyz(c), v_mul(dir, isect));
+	m.cur[lane] = { cur.x, cur.y, cur.z, c.w - isect };
+	const uint32_t next = cell_next(g, m.cell[lane], target, dir);
+	m.cell[lane] = next;
+	return (next != 0u && cells < MAX_CELLS) ? WALK_ON : WALK_END;
 }
 
 // The whole walk for the rays of a wave (every lane calls; lanes with walk ==
 // false take part in the shared tests only).
 __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
-	int ignore_tri, int ignore_mat, float& out_dist, int* owner_at)
+	int ignore_tri, int ignore_mat, float& out_dist, WaveMem& m)
 {
-	Walk w = {};
+	const uint32_t lane = __lane_id();
+	uint32_t cells = 0;
+	m.cur[lane] = { start.x, start.y, start.z, distance };
+	m.dir[lane] = { dir.x, dir.y, dir.z, __int_as_float(ignore_mat) };
+	m.last[lane].x = ignore_tri;
 	if (walk)
-		walk_start(g, w, start, distance);
+		m.cell[lane] = cell_start(g, start);
 	out_dist = distance;
 	int result = -1;
 	while (__ballot(walk) != 0ull) {
-		float isect;
+		float isect, safety;
 		int target;
-		const int r = walk_round<false>(g, walk, false, w, dir, ignore_tri, ignore_mat, owner_at, isect, target);
+		const int r = walk_round<false>(g, walk, m, cells, safety, isect, target);
 		if (walk && r != WALK_ON) {
 			walk = false;
 			if (r == WALK_HIT) {
 				result = target;
-				out_dist = distance - w.to_go + isect;
+				out_dist = distance - m.cur[lane].w + isect;
 			}
 		}
 	}
@@ -1234,10 +1347,9 @@ struct Particle { F3 pos, dir; float E; };
 // path is multiplied by the mechanism's scale (exact when it is 1).  logE is
 // m_log(E), computed once per step for both mechanisms.
 template <class R>
-__device__ __forceinline__ float mech_sample_path(const Table1& t, float scale, float logE, R& rng,
-	float& tau)
+__device__ __forceinline__ float mech_sample_path(float log_imfp, float scale, R& rng, float& tau)
 {
-	const float imfp = m_exp(t1_get(t, logE));
+	const float imfp = m_exp(log_imfp);
 	tau = (is_mid(imfp) ? rcp_mid(imfp) : 1.0f / imfp) * scale;
 	return -tau * pf_log_normal(rng_unit(rng));
 }
@@ -1249,15 +1361,15 @@ __device__ __forceinline__ float mech_sample_path(const Table1& t, float scale, 
 struct PathInfo { float tau_el, tau_in, dist; int type; float logE; };
 
 // physics/kieft/elastic.h:67-115; logE = m_log(p.E)
-template <class R>
-__device__ __forceinline__ void elastic_execute(const Material& m, uint32_t fl, Particle& p, R& rng, float logE)
+template <class M, class R>
+__device__ __forceinline__ void elastic_execute(const M& m, uint32_t fl, Particle& p, R& rng, float logE)
 {
 	Particle tp = p;
 	float cos_theta, sin_theta;
 	{
 		const float x = logE;
 		const float y = rng_unit(rng);
-		cos_theta = clampr(t2_get(m.el_icdf, x, y), -1.0f, 1.0f);
+		cos_theta = clampr(el_cosine(m, x, y), -1.0f, 1.0f);
 		sin_theta = sqrt_mid(1.0f - cos_theta * cos_theta);   // 0 or at least 2^-24
 	}
 	tp.dir = normalised(tp.dir);
@@ -1466,8 +1578,8 @@ __device__ inline bool kieft_execute(const Material& m, uint32_t fl, Particle& p
 // With `g` given, it receives d log p / d dU of the random choices made
 // (transmission, reflection, absorption; 0 if none), and mi / mo the
 // materials with dU = b(mo) - b(mi).
-template <class R>
-__device__ __forceinline__ int boundary_execute(const Material* mats, uint32_t fl, const Tri& tri,
+template <class M, class R>
+__device__ __forceinline__ int boundary_execute(const M* mats, uint32_t fl, const Tri& tri,
 	Particle& p, int& mat, R& rng, float* g = nullptr, int* g_mi = nullptr, int* g_mo = nullptr)
 {
 	if (g) *g = 0.0f;
@@ -1568,8 +1680,8 @@ struct WorldDesc {
 // TERMINATED; for ALIVE, `distance` and `type` are the free path and its
 // mechanism (0 in vacuum), `nd` the normalised direction (the direction
 // itself when the step was `planned` before, FL_PLANNED).
-template <class R>
-__device__ __forceinline__ int step_plan(const World& W, const State& s, R& rng, F3& nd, float& distance,
+template <class M, class R>
+__device__ __forceinline__ int step_plan(const World& W, const M* mats, const State& s, R& rng, F3& nd, float& distance,
 	int& type, PathInfo& pinfo, bool planned = false)
 {
 	pinfo.type = 0;
@@ -1580,7 +1692,7 @@ __device__ __forceinline__ int step_plan(const World& W, const State& s, R& rng,
 	distance = W.g.max_extent;
 	float tau_el = 0.0f, tau_in = 0.0f;
 	if (s.mat >= 0) {
-		const Material& m = W.mats[s.mat];
+		const M& m = mats[s.mat];
 		if (s.p.E < m.barrier + W.threshold)
 			return TERMINATED;
 		// core/scatter_list.h:101-107 with the reverse visiting order of
@@ -1588,9 +1700,11 @@ __device__ __forceinline__ int step_plan(const World& W, const State& s, R& rng,
 		float dist = __builtin_inff();
 		const float logE = m_log(s.p.E);
 		pinfo.logE = logE;
-		const float pe = mech_sample_path(m.el_imfp, m.el_scale, logE, rng, tau_el);
+		float log_el, log_in;
+		log_imfps(m, logE, log_el, log_in);
+		const float pe = mech_sample_path(log_el, m.el_scale, rng, tau_el);
 		if (pe < dist) { type = 2; dist = pe; }
-		const float pi = mech_sample_path(m.in_imfp, m.in_scale, logE, rng, tau_in);
+		const float pi = mech_sample_path(log_in, m.in_scale, rng, tau_in);
 		if (pi < dist) { type = 1; dist = pi; }
 		distance = dist;
 	}
@@ -1628,7 +1742,7 @@ __device__ inline int step_init(const World& W, State& s, Rng& rng, int& event, 
 	F3 nd;
 	float distance;
 	int type;
-	if (step_plan(W, s, rng, nd, distance, type, pinfo) != ALIVE)
+	if (step_plan(W, W.mats, s, rng, nd, distance, type, pinfo) != ALIVE)
 		return TERMINATED;
 	float hd;
 	hit = propagate(W.g, s.p.pos, nd, distance, s.last_tri, s.mat, hd);
@@ -1665,17 +1779,17 @@ __device__ inline int step_event(const World& W, State& s, Rng& rng, int event, 
 // sends inelastic events to their own kernel, so its code holds neither the
 // inelastic models nor their register pressure.  logE is m_log(s.p.E)
 // from the step's path sampling.
-template <class R>
-__device__ __forceinline__ int step_event_elastic_or_boundary(const World& W, State& s, R& rng, int event,
+template <class M, class R>
+__device__ __forceinline__ int step_event_elastic_or_boundary(const World& W, const M* mats, State& s, R& rng, int event,
 	int hit, float logE, float* g = nullptr, int* g_mi = nullptr, int* g_mo = nullptr)
 {
 	if (event == EV_INTERSECT) {
 		const Tri tri = load_tri(W.g.tris, hit);
-		return boundary_execute(W.mats, W.flags, tri, s.p, s.mat, rng, g, g_mi, g_mo);
+		return boundary_execute(mats, W.flags, tri, s.p, s.mat, rng, g, g_mi, g_mo);
 	}
 	if (event == EV_ELASTIC) {
 		s.last_tri = -1;
-		elastic_execute(W.mats[s.mat], W.flags, s.p, rng, logE);
+		elastic_execute(mats[s.mat], W.flags, s.p, rng, logE);
 	}
 	return ALIVE;
 }
