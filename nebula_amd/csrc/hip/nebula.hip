@@ -1,8 +1,8 @@
 // HIP half of libnebula.so: device objects, the tracking kernels and the
 // device side of the C ABI (include/nebula.h).
 //
-// Particle buffer design.  Particles in flight live in two structure-of-arrays
-// buffers of `slots` entries used ping-pong.  In the buffer being read,
+// Particle buffer design.  Particles in flight live in two tiled buffers of
+// `slots` entries used ping-pong.  In the buffer being read,
 // survivors of the previous launch occupy [0, n_surv) and secondary electrons
 // [slots - n_se, slots).  A launch of k_step moves every particle through up
 // to K steps (init + event each), then appends it to the other buffer:
@@ -33,25 +33,26 @@ using namespace nbl::dev;
 	return fail(NBL_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(e_)); } while (0)
 
 // ------------------------------------------------------------- buffers --
-// One allocation per buffer of n entries: sid (8 bytes x n), then thirteen
-// 4-byte fields x n (px py pz dx dy dz E mat last_tri tag step flags safe).  A
-// buffer is one base pointer and its size, so a kernel holds four buffers
-// in a few scalar registers instead of 13 pointers each.
+// One allocation per buffer, in tiles of 64 entries and 4 KB: four groups of
+// 1 KB, 16 bytes an entry: position and energy; direction and material; last
+// triangle, tag, step, flags; stream id, safety, 4 bytes unused.  A wave's
+// particles are four wide loads or stores within a page or two.  (As an array
+// a field they were 15 narrow ones with an address each, each in a page of its
+// own: of the full image k_inel took 29.3 ms, now 27.8, k_step 205 and 203.)
 struct Bufs {
 	char* base;
 	double* sc;             // scores, [parameter][entry], or null
 	uint32_t sc_stride;     // entries of this buffer (n)
 };
-enum { F_PX, F_PY, F_PZ, F_DX, F_DY, F_DZ, F_E, F_MAT, F_LAST, F_TAG, F_STEP, F_FLAGS, F_SAFE, N_FIELDS };
-
-__device__ __forceinline__ float* fld_f(const Bufs& b, int f)
+constexpr size_t TILE_BYTES = 4096;
+constexpr size_t tile_bytes(size_t n) { return (n + 63) / 64 * TILE_BYTES; }
+__device__ __forceinline__ uint4* entry_at(const Bufs& b, uint32_t i)
 {
-	return (float*)(b.base + 8ull * b.sc_stride) + (size_t)f * b.sc_stride;
+	return (uint4*)(b.base + ((size_t)(i >> 6) * TILE_BYTES + ((i & 63u) << 4)));
 }
-__device__ __forceinline__ uint32_t* fld_u(const Bufs& b, int f)
-{
-	return (uint32_t*)(b.base + 8ull * b.sc_stride) + (size_t)f * b.sc_stride;
-}
+// Tag and flags of an entry
+__device__ __forceinline__ uint32_t& tag_at(const Bufs& b, uint32_t i) { return entry_at(b, i)[128].y; }
+__device__ __forceinline__ uint32_t& flags_at(const Bufs& b, uint32_t i) { return entry_at(b, i)[128].w; }
 
 // Likelihood-ratio scores carried by a particle (FP64 accumulation).
 constexpr int MAX_PARAMS = 8;
@@ -130,12 +131,12 @@ struct StepArgs {
 	const uint32_t* perm;
 	const uint32_t* perm_n;   // its padded length; perm_n[1]: one world, perm unused
 	// walks that a launch leaves unfinished, for the particles of buf[0] and
-	// buf[1] (WALK_FIELDS words a slot, [field][slot]), or null: a launch
-	// then finishes its walks
-	uint32_t* walk[2];
+	// buf[1] (tiles of 64 slots: position and what is left of the free path,
+	// then cell and cells been in), or null: a launch then finishes its walks
+	char* walk[2];
 	uint32_t max_mats;      // most materials of a world
 };
-constexpr uint32_t WALK_FIELDS = 6;
+constexpr size_t WALK_TILE = 64 * (16 + 8);
 // Particles in flight from which a launch leaves walks unfinished: with so
 // many some steps end in every launch, which the callers' checks for a run
 // that makes no progress count on.
@@ -143,32 +144,31 @@ constexpr uint32_t KEEP_WALKS_MIN = 65536;
 
 __device__ __forceinline__ State load_state(const Bufs& b, uint32_t i)
 {
+	const uint4* e = entry_at(b, i);
+	const uint4 p = e[0], d = e[64], m = e[128], x = e[192];
 	State s;
-	s.p.pos = { fld_f(b, F_PX)[i], fld_f(b, F_PY)[i], fld_f(b, F_PZ)[i] };
-	s.p.dir = { fld_f(b, F_DX)[i], fld_f(b, F_DY)[i], fld_f(b, F_DZ)[i] };
-	s.p.E = fld_f(b, F_E)[i];
-	s.mat = (int)fld_u(b, F_MAT)[i];
-	s.last_tri = (int)fld_u(b, F_LAST)[i];
-	s.tag = fld_u(b, F_TAG)[i];
-	s.step = fld_u(b, F_STEP)[i];
-	s.flags = fld_u(b, F_FLAGS)[i];
-	s.safe = fld_f(b, F_SAFE)[i];
-	s.sid = ((const uint64_t*)b.base)[i];
+	s.p.pos = { __uint_as_float(p.x), __uint_as_float(p.y), __uint_as_float(p.z) };
+	s.p.E = __uint_as_float(p.w);
+	s.p.dir = { __uint_as_float(d.x), __uint_as_float(d.y), __uint_as_float(d.z) };
+	s.mat = (int)d.w;
+	s.last_tri = (int)m.x;
+	s.tag = m.y;
+	s.step = m.z;
+	s.flags = m.w;
+	s.sid = ((uint64_t)x.y << 32) | x.x;
+	s.safe = __uint_as_float(x.z);
 	return s;
 }
 
 __device__ __forceinline__ void store_state(const Bufs& b, uint32_t i, const State& s)
 {
-	fld_f(b, F_PX)[i] = s.p.pos.x; fld_f(b, F_PY)[i] = s.p.pos.y; fld_f(b, F_PZ)[i] = s.p.pos.z;
-	fld_f(b, F_DX)[i] = s.p.dir.x; fld_f(b, F_DY)[i] = s.p.dir.y; fld_f(b, F_DZ)[i] = s.p.dir.z;
-	fld_f(b, F_E)[i] = s.p.E;
-	fld_u(b, F_MAT)[i] = (uint32_t)s.mat;
-	fld_u(b, F_LAST)[i] = (uint32_t)s.last_tri;
-	fld_u(b, F_TAG)[i] = s.tag;
-	fld_u(b, F_STEP)[i] = s.step;
-	fld_u(b, F_FLAGS)[i] = s.flags;
-	fld_f(b, F_SAFE)[i] = s.safe;
-	((uint64_t*)b.base)[i] = s.sid;
+	uint4* e = entry_at(b, i);
+	e[0] = make_uint4(__float_as_uint(s.p.pos.x), __float_as_uint(s.p.pos.y), __float_as_uint(s.p.pos.z),
+		__float_as_uint(s.p.E));
+	e[64] = make_uint4(__float_as_uint(s.p.dir.x), __float_as_uint(s.p.dir.y), __float_as_uint(s.p.dir.z),
+		(uint32_t)s.mat);
+	e[128] = make_uint4((uint32_t)s.last_tri, s.tag, s.step, s.flags);
+	e[192] = make_uint4((uint32_t)s.sid, (uint32_t)(s.sid >> 32), __float_as_uint(s.safe), 0u);
 }
 
 __device__ __forceinline__ void load_score(const Bufs& b, uint32_t i, int np, Score& sc)
@@ -422,7 +422,7 @@ __global__ __launch_bounds__(256) void k_world_group(const Ctrl* c, Bufs b0, Buf
 			const bool valid = i < hi;
 			uint32_t world = 0;
 			if (valid)
-				world = min(fld_u(b, F_FLAGS)[in_slot(i, n_surv, slots)] >> FL_WORLD_SHIFT, nw - 1u);
+				world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
 			uint64_t left = __ballot(valid);
 			while (left) {
 				const int first = __builtin_ctzll(left);
@@ -484,7 +484,7 @@ __global__ __launch_bounds__(256) void k_world_place_wide(const Ctrl* c, Bufs b0
 		const bool valid = i < n_in;
 		uint32_t world = 0;
 		if (valid)
-			world = min(fld_u(b, F_FLAGS)[in_slot(i, n_surv, slots)] >> FL_WORLD_SHIFT, nw - 1u);
+			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
 		uint64_t left = __ballot(valid);
 		while (left) {
 			const int first = __builtin_ctzll(left);
@@ -698,26 +698,25 @@ __device__ __forceinline__ void get_state(const WaveMem& m, uint32_t lane, State
 __device__ __forceinline__ void load_walk(const StepArgs& a, uint32_t buf, uint32_t slot, WaveMem& m, uint32_t lane,
 	InFlight& f)
 {
-	const uint32_t* p = a.walk[buf];
-	const size_t n = a.slots;
-	m.cur[lane] = { __uint_as_float(p[slot]), __uint_as_float(p[n + slot]), __uint_as_float(p[2 * n + slot]),
-		__uint_as_float(p[3 * n + slot]) };
-	m.cell[lane] = p[4 * n + slot];
-	f.cells = p[5 * n + slot];
+	const char* t = a.walk[buf] + (size_t)(slot >> 6) * WALK_TILE;
+	m.cur[lane] = ((const float4*)t)[slot & 63u];
+	const uint2 c = ((const uint2*)(t + 1024))[slot & 63u];
+	m.cell[lane] = c.x;
+	f.cells = c.y;
 }
 
-__device__ __forceinline__ void store_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const WaveMem& m,
+// Keep an unfinished walk; returns the particle's flags.  Where walks have no
+// room (a launch that stops early, its deposits' buffer half full) the step
+// stays planned and is walked again from its start.
+__device__ __forceinline__ uint32_t keep_walk(const StepArgs& a, uint32_t buf, uint32_t slot, const WaveMem& m,
 	uint32_t lane, const InFlight& f)
 {
-	uint32_t* p = a.walk[buf];
-	const size_t n = a.slots;
-	const float4 c = m.cur[lane];
-	p[slot] = __float_as_uint(c.x);
-	p[n + slot] = __float_as_uint(c.y);
-	p[2 * n + slot] = __float_as_uint(c.z);
-	p[3 * n + slot] = __float_as_uint(c.w);
-	p[4 * n + slot] = m.cell[lane];
-	p[5 * n + slot] = f.cells;
+	if (!a.walk[0])
+		return FL_PLANNED;
+	char* t = a.walk[buf] + (size_t)(slot >> 6) * WALK_TILE;
+	((float4*)t)[slot & 63u] = m.cur[lane];
+	((uint2*)(t + 1024))[slot & 63u] = make_uint2(m.cell[lane], f.cells);
+	return FL_PLANNED | FL_WALK;
 }
 
 // One turn of a wave (every lane calls): lanes with `plan` set plan their
@@ -880,10 +879,8 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 		if (SC) store_score(a.inel, qslot, np, sc);
 	}
 	if (survive) {
-		if (m && f.on) {
-			s.flags |= FL_PLANNED | FL_WALK;
-			store_walk(a, out_buf, oslot, *m, __lane_id(), f);
-		}
+		if (m && f.on)
+			s.flags |= keep_walk(a, out_buf, oslot, *m, __lane_id(), f);
 		store_state(out, oslot, s);
 		if (SC) store_score(out, oslot, np, sc);
 	}
@@ -989,8 +986,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		if (valid) {
 			get_state(m, lane, s);
 			// (read again rather than kept: two registers less in the loop)
-			s.tag = fld_u(in, F_TAG)[slot];
-			s.flags = fld_u(in, F_FLAGS)[slot] & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
+			s.tag = tag_at(in, slot);
+			s.flags = flags_at(in, slot) & ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
 		}
 		// of a walk that goes on: the safety of its start point
 		s.safe = rem;
@@ -1527,8 +1524,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			s.safe = rem;
 			if (!MULTI && f.on) {
 				// the walk goes on in the next launch, with its start's safety
-				s.flags |= FL_PLANNED | FL_WALK;
-				store_walk(a, bi ^ 1u, oslot, m, lane, f);
+				s.flags |= keep_walk(a, bi ^ 1u, oslot, m, lane, f);
 			} else if (MULTI && f.planned) {
 				s.flags |= FL_PLANNED;   // not taken up here
 			}
@@ -1563,7 +1559,7 @@ __global__ __launch_bounds__(256) void k_queue_ids(uint32_t* tag, uint64_t* sid,
 __global__ __launch_bounds__(256) void k_drop_walks(Bufs b)
 {
 	for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < b.sc_stride; i += gridDim.x * blockDim.x)
-		fld_u(b, F_FLAGS)[i] &= ~FL_WALK;
+		flags_at(b, i) &= ~FL_WALK;
 }
 
 __global__ void k_reset_det(Ctrl* c)
@@ -1741,7 +1737,7 @@ constexpr uint32_t NA_SLOTS = 2u * NA_MAX_CAPACITY;
 constexpr uint32_t NA_SPILL = 1u << 19;
 constexpr int NA_MAX_MATERIALS = 64;
 constexpr size_t na_round(size_t b) { return (b + 255) & ~(size_t)255; }
-constexpr size_t na_bufs_bytes(size_t n) { return na_round(n * (8 + 4 * N_FIELDS)); }
+constexpr size_t na_bufs_bytes(size_t n) { return na_round(tile_bytes(n)); }
 constexpr size_t NA_OFF_MATS = na_round(sizeof(Ctrl));
 constexpr size_t NA_OFF_BUF0 = NA_OFF_MATS + na_round(sizeof(Material) * NA_MAX_MATERIALS);
 constexpr size_t NA_OFF_BUF1 = NA_OFF_BUF0 + na_bufs_bytes(NA_SLOTS);
@@ -1803,7 +1799,7 @@ struct nbl_driver {
 	uint32_t spill_cap;
 	Bufs inel;
 	void* inel_mem;
-	uint32_t* walk[2];      // unfinished walks of the particles of buf[0] and buf[1], or null
+	char* walk[2];          // unfinished walks of the particles of buf[0] and buf[1], or null
 	Ctrl* ctrl;
 	Ctrl* h_ctrl;
 	nbl_detected* det;
@@ -1915,8 +1911,7 @@ uint32_t blocks_for(uint64_t n, uint32_t bs = 256)
 
 int alloc_bufs(Bufs& b, void*& mem, uint32_t slots)
 {
-	const size_t n = slots;
-	const size_t bytes = n * (8 + 4 * N_FIELDS) + 256;
+	const size_t bytes = tile_bytes(slots);
 	char* p = nullptr;
 	if (hipMalloc((void**)&p, bytes) != hipSuccess)
 		return fail(NBL_ERR_ALLOC, "hipMalloc of the particle buffers failed");
@@ -2496,11 +2491,12 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 	d->spill_cap = std::max<uint32_t>(1024u, std::min<uint64_t>(8ull * d->slots, 1ull << 28));
 	if ((rc = alloc_bufs(d->spill, d->spill_mem, d->spill_cap))) return cleanup(rc);
 	if ((rc = alloc_bufs(d->inel, d->inel_mem, d->slots))) return cleanup(rc);
-	// Unfinished walks, 24 bytes a slot and buffer.  Very large drivers (over
-	// 3.2 GB of them) go without: their launches finish every walk.
-	if (d->slots <= 1u << 26)
-		for (uint32_t*& w : d->walk)
-			if ((rc = dev_alloc(&w, (size_t)WALK_FIELDS * d->slots))) return cleanup(rc);
+	// Unfinished walks, 24 bytes a slot and buffer, where a launch may have
+	// enough particles to leave some.  Very large drivers (over 3.2 GB of them)
+	// go without: their launches finish every walk.
+	if (d->slots >= KEEP_WALKS_MIN && d->slots <= 1u << 26)
+		for (char*& w : d->walk)
+			if ((rc = dev_alloc(&w, WALK_TILE * ((d->slots + 63) / 64)))) return cleanup(rc);
 	if ((rc = dev_alloc(&d->ctrl, 1))) return cleanup(rc);
 	if (hipHostMalloc((void**)&d->h_ctrl, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess)
 		return cleanup(fail(NBL_ERR_ALLOC, "hipHostMalloc failed"));
@@ -3090,13 +3086,8 @@ int grow_spill(nbl_driver* d)
 		return rc;
 	}
 	const size_t on = d->spill_cap, nn = ncap, u = used;
-	char* ob = d->spill.base;
-	char* nbb = nb.base;
 	if (u) {
-		HIP_OK(hipMemcpyAsync(nbb, ob, 8 * u, hipMemcpyDeviceToDevice, d->stream));
-		for (int f = 0; f < N_FIELDS; ++f)
-			HIP_OK(hipMemcpyAsync(nbb + 8 * nn + 4 * f * nn, ob + 8 * on + 4 * f * on, 4 * u,
-				hipMemcpyDeviceToDevice, d->stream));
+		HIP_OK(hipMemcpyAsync(nb.base, d->spill.base, tile_bytes(u), hipMemcpyDeviceToDevice, d->stream));
 		for (int q = 0; q < d->map.np; ++q)
 			HIP_OK(hipMemcpyAsync(nsc + q * nn, d->spill.sc + q * on, 8 * u, hipMemcpyDeviceToDevice,
 				d->stream));
