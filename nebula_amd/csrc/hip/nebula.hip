@@ -127,7 +127,7 @@ struct StepArgs {
 	uint32_t spill_cap;
 	uint32_t K;
 	// world-per-wave variant: the coming launch's particles grouped by
-	// world (k_world_group); k_step's wave takes perm[i] for index i
+	// world (k_world_place); k_step's wave takes perm[i] for index i
 	const uint32_t* perm;
 	const uint32_t* perm_n;   // its padded length; perm_n[1]: one world, perm unused
 	// walks that a launch leaves unfinished, for the particles of buf[0] and
@@ -325,37 +325,133 @@ __device__ __forceinline__ uint32_t in_slot(uint32_t i, uint32_t n_surv, uint32_
 }
 
 // Grouping by world for the world-per-wave step kernel, in three kernels:
-// k_world_group<false> counts the coming launch's particles per world;
-// k_world_scan turns the counts into the worlds' starts, each a multiple
-// of 64 so that every step wave holds one world, marks the padding after
-// each world's range empty (~0u) and clears the counters;
-// k_world_group<true> writes each index into its world's range, a wave's
-// lanes of one world together, so that the step kernel's waves read runs
-// of neighbouring slots.  wg holds counts [0, nw), starts [nw, 2 nw), fill
-// levels [2 nw, 3 nw), the padded length of the index array at 3 nw, and
-// at 3 nw + 1 a flag set when at most one world has particles: the
-// launch's indices are then grouped as they stand, the placing pass
-// returns at once and the step kernel reads index i as itself.
-// Exclusive prefix of the counts into the starts (each padded to a
-// multiple of 64, the padding marked ~0u), the padded length at wg[3 nw],
-// the one-world flag at wg[3 nw + 1], counters and fill levels cleared for
-// the next launch.
-__device__ void world_scan(uint32_t nw, uint32_t* __restrict__ wg, uint32_t* __restrict__ perm)
+// k_world_count counts the coming launch's particles per world; k_world_scan
+// turns the counts into the worlds' starts, each a multiple of 64 so that
+// every step wave holds one world, and marks the padding after each world's
+// range empty (~0u); k_world_place writes each index into its world's range, a
+// wave's lanes of one world together, so that the step kernel's waves read
+// runs of neighbouring slots.  wg holds counts [0, nw), starts [nw, 2 nw), fill
+// levels [2 nw, 3 nw) (for more than NW_LDS worlds), the padded length of the
+// index array at 3 nw, and at 3 nw + 1 a flag set when at most one world has
+// particles: the launch's indices are then grouped as they stand, the placing
+// pass returns at once and the step kernel reads index i as itself.
+//
+// Each of WG_BLOCKS blocks takes a contiguous chunk of the indices (whole
+// waves), counts them per world in LDS (one LDS atomic per world present in a
+// wave) and leaves the counts in wb[world][block]; the scan turns them into
+// each block's place within its world's range, so the placing pass needs no
+// counting and no atomics in memory.  (With counters in memory, 1024 blocks'
+// atomics on the few of the worlds in flight serialised in L2: the three took
+// 86 us a launch for six scans of 294 720 primaries in all, now 17.)
+// Worlds beyond NW_LDS are counted and placed with one atomic per world
+// present in a wave instead.
+constexpr uint32_t NW_LDS = 1024, WG_BLOCKS = 256, WG_THREADS = 1024;
+__host__ __device__ inline uint32_t wb_offset(uint32_t nw) { return (3u * nw + 2u + 3u) & ~3u; }
+inline size_t wg_words(size_t nw) { return wb_offset((uint32_t)nw) + (nw <= NW_LDS ? (size_t)WG_BLOCKS * nw : 0); }
+
+// A block's chunk of n indices: whole waves
+__device__ __forceinline__ void wg_chunk(uint32_t n, uint32_t& lo, uint32_t& hi)
 {
-	__shared__ uint32_t s_v[256];
+	const uint32_t per = ((n + WG_BLOCKS - 1) / WG_BLOCKS + 63u) & ~63u;
+	lo = min(n, blockIdx.x * per);
+	hi = min(n, lo + per);
+}
+
+__global__ __launch_bounds__(WG_THREADS) void k_world_count(const Ctrl* c, Bufs b0, Bufs b1, uint32_t slots,
+	uint32_t nw, uint32_t* __restrict__ wg)
+{
+	__shared__ uint32_t s_h[NW_LDS];
+	const uint32_t n_surv = c->n_surv, n_in = n_surv + c->n_se;
+	const Bufs& b = c->buf_in ? b1 : b0;
+	const uint32_t lane = __lane_id();
+	uint32_t lo, hi;
+	wg_chunk(n_in, lo, hi);
+	for (uint32_t w = threadIdx.x; w < nw; w += WG_THREADS)
+		s_h[w] = 0;
+	__syncthreads();
+	for (uint32_t w0 = lo + (threadIdx.x & ~63u); w0 < hi; w0 += WG_THREADS) {
+		const uint32_t i = w0 + lane;
+		const bool valid = i < hi;
+		uint32_t world = 0;
+		if (valid)
+			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
+		uint64_t left = __ballot(valid);
+		while (left) {
+			const int first = __builtin_ctzll(left);
+			const uint32_t w = __builtin_amdgcn_readlane(world, first);
+			const uint64_t m = __ballot(valid && world == w);
+			left &= ~m;
+			if ((int)lane == first)
+				atomicAdd(&s_h[w], (uint32_t)__popcll(m));
+		}
+	}
+	__syncthreads();
+	uint32_t* const wb = wg + wb_offset(nw);
+	for (uint32_t w = threadIdx.x; w < nw; w += WG_THREADS)
+		wb[w * WG_BLOCKS + blockIdx.x] = s_h[w];
+}
+
+// The counting sweep for more than NW_LDS worlds
+__global__ __launch_bounds__(256) void k_world_count_wide(const Ctrl* c, Bufs b0, Bufs b1, uint32_t slots,
+	uint32_t nw, uint32_t* __restrict__ wg)
+{
+	const uint32_t n_surv = c->n_surv, n_in = n_surv + c->n_se;
+	const Bufs& b = c->buf_in ? b1 : b0;
+	const uint32_t lane = __lane_id();
+	for (uint32_t w0 = blockIdx.x * blockDim.x + (threadIdx.x & ~63u); w0 < n_in; w0 += gridDim.x * blockDim.x) {
+		const uint32_t i = w0 + lane;
+		const bool valid = i < n_in;
+		uint32_t world = 0;
+		if (valid)
+			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
+		uint64_t left = __ballot(valid);
+		while (left) {
+			const int first = __builtin_ctzll(left);
+			const uint32_t w = __builtin_amdgcn_readlane(world, first);
+			const uint64_t m = __ballot(valid && world == w);
+			left &= ~m;
+			if ((int)lane == first)
+				atomicAdd(&wg[w], (uint32_t)__popcll(m));
+		}
+	}
+}
+
+// One block (a separate launch: a count pass whose last block did this
+// needed a device-scope fence in every block, which on this multi-XCD GPU
+// writes back the L2, 67 us against 9 + 5): each world's counts of the blocks
+// into their exclusive prefix and its total, the totals into the starts (each
+// padded to a multiple of 64, the padding marked ~0u), the padded length, the
+// one-world flag, and the counters cleared for the next launch.
+__global__ __launch_bounds__(WG_THREADS) void k_world_scan(uint32_t nw, uint32_t* __restrict__ wg,
+	uint32_t* __restrict__ perm)
+{
+	__shared__ uint32_t s_v[WG_THREADS];
 	__shared__ uint32_t s_carry;
+	const uint32_t lane = __lane_id();
+	if (nw <= NW_LDS) {
+		static_assert(WG_BLOCKS == 4 * 64, "four blocks' counts a lane");
+		uint4* const wb = (uint4*)(wg + wb_offset(nw));
+		for (uint32_t w = threadIdx.x >> 6; w < nw; w += WG_THREADS / 64) {
+			const uint4 v = wb[w * 64 + lane];
+			const uint32_t sum = v.x + v.y + v.z + v.w;
+			const uint32_t incl = (uint32_t)wave_incl_sum((int)sum), at = incl - sum;
+			wb[w * 64 + lane] = make_uint4(at, at + v.x, at + v.x + v.y, at + v.x + v.y + v.z);
+			if (lane == 63u)
+				wg[w] = incl;
+		}
+	}
 	if (threadIdx.x == 0)
 		s_carry = 0;
 	__syncthreads();
 	uint32_t present = 0;   // worlds with particles
-	for (uint32_t base = 0; base < nw; base += blockDim.x) {
+	for (uint32_t base = 0; base < nw; base += WG_THREADS) {
 		const uint32_t i = base + threadIdx.x;
 		const uint32_t n = (i < nw) ? wg[i] : 0u;
 		const uint32_t v = (n + 63u) & ~63u;
 		present += (uint32_t)__syncthreads_count(n != 0u);
 		s_v[threadIdx.x] = v;
 		__syncthreads();
-		for (uint32_t o = 1; o < blockDim.x; o <<= 1) {
+		for (uint32_t o = 1; o < WG_THREADS && o < nw; o <<= 1) {
 			const uint32_t add = (threadIdx.x >= o) ? s_v[threadIdx.x - o] : 0u;
 			__syncthreads();
 			s_v[threadIdx.x] += add;
@@ -370,7 +466,7 @@ __device__ void world_scan(uint32_t nw, uint32_t* __restrict__ wg, uint32_t* __r
 				perm[start + k] = ~0u;
 		}
 		__syncthreads();
-		if (threadIdx.x == blockDim.x - 1)
+		if (threadIdx.x == min(WG_THREADS, nw - base) - 1u)
 			s_carry += s_v[threadIdx.x];
 		__syncthreads();
 	}
@@ -380,91 +476,41 @@ __device__ void world_scan(uint32_t nw, uint32_t* __restrict__ wg, uint32_t* __r
 	}
 }
 
-// Each block takes a contiguous chunk of the indices (whole waves) and
-// counts them per world in LDS first (one LDS atomic per world present in
-// a wave), so that the counters in memory see one atomic per world present
-// in a block: with one per wave, the waves' atomics on the few counters of
-// the worlds in flight serialised in L2 (165 us per pass on the 64-scan
-// batch).  PLACE: the block reserves its range of each world with those
-// atomics and a second sweep writes the indices from LDS offsets.  Worlds
-// beyond NW_LDS are counted with one atomic per wave instead.
-constexpr uint32_t NW_LDS = 1024;
-template <bool PLACE>
-__global__ __launch_bounds__(256) void k_world_group(const Ctrl* c, Bufs b0, Bufs b1, uint32_t slots,
-	uint32_t nw, uint32_t* __restrict__ wg, uint32_t* __restrict__ perm)
+__global__ __launch_bounds__(WG_THREADS) void k_world_place(const Ctrl* c, Bufs b0, Bufs b1, uint32_t slots,
+	uint32_t nw, const uint32_t* __restrict__ wg, uint32_t* __restrict__ perm)
 {
 	__shared__ uint32_t s_h[NW_LDS];
-	if (PLACE && wg[3 * nw + 1])
+	if (wg[3 * nw + 1])
 		return;   // one world: nothing to place
 	const uint32_t n_surv = c->n_surv, n_in = n_surv + c->n_se;
 	const Bufs& b = c->buf_in ? b1 : b0;
 	const uint32_t lane = __lane_id();
-	const bool lds = nw <= NW_LDS;
-	// this block's chunk: whole waves
-	const uint32_t per = ((n_in + gridDim.x - 1) / gridDim.x + 63u) & ~63u;
-	const uint32_t lo = blockIdx.x * per, hi = min(n_in, lo + per);
-	if (lds) {
-		for (uint32_t w = threadIdx.x; w < nw; w += blockDim.x)
-			s_h[w] = 0;
-		__syncthreads();
-	}
-	// sweep 0 counts; with PLACE, sweep 1 writes
-	for (int sweep = 0; sweep < (PLACE ? 2 : 1); ++sweep) {
-		if (sweep == 1) {
-			__syncthreads();
-			for (uint32_t w = threadIdx.x; w < nw; w += blockDim.x)
-				if (s_h[w])
-					s_h[w] = wg[nw + w] + atomicAdd(&wg[2 * nw + w], s_h[w]);
-			__syncthreads();
-		}
-		for (uint32_t w0 = lo + (threadIdx.x & ~63u); w0 < hi; w0 += blockDim.x) {
-			const uint32_t i = w0 + lane;
-			const bool valid = i < hi;
-			uint32_t world = 0;
-			if (valid)
-				world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
-			uint64_t left = __ballot(valid);
-			while (left) {
-				const int first = __builtin_ctzll(left);
-				const uint32_t w = __builtin_amdgcn_readlane(world, first);
-				const uint64_t m = __ballot(valid && world == w);
-				left &= ~m;
-				const uint32_t cnt = (uint32_t)__popcll(m);
-				if (sweep == 0) {
-					if ((int)lane == first) {
-						if (lds)
-							atomicAdd(&s_h[w], cnt);
-						else
-							atomicAdd(&wg[w], cnt);
-					}
-				} else {
-					uint32_t base = 0;
-					if ((int)lane == first)
-						base = atomicAdd(&s_h[w], cnt);
-					base = __builtin_amdgcn_readlane(base, first);
-					if ((m >> lane) & 1ull)
-						perm[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = i;
-				}
-			}
+	uint32_t lo, hi;
+	wg_chunk(n_in, lo, hi);
+	const uint32_t* const wb = wg + wb_offset(nw);
+	for (uint32_t w = threadIdx.x; w < nw; w += WG_THREADS)
+		s_h[w] = wg[nw + w] + wb[w * WG_BLOCKS + blockIdx.x];
+	__syncthreads();
+	for (uint32_t w0 = lo + (threadIdx.x & ~63u); w0 < hi; w0 += WG_THREADS) {
+		const uint32_t i = w0 + lane;
+		const bool valid = i < hi;
+		uint32_t world = 0;
+		if (valid)
+			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
+		uint64_t left = __ballot(valid);
+		while (left) {
+			const int first = __builtin_ctzll(left);
+			const uint32_t w = __builtin_amdgcn_readlane(world, first);
+			const uint64_t m = __ballot(valid && world == w);
+			left &= ~m;
+			uint32_t base = 0;
+			if ((int)lane == first)
+				base = atomicAdd(&s_h[w], (uint32_t)__popcll(m));
+			base = __builtin_amdgcn_readlane(base, first);
+			if ((m >> lane) & 1ull)
+				perm[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = i;
 		}
 	}
-	if (!PLACE) {
-		if (lds) {
-			__syncthreads();
-			for (uint32_t w = threadIdx.x; w < nw; w += blockDim.x)
-				if (s_h[w])
-					atomicAdd(&wg[w], s_h[w]);
-		}
-	}
-}
-
-// One block: the counts into starts (a separate launch: a count pass
-// whose last block did this needed a device-scope fence in every block,
-// which on this multi-XCD GPU writes back the L2, 67 us against 9 + 5).
-__global__ __launch_bounds__(256) void k_world_scan(uint32_t nw, uint32_t* __restrict__ wg,
-	uint32_t* __restrict__ perm)
-{
-	world_scan(nw, wg, perm);
 }
 
 // The placing sweep for more than NW_LDS worlds: one atomic per world
@@ -2595,9 +2641,9 @@ int nbl_driver_add_world(nbl_driver* d, const nbl_geometry* geom, const nbl_mate
 	// the world grouping's counters (cleared here, then by k_world_scan)
 	// and its index array
 	uint32_t* ng = nullptr;
-	if ((rc = dev_alloc(&ng, 3 * d->h_worlds.size() + 2)))
+	if ((rc = dev_alloc(&ng, wg_words(d->h_worlds.size()))))
 		return rc;
-	HIP_OK(hipMemset(ng, 0, sizeof(uint32_t) * (3 * d->h_worlds.size() + 2)));
+	HIP_OK(hipMemset(ng, 0, sizeof(uint32_t) * wg_words(d->h_worlds.size())));
 	hipFree(d->wgrp);
 	d->wgrp = ng;
 	// every world's range padded to a multiple of 64
@@ -2703,15 +2749,20 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 		// grouped by world, one world per wave
 		const uint32_t nw = (uint32_t)d->h_worlds.size();
 		const dim3 ggrid(std::min<uint32_t>(g, 4u * (uint32_t)d->dev->n_cu));
-		hipLaunchKernelGGL((k_world_group<false>), ggrid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1],
-			d->slots, nw, d->wgrp, d->perm);
-		hipLaunchKernelGGL(k_world_scan, dim3(1), dim3(256), 0, d->stream, nw, d->wgrp, d->perm);
-		if (nw <= NW_LDS)
-			hipLaunchKernelGGL((k_world_group<true>), ggrid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1],
-				d->slots, nw, d->wgrp, d->perm);
+		const bool wide = nw > NW_LDS;
+		if (wide)
+			hipLaunchKernelGGL(k_world_count_wide, ggrid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1], d->slots, nw,
+				d->wgrp);
 		else
+			hipLaunchKernelGGL(k_world_count, dim3(WG_BLOCKS), dim3(WG_THREADS), 0, d->stream, d->ctrl, d->buf[0],
+				d->buf[1], d->slots, nw, d->wgrp);
+		hipLaunchKernelGGL(k_world_scan, dim3(1), dim3(WG_THREADS), 0, d->stream, nw, d->wgrp, d->perm);
+		if (wide)
 			hipLaunchKernelGGL(k_world_place_wide, grid, block, 0, d->stream, d->ctrl, d->buf[0], d->buf[1],
 				d->slots, nw, d->wgrp, d->perm);
+		else
+			hipLaunchKernelGGL(k_world_place, dim3(WG_BLOCKS), dim3(WG_THREADS), 0, d->stream, d->ctrl, d->buf[0],
+				d->buf[1], d->slots, nw, d->wgrp, d->perm);
 		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, mats, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 4 * mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
