@@ -135,6 +135,7 @@ struct StepArgs {
 	// then cell and cells been in), or null: a launch then finishes its walks
 	char* walk[2];
 	uint32_t max_mats;      // most materials of a world
+	uint32_t same_grid;     // every material has its two mean free path tables as one (imfp2)
 };
 constexpr size_t WALK_TILE = 64 * (16 + 8);
 // Particles in flight from which a launch leaves walks unfinished: with so
@@ -808,7 +809,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 		F3 nd;
 		PathInfo pinfo;
 		float distance;
-		oc = step_plan(W, mats, s, rng, nd, distance, f.type, pinfo, f.planned);
+		oc = step_plan_short(W, mats, a.same_grid != 0u, s, rng, nd, distance, f.type, pinfo, f.planned);
 		if (oc == ALIVE) {
 			m.dir[lane] = { nd.x, nd.y, nd.z, d.w };
 			m.evt[lane] = { distance, pinfo.logE, __uint_as_float(rng.b0), __uint_as_float(rng.b1) };
@@ -1975,7 +1976,8 @@ struct Cells {
 	std::vector<uint32_t> next, start;
 	std::vector<uint32_t> inner;      // the inner cells, in the order they are split in
 	std::vector<uint8_t> inner_depth;
-	float half[3], lo[3], inv[3];
+	std::vector<float> scale;         // their half extents over the root's
+	float mid[3], half[3], lo[3], inv[3];
 	float start_eps = 0.0f;
 	uint32_t start_bits = 0;
 
@@ -1995,7 +1997,9 @@ struct Cells {
 	void root(const float center[3], const float halfsize[3])
 	{
 		std::memcpy(half, halfsize, sizeof(half));
-		rec = { make_float4(center[0], center[1], center[2], 0.0f), make_float4(1.0f, 0.0f, 0.0f, 0.0f) };
+		rec = { make_float4(center[0], center[1], center[2], 0.0f), make_float4(0.0f, 0.0f, 0.0f, 0.0f) };
+		std::memcpy(mid, center, sizeof(mid));
+		scale = { 1.0f };
 		next.assign(8, 0u);
 		inner = { 0u };
 		inner_depth = { 0 };
@@ -2010,16 +2014,23 @@ struct Cells {
 		// octree.inl: centre +- halfsize times the scale; the product with
 		// +-0.5 is exact, and scaling by a power of two commutes with rounding
 		// (halfsize >= 1 nm and scale >= 2^-21 stay far from underflow)
-		const float hw = 0.5f * rec[2 * (size_t)up + 1].x;
+		const float hw = 0.5f * scale[k];
 		const float h[3] = { hw * half[0], hw * half[1], hw * half[2] };
 		rec[2 * (size_t)up].w = bits((int32_t)first);
 		rec.resize(rec.size() + 16);
 		next.resize(next.size() + 64, 0u);
 		for (uint32_t o = 0; o < 8; ++o) {
 			const uint32_t i = first + o;
-			rec[2 * (size_t)i] = make_float4(c.x + ((o & 1u) ? h[0] : -h[0]), c.y + ((o & 2u) ? h[1] : -h[1]),
+			const float4 a = make_float4(c.x + ((o & 1u) ? h[0] : -h[0]), c.y + ((o & 2u) ? h[1] : -h[1]),
 				c.z + ((o & 4u) ? h[2] : -h[2]), 0.0f);
-			rec[2 * (size_t)i + 1] = make_float4(hw, bits(-list[o]), bits(length[o]), 0.0f);
+			rec[2 * (size_t)i] = a;
+			if (!inner_child[o]) {
+				// octree.inl: centre +- (half extent + EPS), the extent halfsize
+				// times the scale
+				const float w[3] = { hw * half[0] + EPS, hw * half[1] + EPS, hw * half[2] + EPS };
+				rec[2 * (size_t)i] = make_float4(a.x + -w[0], a.y + -w[1], a.z + -w[2], bits(list[o]));
+				rec[2 * (size_t)i + 1] = make_float4(a.x + w[0], a.y + w[1], a.z + w[2], bits(length[o]));
+			}
 			// the deepest level at which the move stays inside the parent
 			for (uint32_t axis = 0; axis < 3; ++axis)
 				for (uint32_t low = 0; low < 2; ++low) {
@@ -2029,6 +2040,7 @@ struct Cells {
 				}
 			if (inner_child[o]) {
 				inner.push_back(i);
+				scale.push_back(hw);
 				inner_depth.push_back((uint8_t)(inner_depth[k] + 1));
 			}
 		}
@@ -2039,7 +2051,7 @@ struct Cells {
 	{
 		const int32_t child = word(rec[2 * (size_t)i].w);
 		const uint32_t b = start_bits;
-		if (depth == b || child == 0) {
+		if (depth == b || child < 0) {
 			const uint32_t n = 1u << (b - depth);
 			for (uint32_t u = z * n; u < (z + 1) * n; ++u)
 				for (uint32_t v = y * n; v < (y + 1) * n; ++v)
@@ -2062,7 +2074,7 @@ struct Cells {
 			// level), in widths of the grid's cells, with a factor of four
 			start_eps = 0.0f;
 			for (int a = 0; a < 3; ++a) {
-				const float c = a == 0 ? rec[0].x : a == 1 ? rec[0].y : rec[0].z;
+				const float c = mid[a];
 				lo[a] = c - half[a];
 				inv[a] = std::ldexp(0.5f, (int)start_bits) / half[a];
 				const float far = (std::fabs(c) + half[a]) / (2.0f * half[a]);
@@ -2306,6 +2318,7 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 	g->g.next = g->next;
 	g->g.start = g->start;
 	g->g.lo = { cells.lo[0], cells.lo[1], cells.lo[2] };
+	g->g.hi = { center[0] + halfsize[0], center[1] + halfsize[1], center[2] + halfsize[2] };
 	g->g.inv = { cells.inv[0], cells.inv[1], cells.inv[2] };
 	g->g.start_eps = cells.start_eps;
 	g->g.start_bits = cells.start_bits;
@@ -2318,6 +2331,8 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 	g->g.ntri = (int)ntri;
 	g->g.step_eps = 3e-7f * (std::fabs(center[0]) + halfsize[0] + std::fabs(center[1]) + halfsize[1] +
 		std::fabs(center[2]) + halfsize[2]) + 1e-6f;
+	g->g.wall_eps = 4e-6f * (std::fabs(center[0]) + halfsize[0] + std::fabs(center[1]) + halfsize[1] +
+		std::fabs(center[2]) + halfsize[2]) + 1.01e-3f;
 	g->max_material = -1;
 	for (int64_t i = 0; i < ntri; ++i)
 		g->max_material = std::max(g->max_material, std::max(tris[i].material_in, tris[i].material_out));
@@ -2817,6 +2832,12 @@ StepArgs step_args(const nbl_driver* d)
 	a.max_mats = 0;
 	for (const WorldDesc& w : d->h_worlds)
 		a.max_mats = std::max<uint32_t>(a.max_mats, (uint32_t)w.nmats);
+	a.same_grid = 1;
+	for (int i = 0; i < d->W.nmats; ++i)
+		a.same_grid &= d->h_mats[i].imfp2 ? 1u : 0u;
+	for (size_t w = 1; w < d->h_worlds.size(); ++w)
+		for (int i = 0; i < d->h_worlds[w].nmats; ++i)
+			a.same_grid &= d->h_world_mats[w - 1][i].imfp2 ? 1u : 0u;
 	return a;
 }
 
@@ -3848,6 +3869,9 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 	a.slots = slots;
 	a.K = steps_per_launch;
 	a.max_mats = (uint32_t)n_mats;
+	a.same_grid = 1;
+	for (int i = 0; i < n_mats; ++i)
+		a.same_grid &= mats[i]->m.imfp2 ? 1u : 0u;
 	static_assert(NA_MAX_MATERIALS <= STEP_MATS, "materials in LDS");
 	const size_t lds_mats = sizeof(StepMat) * a.max_mats;
 	const uint32_t g_refill = blocks_for(capacity);

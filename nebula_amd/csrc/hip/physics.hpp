@@ -169,13 +169,15 @@ __device__ inline float pf_exp(float x)
 }
 
 // pf_exp, short for |x| <= 86 (the power of two is a normal float there)
-__device__ __forceinline__ float pf_exp_fast(float x)
+__device__ __forceinline__ float pf_exp_short(float x)
 {
-	if (!(fabsf(x) <= 86.0f))
-		return pf_exp(x);
 	const float kf = rintf(x * PF_INV_LN2);
 	const float r = (x - kf * PF_LN2_HI) - kf * PF_LN2_LO;
 	return __builtin_amdgcn_ldexpf(1.0f + (r + (r * r) * pf_exp_p(r)), (int)kf);
+}
+__device__ __forceinline__ float pf_exp_fast(float x)
+{
+	return (fabsf(x) <= 86.0f) ? pf_exp_short(x) : pf_exp(x);
 }
 
 __device__ inline float pf_expm1(float x)
@@ -326,6 +328,11 @@ __device__ __forceinline__ float mag2(F3 a) { return a.x * a.x + a.y * a.y + a.z
 __device__ __forceinline__ F3 normalised(F3 a)
 {
 	return v_mul(a, rsqrt_ieee(a.x * a.x + a.y * a.y + a.z * a.z));
+}
+// The same for a normalised vector (or NaN, or zero: then NaN, as above).
+__device__ __forceinline__ F3 normalised_unit(F3 a)
+{
+	return v_mul(a, rcp_mid(sqrt_mid(a.x * a.x + a.y * a.y + a.z * a.z)));
 }
 // vector_math.h:171-186; phi in [0, 2 pi]
 __device__ __forceinline__ F3 make_normal_vec(F3 dir, float phi)
@@ -638,12 +645,13 @@ __device__ __forceinline__ void log_imfps(const Material& m, float x, float& el,
 	el = t1_get(m.el_imfp, x);
 	in = t1_get(m.in_imfp, x);
 }
-__device__ __forceinline__ void log_imfps(const StepMat& m, float x, float& el, float& in)
+// `same`: all tables share their energies (a uniform branch)
+__device__ __forceinline__ void log_imfps(const StepMat& m, float x, float& el, float& in, bool same = false)
 {
 	const float xe = (x - m.el.xmin) * m.el.xstep;
 	const float le = t_index(xe, m.el.topx), fe = xe - le;
 	float e0, e1, i0, i1, fi;
-	if (m.imfp2) {
+	if (same || m.imfp2) {
 		const float4a8 v = *(const __attribute__((address_space(1))) float4a8*)((GFloat2*)m.imfp2 + (int)le);
 		e0 = v.x; i0 = v.y; e1 = v.z; i1 = v.w;
 		fi = fe;
@@ -707,11 +715,12 @@ struct Geometry {
 	// triangle index.
 	const float4* scr;
 	// The octree's cells, inner ones and leaves, numbered from 1 with the
-	// eight children of a cell in a row (0: the root).  cells[2 i]: centre of
-	// cell i, with the roundings of the reference's descent, and its first
-	// child in integer bits (0: a leaf); cells[2 i + 1], of a leaf: its scale
-	// (half extents over the root's) and in integer bits the start of its list
-	// in `od` and the list's length.
+	// eight children of a cell in a row (0: the root).  Of an inner cell,
+	// cells[2 i] is its centre, with the roundings of the reference's descent,
+	// and in integer bits its first child; of a leaf, cells[2 i] are its lower
+	// walls as a ray meets them (EPS outside, in the reference's roundings) and
+	// the negative start of its list in `od`, cells[2 i + 1] its upper walls
+	// and the list's length.
 	const float4* cells;
 	// next[8 i + 2 axis + (0 or 1)]: the cell that a ray leaving leaf i
 	// through its upper (0) or lower (1) wall of that axis enters, or an inner
@@ -722,7 +731,8 @@ struct Geometry {
 	// above that level fills its part.  A position closer than start_eps (in
 	// these cells' widths) to one of their walls starts at the root instead.
 	const uint32_t* start;
-	F3 lo, inv;
+	F3 lo, inv;             // lo: the domain's lower walls, centre - halfsize
+	F3 hi;                  // its upper walls
 	float start_eps, start_n;   // start_n: 2^b
 	uint32_t start_bits;
 	F3 center, halfsize;
@@ -732,6 +742,7 @@ struct Geometry {
 	// update's error, summed over components, plus the safety's own
 	// subtraction): 3e-7 x the domain's largest 1-norm + 1e-6 nm.
 	float step_eps;
+	float wall_eps;         // wall_safety's margin
 };
 
 // core/triangle.inl:7-28
@@ -760,10 +771,9 @@ __device__ __forceinline__ float intersect_ray(const Tri& t, F3 start, F3 dir)
 // geometry/octree.inl:24-30
 __device__ __forceinline__ bool in_domain(const Geometry& g, F3 p)
 {
-	const F3 c = g.center, h = g.halfsize;
-	return (p.x > c.x - h.x) && (p.x < c.x + h.x)
-		&& (p.y > c.y - h.y) && (p.y < c.y + h.y)
-		&& (p.z > c.z - h.z) && (p.z < c.z + h.z);
+	return (p.x > g.lo.x) && (p.x < g.hi.x)
+		&& (p.y > g.lo.y) && (p.y < g.hi.y)
+		&& (p.z > g.lo.z) && (p.z < g.hi.z);
 }
 
 // Levels of the octree at most (the builder's limit).
@@ -790,53 +800,47 @@ __device__ __forceinline__ uint32_t cell_start(const Geometry& g, F3 p)
 	const float fx = __builtin_amdgcn_fractf(tx), fy = __builtin_amdgcn_fractf(ty), fz = __builtin_amdgcn_fractf(tz);
 	// near a wall, where the rounding of t could name the other side, and
 	// outside the domain (also for a NaN): from the root
-	if (!(tx >= 0.0f && ty >= 0.0f && tz >= 0.0f && fmaxf(fmaxf(tx, ty), tz) < g.start_n
-			&& fminf(fminf(fx, fy), fz) >= g.start_eps && fmaxf(fmaxf(fx, fy), fz) <= 1.0f - g.start_eps))
+	const bool sure = (int)(tx >= 0.0f) & (int)(ty >= 0.0f) & (int)(tz >= 0.0f) & (int)(fmaxf(fmaxf(tx, ty), tz) < g.start_n)
+		& (int)(fminf(fminf(fx, fy), fz) >= g.start_eps) & (int)(fmaxf(fmaxf(fx, fy), fz) <= 1.0f - g.start_eps);
+	if (!sure)
 		return 0u;
 	return g.start[((((uint32_t)tz << g.start_bits) | (uint32_t)ty) << g.start_bits) | (uint32_t)tx];
 }
 
-// cell_find: the leaf that holds `cur`, from `cell` downwards, with its centre
-// (ax, ay, az) and scale aw; returns the start of its triangle list and its
-// length in `count`.
-__device__ __forceinline__ int cell_find(const Geometry& g, F3 cur, uint32_t& cell,
-	float& ax, float& ay, float& az, float& aw, int& count)
+// cell_find: the leaf that holds `cur`, from `cell` downwards, with its walls;
+// returns the start of its triangle list and its length in `count`.
+__device__ __forceinline__ int cell_find(const Geometry& g, F3 cur, uint32_t& cell, F3& lo, F3& hi, int& count)
 {
 	for (;;) {
 		const float4 a = g.cells[2 * (size_t)cell];
-		const uint32_t child = __float_as_uint(a.w);
-		if (child == 0u) {
-			const float4 e = g.cells[2 * (size_t)cell + 1];
-			ax = a.x; ay = a.y; az = a.z; aw = e.x;
-			count = __float_as_int(e.z);
-			return __float_as_int(e.y);
+		const int child = __float_as_int(a.w);
+		if (child < 0) {
+			const float4 b = g.cells[2 * (size_t)cell + 1];
+			lo = { a.x, a.y, a.z };
+			hi = { b.x, b.y, b.z };
+			count = __float_as_int(b.w);
+			return -child;
 		}
-		cell = child + ((cur.x > a.x) ? 1u : 0u) + ((cur.y > a.y) ? 2u : 0u) + ((cur.z > a.z) ? 4u : 0u);
+		cell = (uint32_t)child + ((cur.x > a.x) ? 1u : 0u) + ((cur.y > a.y) ? 2u : 0u) + ((cur.z > a.z) ? 4u : 0u);
 	}
 }
 
-// Distance to the cell wall the ray leaves through (target -1/-2/-4 for the
+// Distance to the cell wall the ray leaves through (target -1/-2/-3 for the
 // x/y/z wall).
-__device__ __forceinline__ void cell_exit(const Geometry& g, F3 cur, F3 dir, float ax, float ay, float az,
-	float aw, float& isect, int& target)
+__device__ __forceinline__ void cell_exit(F3 cur, F3 dir, F3 lo, F3 hi, float& isect, int& target)
 {
-	const F3 hs = g.halfsize;
-	const float hx = aw * hs.x, hy = aw * hs.y, hz = aw * hs.z;
-	const float nx = ax + copysignf(hx + EPS, dir.x) - cur.x, ny = ay + copysignf(hy + EPS, dir.y) - cur.y,
-		nz = az + copysignf(hz + EPS, dir.z) - cur.z;
-	float tx, ty, tz;
-	if (fminf(fminf(fabsf(dir.x), fabsf(dir.y)), fabsf(dir.z)) >= 0x1p-90f) {
-		tx = div_mid(nx, dir.x);
-		ty = div_mid(ny, dir.y);
-		tz = div_mid(nz, dir.z);
-	} else {
+	const float nx = ((__float_as_int(dir.x) < 0) ? lo.x : hi.x) - cur.x,
+		ny = ((__float_as_int(dir.y) < 0) ? lo.y : hi.y) - cur.y,
+		nz = ((__float_as_int(dir.z) < 0) ? lo.z : hi.z) - cur.z;
+	float tx = div_mid(nx, dir.x), ty = div_mid(ny, dir.y), tz = div_mid(nz, dir.z);
+	if (!(fminf(fminf(fabsf(dir.x), fabsf(dir.y)), fabsf(dir.z)) >= 0x1p-90f)) {
 		tx = nx / dir.x;
 		ty = ny / dir.y;
 		tz = nz / dir.z;
 	}
 	if ((tx < ty) && (tx < tz)) { isect = tx; target = -1; }
 	else if ((ty < tx) && (ty < tz)) { isect = ty; target = -2; }
-	else { isect = tz; target = -4; }
+	else { isect = tz; target = -3; }
 }
 
 // Candidate test: octree.inl:128-138 skips triangles whose outgoing material
@@ -935,26 +939,24 @@ __device__ __forceinline__ float pair_safety(const Screen& s)
 	return __builtin_fmaf(-2e-6f * s.slen, s.ee, fabsf(s.d0)) * s.rden;
 }
 
-// Wall part: distance from `cur` to the walls of its leaf cell (centre
-// a, half extents aw x halfsize), less a margin that covers the rounding of
-// cell_exit's exit distances (a few unit roundoffs of the coordinates'
-// magnitudes, and EPS pushes the walls outwards): a segment that ends at
-// least that far inside the cell is seen to end before the cell's exit.
-__device__ __forceinline__ float wall_safety(const Geometry& g, F3 cur, float ax, float ay, float az, float aw)
+// Wall part: distance from `cur` to the walls of its leaf cell, less a margin
+// that covers the rounding of cell_exit's exit distances (a few unit roundoffs
+// of the coordinates' magnitudes: 4e-6 of the domain's largest 1-norm, and 1e-3
+// nm, which holds the EPS by which the walls are outside): a segment that ends
+// at least that far inside the cell is seen to end before the cell's exit.
+__device__ __forceinline__ float wall_safety(const Geometry& g, F3 cur, F3 lo, F3 hi)
 {
-	const F3 hs = g.halfsize;
-	const float hx = aw * hs.x, hy = aw * hs.y, hz = aw * hs.z;
-	const float w = fminf(fminf(hx - fabsf(cur.x - ax), hy - fabsf(cur.y - ay)), hz - fabsf(cur.z - az));
-	const float mag = fabsf(ax) + fabsf(ay) + fabsf(az) + hx + hy + hz;
-	return w - (1e-3f + 4e-6f * mag);
+	const float a = fminf(fminf(cur.x - lo.x, cur.y - lo.y), cur.z - lo.z);
+	const float b = fminf(fminf(hi.x - cur.x, hi.y - cur.y), hi.z - cur.z);
+	return fminf(a, b) - g.wall_eps;
 }
 
-// The cell across wall `target` (-1/-2/-4); 0 means the ray left the octree.
+// The cell across wall `target` (-1/-2/-3); 0 means the ray left the octree.
 __device__ __forceinline__ uint32_t cell_next(const Geometry& g, uint32_t cell, int target, F3 dir)
 {
 	const float d = target == -1 ? dir.x : target == -2 ? dir.y : dir.z;
-	const uint32_t axis = (uint32_t)(-target) >> 1;   // 0, 1, 2
-	return g.next[8 * (size_t)cell + 2u * axis + ((d >= 0.0f) ? 0u : 1u)];
+	const uint32_t axis = (uint32_t)~target;
+	return g.next[8 * (size_t)cell + (2u * axis + (__float_as_uint(d) >> 31))];
 }
 
 // geometry/octree.inl:32-192: walk from leaf to leaf; returns the
@@ -968,13 +970,13 @@ __device__ inline int propagate(const Geometry& g, F3 start, F3 dir, float dista
 	uint32_t cell = cell_start(g, start);
 	uint32_t cells = 0;
 	do {
-		float ax, ay, az, aw;
+		F3 lo, hi;
 		int count;
-		int index = cell_find(g, cur, cell, ax, ay, az, aw, count);
+		int index = cell_find(g, cur, cell, lo, hi, count);
 		++cells;
 		float isect;
 		int target;
-		cell_exit(g, cur, dir, ax, ay, az, aw, isect, target);
+		cell_exit(cur, dir, lo, hi, isect, target);
 		for (;;) {
 			const int ti = od[index++];
 			if (ti < 0)
@@ -1140,15 +1142,15 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, WaveMe
 	target = 0;
 	isect = 0.0f;
 	if (active) {
-		float ax, ay, az, aw;
+		F3 lo, hi;
 		const F3 cur = xyz(m.cur[lane]), dir = xyz(m.dir[lane]);
 		uint32_t cell = m.cell[lane];
-		off = cell_find(g, cur, cell, ax, ay, az, aw, n);
+		off = cell_find(g, cur, cell, lo, hi, n);
 		m.cell[lane] = cell;
 		++cells;
-		cell_exit(g, cur, dir, ax, ay, az, aw, isect, target);
+		cell_exit(cur, dir, lo, hi, isect, target);
 		if (SAF)
-			m.saf[lane] = __float_as_uint(fmaxf(wall_safety(g, cur, ax, ay, az, aw), 0.0f));
+			m.saf[lane] = __float_as_uint(fmaxf(wall_safety(g, cur, lo, hi), 0.0f));
 	}
 	const int incl = wave_incl_sum(n);
 	const int excl = incl - n;
@@ -1272,10 +1274,10 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 		int n = 0, off = 0, target = 0;
 		float isect = 0.0f;
 		if (active) {
-			float ax, ay, az, aw;
-			off = cell_find(g, w.cur, w.cell, ax, ay, az, aw, n);
+			F3 lo, hi;
+			off = cell_find(g, w.cur, w.cell, lo, hi, n);
 			++w.cells;
-			cell_exit(g, w.cur, dir, ax, ay, az, aw, isect, target);
+			cell_exit(w.cur, dir, lo, hi, isect, target);
 		}
 		const int incl = wave_incl_sum(n);
 		const int excl = incl - n;
@@ -1372,8 +1374,9 @@ __device__ __forceinline__ void elastic_execute(const M& m, uint32_t fl, Particl
 		cos_theta = clampr(el_cosine(m, x, y), -1.0f, 1.0f);
 		sin_theta = sqrt_mid(1.0f - cos_theta * cos_theta);   // 0 or at least 2^-24
 	}
-	tp.dir = normalised(tp.dir);
-	const F3 normal_dir = normalised(make_normal_vec(tp.dir, rng_phi(rng)));
+	// the direction is the step's normalised one
+	tp.dir = normalised_unit(tp.dir);
+	const F3 normal_dir = normalised_unit(make_normal_vec(tp.dir, rng_phi(rng)));
 	tp.dir = v_add(v_mul(tp.dir, cos_theta), v_mul(normal_dir, sin_theta));
 	if (tp.E < 200.0f) {
 		if (fl & PH_EL_PHONON)
@@ -1584,7 +1587,7 @@ __device__ __forceinline__ int boundary_execute(const M* mats, uint32_t fl, cons
 {
 	if (g) *g = 0.0f;
 	Particle tp = p;
-	const F3 nd = normalised(tp.dir);
+	const F3 nd = normalised_unit(tp.dir);   // the step's normalised direction
 	const F3 n = normalised(cross(tri.e1, tri.e2));
 	const float cos_theta = dot(n, nd);
 	int mi, mo;
@@ -1711,6 +1714,50 @@ __device__ __forceinline__ int step_plan(const World& W, const M* mats, const St
 	nd = planned ? s.p.dir : normalised(s.p.dir);
 	pinfo.tau_el = tau_el;
 	pinfo.tau_in = tau_in;
+	return ALIVE;
+}
+
+// The same without its special cases one by one: the short forms in a row and
+// one check that their operands were in range (else step_plan).
+template <class R>
+__device__ __forceinline__ int step_plan_short(const World& W, const StepMat* mats, bool same, const State& s, R& rng,
+	F3& nd, float& distance, int& type, PathInfo& pinfo, bool planned)
+{
+	pinfo.type = 0;
+	pinfo.logE = 0.0f;
+	pinfo.tau_el = pinfo.tau_in = 0.0f;
+	type = 0;
+	if (!in_domain(W.g, s.p.pos))
+		return TERMINATED;
+	distance = W.g.max_extent;
+	const R rng0 = rng;
+	const float m2 = s.p.dir.x * s.p.dir.x + s.p.dir.y * s.p.dir.y + s.p.dir.z * s.p.dir.z;
+	nd = planned ? s.p.dir : v_mul(s.p.dir, rcp_mid(sqrt_mid(m2)));
+	bool ok = planned || is_mid(m2);
+	if (s.mat >= 0) {
+		const StepMat& m = mats[s.mat];
+		if (s.p.E < m.barrier + W.threshold)
+			return TERMINATED;
+		const float logE = pf_log_normal(s.p.E);
+		pinfo.logE = logE;
+		float log_el, log_in;
+		log_imfps(m, logE, log_el, log_in, same);
+		pinfo.tau_el = rcp_mid(pf_exp_short(log_el)) * m.el_scale;
+		pinfo.tau_in = rcp_mid(pf_exp_short(log_in)) * m.in_scale;
+		const float pe = -pinfo.tau_el * pf_log_normal(rng_unit(rng));
+		const float pi = -pinfo.tau_in * pf_log_normal(rng_unit(rng));
+		// normal energy, exponentials in [2^-100, 2^100] (or NaN)
+		ok = ok && __float_as_uint(s.p.E) - 0x00800000u < 0x7f000000u && fmaxf(fabsf(log_el), fabsf(log_in)) <= 69.0f;
+		// (as in step_plan: elastic first, strictly shorter wins)
+		float dist = __builtin_inff();
+		if (pe < dist) { type = 2; dist = pe; }
+		if (pi < dist) { type = 1; dist = pi; }
+		distance = dist;
+	}
+	if (!ok) {
+		rng = rng0;
+		return step_plan(W, mats, s, rng, nd, distance, type, pinfo, planned);
+	}
 	return ALIVE;
 }
 

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from nebula_amd import api as A
+from nebula_amd import workloads as W
 from oracle import pyoracle as O
 from tests.helpers import material, slab_tris
 from tests.test_gpu_parity import _to_oracle_states
@@ -46,6 +47,42 @@ def test_steps_off_the_usual_range(model, scale):
     assert np.array_equal(g_made, o_made)
     for k in ("pos", "dir", "E"):
         a, b = g_st[k].reshape(n, -1), o_st[k].reshape(n, -1)
+        same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))
+        assert same.all(), (k, int((~same).any(axis=1).sum()))
+    dev.close()
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-12, 3e4])
+@pytest.mark.parametrize("few", [0, None])
+def test_tracks_off_the_usual_range(scale, few):
+    """Primaries of such directions and energies through the step kernels."""
+    dev = A.Device(0)
+    tris, raw = slab_tris(), [material("si"), material("pmma")]
+    ow = O.OracleWorld(tris, raw)
+    d = A.Driver(dev, 4096, A.Geometry(dev, tris), [A.Material(dev, A.HostMaterial(m)) for m in raw], seed=7)
+    if few is not None:
+        d.set_cascade(few)
+    rng = np.random.default_rng(4)
+    n = 700
+    pri = W.raster_scan(n, 1, 1, 300.0, -60.0, 60.0, -60.0, 60.0, 5.0, seed=1)
+    for a in range(3):
+        pri["dir"][:, a] = SMALL[rng.integers(0, len(SMALL), n)] * np.float32(scale)
+    pri["dir"][:, 2] = -np.abs(pri["dir"][:, 2])
+    zero = ~np.any(np.abs(pri["dir"]) > 1e-18, axis=1)
+    pri["dir"][zero, 2] = -1.0
+    pri["E"] = np.exp(rng.uniform(np.log(12.0), np.log(900.0), n)).astype(np.float32)
+    pri["E"][::53] = np.float32(1e-40)
+    pri["E"][1::53] = np.float32(1.0)
+    tags = np.arange(n, dtype=np.uint32)
+    print(scale, few, flush=True)
+    d.push(pri, tags)
+    det = np.sort(d.run(100 * n), order="sid")
+    ref, steps = ow.run_philox(pri, 7, 100 * n, threads=8)
+    ref = np.sort(ref.astype(det.dtype), order="sid")
+    assert d.steps() == steps
+    assert len(det) == len(ref) > n // 10
+    for k in ("pos", "dir", "E"):
+        a, b = det[k].reshape(len(det), -1), ref[k].reshape(len(ref), -1)
         same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))
         assert same.all(), (k, int((~same).any(axis=1).sum()))
     dev.close()
