@@ -896,10 +896,10 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 
 // Write the wave's particles out: detected records, the inelastic queue and
 // the survivors, with one ballot per kind and one atomic per wave for the
-// last two together.  `m`: with walks that go on in the next launch, or null.
+// last two together (the general variant).
 template <bool SC>
 __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
-	bool keep, bool det, bool to_inel, const WaveMem* m, const InFlight& f)
+	bool keep, bool det, bool to_inel)
 {
 	const Bufs out = out_buf ? a.buf[1] : a.buf[0];
 	const int np = a.map.np;
@@ -926,12 +926,93 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 		if (SC) store_score(a.inel, qslot, np, sc);
 	}
 	if (survive) {
-		if (m && f.on)
-			s.flags |= keep_walk(a, out_buf, oslot, *m, __lane_id(), f);
 		store_state(out, oslot, s);
 		if (SC) store_score(out, oslot, np, sc);
 	}
 }
+
+// The same for a block's waves together, with one atomic a block and counter
+// (every thread calls).  All atomics of a launch on one counter are served one
+// after the other, beyond the L2s (each XCD has its own), at about ATOMIC_NS ns
+// each: with two or three for each of the 67 000 waves of a launch of 4.2
+// million particles, the counters took most of the launch.  A wave waits for
+// the block's others, which are as long on their way (K turns).
+template <bool SC, uint32_t WAVES>
+__device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
+	bool keep, bool det, bool to_inel, const WaveMem& m, const InFlight& f, uint32_t wave_steps)
+{
+	__shared__ uint32_t s_n[4][WAVES];   // detected, survivors, queued, steps of each wave
+	__shared__ uint32_t s_at[3];
+	const Bufs out = out_buf ? a.buf[1] : a.buf[0];
+	const int np = a.map.np;
+	const uint32_t wave = threadIdx.x >> 6, lane = __lane_id();
+	const bool queue = keep && to_inel;
+	bool survive = keep && !to_inel && !det;
+	const uint64_t md = __ballot(det), ms = __ballot(survive), mq = __ballot(queue);
+	if (lane == 0) {
+		s_n[0][wave] = (uint32_t)__popcll(md);
+		s_n[1][wave] = (uint32_t)__popcll(ms);
+		s_n[2][wave] = (uint32_t)__popcll(mq);
+		s_n[3][wave] = wave_steps;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		uint32_t n[4] = {};
+		for (uint32_t w = 0; w < WAVES; ++w)
+			for (int k = 0; k < 4; ++k)
+				n[k] += s_n[k][w];
+		if (n[3])
+			atomicAdd((unsigned long long*)&C->steps, (unsigned long long)n[3]);
+		const uint64_t at = (n[1] | n[2]) ? atomicAdd((unsigned long long*)&C->step_out,
+			((unsigned long long)n[2] << 32) | n[1]) : 0ull;
+		s_at[0] = n[0] ? atomicAdd(&C->det_ctr, n[0]) : 0u;
+		s_at[1] = lo32(at);
+		s_at[2] = hi32(at);
+	}
+	__syncthreads();
+	const uint64_t below = (1ull << lane) - 1ull;
+	uint32_t dslot = s_at[0] + (uint32_t)__popcll(md & below), oslot = s_at[1] + (uint32_t)__popcll(ms & below),
+		qslot = s_at[2] + (uint32_t)__popcll(mq & below);
+	for (uint32_t w = 0; w < wave; ++w) {
+		dslot += s_n[0][w];
+		oslot += s_n[1][w];
+		qslot += s_n[2][w];
+	}
+	const bool over = det && dslot >= a.det_cap;
+	if (__ballot(over)) {
+		// no record slot: wait as a survivor and retry next launch
+		uint32_t at, none;
+		wave_alloc2(&C->step_out, over, false, at, none);
+		if (over) {
+			s.flags |= FL_PEND_DET;
+			survive = true;
+			oslot = at;
+		}
+	}
+	if (det && !over) {
+		store_detected(a, dslot, s);
+		if (SC) {
+			for (int q = 0; q < np; ++q)
+				a.det_sc[(size_t)dslot * np + q] = sc.at[q * sc.stride];
+		}
+	}
+	if (queue) {
+		store_state(a.inel, qslot, s);
+		if (SC) store_score(a.inel, qslot, np, sc);
+	}
+	if (survive) {
+		if (f.on)
+			s.flags |= keep_walk(a, out_buf, oslot, m, lane, f);
+		store_state(out, oslot, s);
+		if (SC) store_score(out, oslot, np, sc);
+	}
+}
+
+#ifndef STEP_W
+#define STEP_W 4
+#endif
+// Waves of a block of k_step
+template <bool SC> constexpr uint32_t step_waves() { return SC ? 4u : STEP_W; }
 
 template <bool SC, bool WUNI, bool DEP>
 __device__ __forceinline__ void step_body(const StepArgs& a)
@@ -948,34 +1029,36 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	World Wl = a.W;
 	const World& W = WUNI ? Wl : a.W;
-	__shared__ WaveMem s_mem[4];
+	constexpr uint32_t WAVES = step_waves<SC>();
+	__shared__ WaveMem s_mem[WAVES];
 	WaveMem& m = s_mem[threadIdx.x >> 6];
 	const uint32_t lane = __lane_id();
 	// scores, then the materials (the block's, or with several worlds each
 	// wave's); step_lds is their size
 	extern __shared__ double s_dyn[];
-	ScoreLds sc = { s_dyn + threadIdx.x, 256 };
-	StepMat* const mats = (StepMat*)(s_dyn + (SC ? np * 256 : 0)) + (WUNI ? (threadIdx.x >> 6) * a.max_mats : 0u);
+	ScoreLds sc = { s_dyn + threadIdx.x, 64 * (int)WAVES };
+	StepMat* const mats = (StepMat*)(s_dyn + (SC ? np * 64 * (int)WAVES : 0)) + (WUNI ? (threadIdx.x >> 6) * a.max_mats : 0u);
 	if (!WUNI) {
 		if (threadIdx.x < (uint32_t)a.W.nmats)
 			load_step_mat(mats[threadIdx.x], a.W.mats[threadIdx.x]);
 		__syncthreads();
 	}
 
-	uint32_t wave_steps = 0;
-	const uint32_t stride = gridDim.x * blockDim.x;
+	const uint32_t stride = gridDim.x * 64u * WAVES;
 	// Whole waves take consecutive particles and step in lockstep: the walk
 	// shares its triangle tests across the wave (walk_round), so every
 	// lane joins it each turn, also lanes whose particle has stopped.
-	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
+	// (A block's waves go through the loop together: emit_block.)
+	const uint32_t wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
 	// world-per-wave: index i names particle perm[i] (~0u: padding), or
 	// particle i when the launch holds one world's particles only
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
-	for (uint32_t w0 = wave0; w0 < n_loop; w0 += stride) {
-		const uint32_t i = w0 + lane;
+	for (uint32_t b0 = blockIdx.x * 64u * WAVES; b0 < n_loop; b0 += stride) {
+		const uint32_t i = b0 + wave0 + lane;
 		const uint32_t li = (WUNI && !ident) ? ((i < n_loop) ? a.perm[i] : ~0u) : i;
 		const bool valid = (WUNI && !ident) ? li != ~0u : i < n_in;
+		uint32_t wave_steps = 0;
 		const uint32_t slot = valid ? in_slot(li, n_surv, a.slots) : 0u;
 		InFlight f = {};
 		float rem = -1.0f;
@@ -994,9 +1077,9 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		}
 		if (WUNI) {
 			// lane 0 holds a particle (each world's range starts at a multiple
-			// of 64 and has no padding before its last particle; with one
-			// world, w0 < n_in): its world is the wave's, and no lane holds
-			// another world's particle
+			// of 64 and has no padding before its last particle), unless the
+			// wave has none: its world is the wave's, and no lane holds another
+			// world's particle
 			load_world(a, __builtin_amdgcn_readfirstlane(flags >> FL_WORLD_SHIFT), Wl);
 			if (lane < (uint32_t)Wl.nmats)
 				load_step_mat(mats[lane], Wl.mats[lane]);
@@ -1038,10 +1121,10 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		}
 		// of a walk that goes on: the safety of its start point
 		s.safe = rem;
-		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, &m, f);
+		emit_block<SC, WAVES>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, m, f, wave_steps);
+		if (b0 + stride < n_loop && b0 + stride > b0)
+			__syncthreads();   // its counts are rewritten by the next round
 	}
-	if (lane == 0 && wave_steps)
-		atomicAdd((unsigned long long*)&C->steps, (unsigned long long)wave_steps);
 }
 
 // The general variant: lanes of different worlds (flags bits 16..31), each
@@ -1142,7 +1225,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 			}
 		}
 		s.safe = -1.0f;
-		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel, nullptr, InFlight());
+		emit<SC>(a, C, bi ^ 1u, s, sc, valid && !dead, det, to_inel);
 	}
 	count_steps(C, my_steps);
 }
@@ -1155,7 +1238,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 #define NBL_PLAIN_WAVES 5
 #endif
 template <bool SC, bool MULTI, bool WUNI = false, bool DEP = false>
-__global__ __launch_bounds__(256) void k_step(StepArgs a)
+__global__ __launch_bounds__(MULTI ? 256 : 64 * step_waves<SC>()) void k_step(StepArgs a)
 {
 	if constexpr (MULTI)
 		step_multi<SC>(a);
@@ -1163,13 +1246,13 @@ __global__ __launch_bounds__(256) void k_step(StepArgs a)
 		step_body<SC, WUNI, DEP>(a);
 }
 template <>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
+__global__ __launch_bounds__(64 * STEP_W) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, false, false>(StepArgs a)
 {
 	step_body<false, false, false>(a);
 }
 template <>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
+__global__ __launch_bounds__(64 * STEP_W) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, true, false>(StepArgs a)
 {
 	step_body<false, true, false>(a);
@@ -2758,7 +2841,7 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 	// these, and more materials than LDS is to hold
 	const bool multi = d->h_worlds.size() > 1 || (d->dep && d->map.np) || a.max_mats > STEP_MATS;
 	const size_t mats = sizeof(StepMat) * a.max_mats;
-	const dim3 grid(g), block(256), cgrid(cascade_waves(d->dev)), cblock(64);
+	const dim3 grid(g), block(256), sgrid((g * 4u + STEP_W - 1) / STEP_W), sblock(64 * STEP_W), cgrid(cascade_waves(d->dev)), cblock(64);
 	if (multi && !d->dep && !d->map.np && a.max_mats <= STEP_MATS) {
 		// several worlds, nothing but records: the launch's particles
 		// grouped by world, one world per wave
@@ -2779,7 +2862,7 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 			hipLaunchKernelGGL(k_world_place, dim3(WG_BLOCKS), dim3(WG_THREADS), 0, d->stream, d->ctrl, d->buf[0],
 				d->buf[1], d->slots, nw, d->wgrp, d->perm);
 		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 4 * mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, true>), sgrid, sblock, STEP_W * mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else if (d->map.np && multi) {
 		hipLaunchKernelGGL((k_cascade<true, true>), cgrid, cblock, 0, d->stream, a);
@@ -2795,11 +2878,11 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else if (d->dep) {
 		hipLaunchKernelGGL((k_cascade<false, false, false, true>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, false, true>), grid, block, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, false, true>), sgrid, sblock, mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
 	} else {
 		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false>), grid, block, mats, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false>), sgrid, sblock, mats, d->stream, a);
 		hipLaunchKernelGGL((k_inel<false, false>), grid, block, 0, d->stream, a);
 	}
 }
@@ -3890,7 +3973,7 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 			hipLaunchKernelGGL(k_refill, dim3(g_refill), dim3(256), 0, st, ctrl, a.buf[0], a.buf[1], a.spill,
 				primaries, tags, (const uint64_t*)nullptr, (const uint16_t*)nullptr, 0u, sid_base);
 			hipLaunchKernelGGL((k_cascade<false, false>), dim3(cascade_waves(dev)), dim3(64), lds_mats, st, a);
-			hipLaunchKernelGGL((k_step<false, false>), dim3(g_step), dim3(256), lds_mats, st, a);
+			hipLaunchKernelGGL((k_step<false, false>), dim3((g_step * 4u + STEP_W - 1) / STEP_W), dim3(64 * STEP_W), lds_mats, st, a);
 			hipLaunchKernelGGL((k_inel<false, false>), dim3(g_step), dim3(256), 0, st, a);
 		}
 		HIP_OK(hipGetLastError());
