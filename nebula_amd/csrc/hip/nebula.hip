@@ -600,38 +600,33 @@ __device__ __forceinline__ void count_steps(Ctrl* C, uint32_t my_steps)
 		atomicAdd((unsigned long long*)&C->steps, (unsigned long long)v);
 }
 
-// Place a new secondary: the output buffer's SE region, else the spill
-// stack; returns false when both are full.  With scores, the secondary
-// starts from its parent's score.
+// Place a new secondary: the output buffer's SE region (slots below se_limit),
+// else entry `pslot` of the spill stack; returns false when both are full.
+// With scores, the secondary starts from its parent's score.
 template <bool SC, class S>
-__device__ __forceinline__ bool place_secondary(const StepArgs& a, Ctrl* C, const Bufs& out,
-	uint32_t se_limit, bool made, uint32_t sslot, const Particle& se, const State& parent, const S& psc)
+__device__ __forceinline__ bool place_secondary(const StepArgs& a, const Bufs& out, uint32_t se_limit, uint32_t sslot,
+	uint32_t pslot, const Particle& se, const State& parent, const S& psc)
 {
-	bool ok = true;
-	if (made) {
-		State ns;
-		ns.p = se;
-		ns.mat = parent.mat;
-		ns.last_tri = -1;
-		ns.tag = parent.tag;
-		ns.step = 0;
-		ns.flags = parent.flags & FL_WORLD_MASK;
-		ns.sid = se_sid(parent.sid, parent.step);
-		// it starts where its parent stands, so the parent's safety holds
-		ns.safe = parent.safe;
-		const bool spill = sslot >= se_limit;
-		const uint32_t pslot = wave_alloc(&C->spill_ctr, spill);
-		if (!spill) {
-			store_state(out, a.slots - 1u - sslot, ns);
-			if (SC) store_score(out, a.slots - 1u - sslot, a.map.np, psc);
-		} else if (pslot < a.spill_cap) {
-			store_state(a.spill, pslot, ns);
-			if (SC) store_score(a.spill, pslot, a.map.np, psc);
-		} else {
-			ok = false;
-		}
+	State ns;
+	ns.p = se;
+	ns.mat = parent.mat;
+	ns.last_tri = -1;
+	ns.tag = parent.tag;
+	ns.step = 0;
+	ns.flags = parent.flags & FL_WORLD_MASK;
+	ns.sid = se_sid(parent.sid, parent.step);
+	// it starts where its parent stands, so the parent's safety holds
+	ns.safe = parent.safe;
+	if (sslot < se_limit) {
+		store_state(out, a.slots - 1u - sslot, ns);
+		if (SC) store_score(out, a.slots - 1u - sslot, a.map.np, psc);
+	} else if (pslot < a.spill_cap) {
+		store_state(a.spill, pslot, ns);
+		if (SC) store_score(a.spill, pslot, a.map.np, psc);
+	} else {
+		return false;
 	}
-	return ok;
+	return true;
 }
 
 // Up to K steps per particle: init (domain, threshold, path sampling, octree
@@ -933,10 +928,11 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 
 // The same for a block's waves together, with one atomic a block and counter
 // (every thread calls).  All atomics of a launch on one counter are served one
-// after the other, beyond the L2s (each XCD has its own), at about ATOMIC_NS ns
-// each: with two or three for each of the 67 000 waves of a launch of 4.2
-// million particles, the counters took most of the launch.  A wave waits for
-// the block's others, which are as long on their way (K turns).
+// after the other, beyond the L2s (each XCD has its own), at 12 ns each: with
+// two or three for each of the 67 000 waves of a launch of 4.2 million
+// particles, the counters took most of the launch (the full image 239 ms, now
+// 200; blocks of 2 waves 209, of 8 205).  A wave waits for the block's others,
+// which are as long on their way (K turns).
 template <bool SC, uint32_t WAVES>
 __device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
 	bool keep, bool det, bool to_inel, const WaveMem& m, const InFlight& f, uint32_t wave_steps)
@@ -1008,11 +1004,6 @@ __device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t 
 	}
 }
 
-#ifndef STEP_W
-#define STEP_W 4
-#endif
-// Waves of a block of k_step
-template <bool SC> constexpr uint32_t step_waves() { return SC ? 4u : STEP_W; }
 
 template <bool SC, bool WUNI, bool DEP>
 __device__ __forceinline__ void step_body(const StepArgs& a)
@@ -1029,7 +1020,7 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 	const bool keep_walks = a.walk[0] && n_in >= KEEP_WALKS_MIN;
 	World Wl = a.W;
 	const World& W = WUNI ? Wl : a.W;
-	constexpr uint32_t WAVES = step_waves<SC>();
+	constexpr uint32_t WAVES = 4;
 	__shared__ WaveMem s_mem[WAVES];
 	WaveMem& m = s_mem[threadIdx.x >> 6];
 	const uint32_t lane = __lane_id();
@@ -1238,7 +1229,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 #define NBL_PLAIN_WAVES 5
 #endif
 template <bool SC, bool MULTI, bool WUNI = false, bool DEP = false>
-__global__ __launch_bounds__(MULTI ? 256 : 64 * step_waves<SC>()) void k_step(StepArgs a)
+__global__ __launch_bounds__(256) void k_step(StepArgs a)
 {
 	if constexpr (MULTI)
 		step_multi<SC>(a);
@@ -1246,13 +1237,13 @@ __global__ __launch_bounds__(MULTI ? 256 : 64 * step_waves<SC>()) void k_step(St
 		step_body<SC, WUNI, DEP>(a);
 }
 template <>
-__global__ __launch_bounds__(64 * STEP_W) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, false, false>(StepArgs a)
 {
 	step_body<false, false, false>(a);
 }
 template <>
-__global__ __launch_bounds__(64 * STEP_W) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NBL_PLAIN_WAVES, 8)))
 void k_step<false, false, true, false>(StepArgs a)
 {
 	step_body<false, true, false>(a);
@@ -1265,12 +1256,15 @@ void k_step<false, false, true, false>(StepArgs a)
 //
 // Every queued particle comes back as a survivor, so queue entry i goes to
 // survivor slot surv0 + i with no atomic.  Secondary slots are counted per
-// block (ballot per wave, the four counts in LDS, one atomic per block):
-// with one atomic per wave, the waves' atomics on one counter serialised in
-// L2 and this kernel took 7 % more of the iteration.  The block loop runs
-// whole blocks, so every thread reaches each barrier.
+// block (ballot per wave, the counts in LDS, one atomic per block, and one more
+// when some go to the spill stack): atomics on one counter are served one
+// after the other (emit_block).  Blocks of 512: the full image in 191.8 ms,
+// 194.6 with 256, 197.0 with 1024; 201 with 256 and an atomic a wave on the
+// spill stack.  The block loop runs whole blocks, so every thread reaches each
+// barrier.
+constexpr uint32_t INEL_THREADS = 512;
 template <bool SC, bool MULTI>
-__global__ __launch_bounds__(256) void k_inel(StepArgs a)
+__global__ __launch_bounds__(INEL_THREADS) void k_inel(StepArgs a)
 {
 	Ctrl* C = a.ctrl;
 	const uint32_t bi = C->buf_in;
@@ -1280,8 +1274,9 @@ __global__ __launch_bounds__(256) void k_inel(StepArgs a)
 	World Wl = a.W;
 	const World& W = MULTI ? Wl : a.W;
 	const uint32_t stride = gridDim.x * blockDim.x;
-	__shared__ uint32_t s_cnt[4], s_doa[4];
-	__shared__ uint32_t s_base;
+	constexpr uint32_t WAVES = INEL_THREADS / 64;
+	__shared__ uint32_t s_cnt[WAVES], s_doa[WAVES];
+	__shared__ uint32_t s_base, s_spill;
 	const uint32_t wave = threadIdx.x >> 6;
 	for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < n; b0 += stride) {
 		const uint32_t i = b0 + threadIdx.x;
@@ -1322,19 +1317,29 @@ __global__ __launch_bounds__(256) void k_inel(StepArgs a)
 		}
 		__syncthreads();
 		if (threadIdx.x == 0) {
-			const uint32_t tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-			const uint32_t totd = s_doa[0] + s_doa[1] + s_doa[2] + s_doa[3];
-			s_base = (tot | totd) ? lo32(atomicAdd((unsigned long long*)&C->se_ctr,
+			uint32_t tot = 0, totd = 0;
+			for (uint32_t w = 0; w < WAVES; ++w) {
+				tot += s_cnt[w];
+				totd += s_doa[w];
+			}
+			const uint32_t at = (tot | totd) ? lo32(atomicAdd((unsigned long long*)&C->se_ctr,
 				((unsigned long long)totd << 32) | tot)) : 0u;
+			s_base = at;
+			// those from slot se_limit on go to the spill stack, slot sslot to
+			// entry sslot + s_spill
+			const uint32_t first = max(at, se_limit);
+			if (tot && at + tot > first)
+				s_spill = atomicAdd(&C->spill_ctr, at + tot - first) - first;
 		}
 		__syncthreads();
 		uint32_t sslot = s_base + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull));
 		for (uint32_t w = 0; w < wave; ++w)
 			sslot += s_cnt[w];
+		const uint32_t pslot = sslot + s_spill;
 		__syncthreads();   // s_cnt and s_base are rewritten by the next round
 		if (valid) {
 			bool done = true;
-			if (place_secondary<SC>(a, C, out, se_limit, made, sslot, se, s, sc)) {
+			if (!made || place_secondary<SC>(a, out, se_limit, sslot, pslot, se, s, sc)) {
 				s.step++;
 			} else {
 				// no room anywhere: retry the event from the same draws later
@@ -1511,8 +1516,9 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					const bool over = made && r >= nf;
 					const uint32_t sslot = wave_alloc((uint32_t*)&C->se_ctr, over);
 					s.safe = rem;
+					const uint32_t pslot = wave_alloc(&C->spill_ctr, over && sslot >= se_limit);
 					if (over)
-						done = place_secondary<SC>(a, C, out, se_limit, true, sslot, se, s, sc);
+						done = place_secondary<SC>(a, out, se_limit, sslot, pslot, se, s, sc);
 					const uint64_t csid = se_sid(s.sid, s.step);
 					const F3 cp = { __shfl(se.pos.x, src), __shfl(se.pos.y, src), __shfl(se.pos.z, src) };
 					const F3 cd = { __shfl(se.dir.x, src), __shfl(se.dir.y, src), __shfl(se.dir.z, src) };
@@ -2841,7 +2847,7 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 	// these, and more materials than LDS is to hold
 	const bool multi = d->h_worlds.size() > 1 || (d->dep && d->map.np) || a.max_mats > STEP_MATS;
 	const size_t mats = sizeof(StepMat) * a.max_mats;
-	const dim3 grid(g), block(256), sgrid((g * 4u + STEP_W - 1) / STEP_W), sblock(64 * STEP_W), cgrid(cascade_waves(d->dev)), cblock(64);
+	const dim3 grid(g), block(256), igrid((g * 256u + INEL_THREADS - 1) / INEL_THREADS), iblock(INEL_THREADS), cgrid(cascade_waves(d->dev)), cblock(64);
 	if (multi && !d->dep && !d->map.np && a.max_mats <= STEP_MATS) {
 		// several worlds, nothing but records: the launch's particles
 		// grouped by world, one world per wave
@@ -2862,28 +2868,28 @@ void launch_step_pair(nbl_driver* d, const StepArgs& a, uint32_t g)
 			hipLaunchKernelGGL(k_world_place, dim3(WG_BLOCKS), dim3(WG_THREADS), 0, d->stream, d->ctrl, d->buf[0],
 				d->buf[1], d->slots, nw, d->wgrp, d->perm);
 		hipLaunchKernelGGL((k_cascade<false, false, true>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, true>), sgrid, sblock, STEP_W * mats, d->stream, a);
-		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, true>), grid, block, 4 * mats, d->stream, a);
+		hipLaunchKernelGGL((k_inel<false, true>), igrid, iblock, 0, d->stream, a);
 	} else if (d->map.np && multi) {
 		hipLaunchKernelGGL((k_cascade<true, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<true, true>), grid, block, 0, d->stream, a);
-		hipLaunchKernelGGL((k_inel<true, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_inel<true, true>), igrid, iblock, 0, d->stream, a);
 	} else if (d->map.np) {
 		hipLaunchKernelGGL((k_cascade<true, false>), cgrid, cblock, mats, d->stream, a);
 		hipLaunchKernelGGL((k_step<true, false>), grid, block, mats + 256 * sizeof(double) * d->map.np, d->stream, a);
-		hipLaunchKernelGGL((k_inel<true, false>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_inel<true, false>), igrid, iblock, 0, d->stream, a);
 	} else if (multi) {
 		hipLaunchKernelGGL((k_cascade<false, true>), cgrid, cblock, 0, d->stream, a);
 		hipLaunchKernelGGL((k_step<false, true>), grid, block, 0, d->stream, a);
-		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_inel<false, true>), igrid, iblock, 0, d->stream, a);
 	} else if (d->dep) {
 		hipLaunchKernelGGL((k_cascade<false, false, false, true>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false, false, true>), sgrid, sblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_inel<false, true>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false, false, true>), grid, block, mats, d->stream, a);
+		hipLaunchKernelGGL((k_inel<false, true>), igrid, iblock, 0, d->stream, a);
 	} else {
 		hipLaunchKernelGGL((k_cascade<false, false>), cgrid, cblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_step<false, false>), sgrid, sblock, mats, d->stream, a);
-		hipLaunchKernelGGL((k_inel<false, false>), grid, block, 0, d->stream, a);
+		hipLaunchKernelGGL((k_step<false, false>), grid, block, mats, d->stream, a);
+		hipLaunchKernelGGL((k_inel<false, false>), igrid, iblock, 0, d->stream, a);
 	}
 }
 } // namespace
@@ -3973,8 +3979,8 @@ int nbl_track_noalloc(nbl_device* dev, const nbl_geometry* geom, const nbl_mater
 			hipLaunchKernelGGL(k_refill, dim3(g_refill), dim3(256), 0, st, ctrl, a.buf[0], a.buf[1], a.spill,
 				primaries, tags, (const uint64_t*)nullptr, (const uint16_t*)nullptr, 0u, sid_base);
 			hipLaunchKernelGGL((k_cascade<false, false>), dim3(cascade_waves(dev)), dim3(64), lds_mats, st, a);
-			hipLaunchKernelGGL((k_step<false, false>), dim3((g_step * 4u + STEP_W - 1) / STEP_W), dim3(64 * STEP_W), lds_mats, st, a);
-			hipLaunchKernelGGL((k_inel<false, false>), dim3(g_step), dim3(256), 0, st, a);
+			hipLaunchKernelGGL((k_step<false, false>), dim3(g_step), dim3(256), lds_mats, st, a);
+			hipLaunchKernelGGL((k_inel<false, false>), dim3((g_step * 256u + INEL_THREADS - 1) / INEL_THREADS), dim3(INEL_THREADS), 0, st, a);
 		}
 		HIP_OK(hipGetLastError());
 		HIP_OK(hipMemcpyAsync(&h, ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, st));
