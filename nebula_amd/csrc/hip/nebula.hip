@@ -241,7 +241,7 @@ __device__ __forceinline__ void score_barrier(ScoreLds& sc, const ScoreMap& map,
 // per wave, ranks by prefix popcount of the ballot.
 __device__ __forceinline__ uint32_t wave_alloc(uint32_t* ctr, bool want)
 {
-	const uint64_t m = __ballot(want);
+	const uint64_t m = ballot(want);
 	if (m == 0)
 		return 0;
 	const uint32_t lane = __lane_id();
@@ -258,7 +258,7 @@ __device__ __forceinline__ uint32_t wave_alloc(uint32_t* ctr, bool want)
 __device__ __forceinline__ void wave_alloc2(uint64_t* ctr, bool want_a, bool want_b, uint32_t& slot_a,
 	uint32_t& slot_b)
 {
-	const uint64_t ma = __ballot(want_a), mb = __ballot(want_b);
+	const uint64_t ma = ballot(want_a), mb = ballot(want_b);
 	slot_a = slot_b = 0;
 	if ((ma | mb) == 0)
 		return;
@@ -376,11 +376,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_world_count(const Ctrl* c, Bufs 
 		uint32_t world = 0;
 		if (valid)
 			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
-		uint64_t left = __ballot(valid);
+		uint64_t left = ballot(valid);
 		while (left) {
 			const int first = __builtin_ctzll(left);
 			const uint32_t w = __builtin_amdgcn_readlane(world, first);
-			const uint64_t m = __ballot(valid && world == w);
+			const uint64_t m = ballot(valid && world == w);
 			left &= ~m;
 			if ((int)lane == first)
 				atomicAdd(&s_h[w], (uint32_t)__popcll(m));
@@ -405,11 +405,11 @@ __global__ __launch_bounds__(256) void k_world_count_wide(const Ctrl* c, Bufs b0
 		uint32_t world = 0;
 		if (valid)
 			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
-		uint64_t left = __ballot(valid);
+		uint64_t left = ballot(valid);
 		while (left) {
 			const int first = __builtin_ctzll(left);
 			const uint32_t w = __builtin_amdgcn_readlane(world, first);
-			const uint64_t m = __ballot(valid && world == w);
+			const uint64_t m = ballot(valid && world == w);
 			left &= ~m;
 			if ((int)lane == first)
 				atomicAdd(&wg[w], (uint32_t)__popcll(m));
@@ -498,11 +498,11 @@ __global__ __launch_bounds__(WG_THREADS) void k_world_place(const Ctrl* c, Bufs 
 		uint32_t world = 0;
 		if (valid)
 			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
-		uint64_t left = __ballot(valid);
+		uint64_t left = ballot(valid);
 		while (left) {
 			const int first = __builtin_ctzll(left);
 			const uint32_t w = __builtin_amdgcn_readlane(world, first);
-			const uint64_t m = __ballot(valid && world == w);
+			const uint64_t m = ballot(valid && world == w);
 			left &= ~m;
 			uint32_t base = 0;
 			if ((int)lane == first)
@@ -532,11 +532,11 @@ __global__ __launch_bounds__(256) void k_world_place_wide(const Ctrl* c, Bufs b0
 		uint32_t world = 0;
 		if (valid)
 			world = min(flags_at(b, in_slot(i, n_surv, slots)) >> FL_WORLD_SHIFT, nw - 1u);
-		uint64_t left = __ballot(valid);
+		uint64_t left = ballot(valid);
 		while (left) {
 			const int first = __builtin_ctzll(left);
 			const uint32_t w = __builtin_amdgcn_readlane(world, first);
-			const uint64_t m = __ballot(valid && world == w);
+			const uint64_t m = ballot(valid && world == w);
 			left &= ~m;
 			uint32_t base = 0;
 			if ((int)lane == first)
@@ -792,7 +792,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 	oc = ALIVE;
 	to_inel = false;
 	bool ended = false, skip = false;
-	wave_steps += (uint32_t)__popcll(__ballot(plan && !f.planned));
+	wave_steps += (uint32_t)__popcll(ballot(plan && !f.planned));
 	if (plan) {
 		State s;
 		const float4 p = m.pos[lane], d = m.dir[lane];
@@ -829,7 +829,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 	int hit = -1;
 	float hd = 0.0f;
 	bool arrive = skip;
-	if (__ballot(f.on) != 0ull) {
+	if (ballot(f.on) != 0ull) {
 		float isect, safety;
 		int target;
 		const int r = walk_round<true>(W.g, f.on, m, f.cells, safety, isect, target);
@@ -944,7 +944,7 @@ __device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t 
 	const uint32_t wave = threadIdx.x >> 6, lane = __lane_id();
 	const bool queue = keep && to_inel;
 	bool survive = keep && !to_inel && !det;
-	const uint64_t md = __ballot(det), ms = __ballot(survive), mq = __ballot(queue);
+	const uint64_t md = ballot(det), ms = ballot(survive), mq = ballot(queue);
 	if (lane == 0) {
 		s_n[0][wave] = (uint32_t)__popcll(md);
 		s_n[1][wave] = (uint32_t)__popcll(ms);
@@ -975,7 +975,7 @@ __device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t 
 		qslot += s_n[2][w];
 	}
 	const bool over = det && dslot >= a.det_cap;
-	if (__ballot(over)) {
+	if (ballot(over)) {
 		// no record slot: wait as a survivor and retry next launch
 		uint32_t at, none;
 		wave_alloc2(&C->step_out, over, false, at, none);
@@ -1081,8 +1081,8 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		bool to_inel = (flags & FL_PEND_INEL) != 0u;
 		bool run = valid && !det && !to_inel, dead = false;
 		// K turns, and if walks are not kept, the walks to their end
-		for (uint32_t k = 0; k < K || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
-			if (__ballot(run) == 0ull)
+		for (uint32_t k = 0; k < K || (!keep_walks && ballot(f.on) != 0ull); ++k) {
+			if (ballot(run) == 0ull)
 				break;
 			int oc;
 			bool inel;
@@ -1159,7 +1159,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 		bool run = valid && !det && !to_inel, dead = false;
 		s.flags &= ~(FL_PEND_INEL | FL_PLANNED | FL_WALK);
 		for (uint32_t k = 0; k < K; ++k) {
-			if (__ballot(run) == 0ull)
+			if (ballot(run) == 0ull)
 				break;
 			int oc = ALIVE;
 			bool walk = false;
@@ -1309,8 +1309,8 @@ __global__ __launch_bounds__(INEL_THREADS) void k_inel(StepArgs a)
 				doa = true;
 			}
 		}
-		const uint64_t m = __ballot(made);
-		const uint64_t md = __ballot(doa);
+		const uint64_t m = ballot(made);
+		const uint64_t md = ballot(doa);
 		if (__lane_id() == 0) {
 			s_cnt[wave] = (uint32_t)__popcll(m);
 			s_doa[wave] = (uint32_t)__popcll(md);
@@ -1437,7 +1437,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		const bool have = lane < g && i < n_loop;
 		const uint32_t li = (WUNI && !ident) ? (have ? a.perm[i] : ~0u) : i;
 		bool occ = have && li != ~0u;   // this lane holds a particle
-		const uint64_t first = __ballot(occ);
+		const uint64_t first = ballot(occ);
 		if (first == 0ull)
 			continue;
 		const int hold = (int)min(64u, (uint32_t)__popcll(first) + extra);
@@ -1471,8 +1471,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		s.flags &= FL_WORLD_MASK;
 		float rem = MULTI ? -1.0f : s.safe;
 		// n_steps turns, and if walks are not kept, the walks to their end
-		for (uint32_t k = 0; k < n_steps || (!keep_walks && __ballot(f.on) != 0ull); ++k) {
-			const uint64_t live = __ballot(occ && !park);
+		for (uint32_t k = 0; k < n_steps || (!keep_walks && ballot(f.on) != 0ull); ++k) {
+			const uint64_t live = ballot(occ && !park);
 			if (live == 0ull)
 				break;
 			// every wave writes at most 64 deposits a step: stop while all of
@@ -1480,7 +1480,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			if (((MULTI && a.dep) || DEP) && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 					+ 64ull * waves > a.dep_cap / 2u)
 				break;
-			if (k < n_steps && pend_share * __popcll(__ballot(pend)) >= __popcll(live)) {
+			if (k < n_steps && pend_share * __popcll(ballot(pend)) >= __popcll(live)) {
 				Particle se = {};
 				Particle pre = {};
 				bool made = false;
@@ -1499,10 +1499,10 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						++my_steps;
 					}
 				}
-				const uint64_t mm = __ballot(made);
+				const uint64_t mm = ballot(made);
 				bool done = true;
 				if (mm) {
-					const uint64_t mf = __ballot(!occ);
+					const uint64_t mf = ballot(!occ);
 					// lanes that may be filled
 					const int nm = (int)__popcll(mm), nf = max(0, hold - 64 + (int)__popcll(mf));
 					const int r = (int)__popcll(mm & below), rf = (int)__popcll(mf & below);
@@ -1571,7 +1571,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					put_state(m, lane, s);
 			}
 			const bool run = occ && !pend && !park && !det;
-			if (__ballot(run) != 0ull) {
+			if (ballot(run) != 0ull) {
 				int oc = ALIVE;
 				bool ended = run;
 				if constexpr (MULTI) {
@@ -1632,7 +1632,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 				}
 			}
 			const bool rec = det && !park;
-			if (__ballot(rec)) {
+			if (ballot(rec)) {
 				const uint32_t dslot = wave_alloc(&C->det_ctr, rec);
 				if (rec) {
 					if (!MULTI)

@@ -42,6 +42,10 @@ constexpr uint32_t FL_WORLD_SHIFT = 16u, FL_WORLD_MASK = 0xffff0000u;
 
 struct F3 { float x, y, z; };
 
+// Lanes with p set.  (HIP's __ballot takes an int: a select and a compare more
+// where p is not a compare's result.)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
 // ------------------------------------------------------------------ math --
 // Float transcendentals built from IEEE float +, -, *, / and integer bit
 // operations only, so that (compiled without FMA contraction) they give the
@@ -1044,7 +1048,7 @@ __device__ __forceinline__ int wave_incl_sum(int v)
 // DPP (as in wave_incl_sum) carries each mark on to the next one.
 __device__ __forceinline__ int chunk_owner(int base, int excl, int n, int* owner_at, int lane)
 {
-	const uint64_t before = __ballot(excl <= base);
+	const uint64_t before = ballot(excl <= base);
 	const int o0 = 63 - (int)__builtin_clzll(before);
 	owner_at[lane] = 0;
 	__builtin_amdgcn_wave_barrier();
@@ -1169,7 +1173,7 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, WaveMe
 			t = intersect_ray(load_tri(g.tris, ti), xyz(m.cur[own]), xyz(m.dir[own]));
 		}
 		__builtin_amdgcn_wave_barrier();
-		uint64_t hits = __ballot(t > 0.0f);
+		uint64_t hits = ballot(t > 0.0f);
 		while (hits) {
 			const int src = (int)__builtin_ctzll(hits);
 			hits &= hits - 1ull;
@@ -1194,7 +1198,7 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, WaveMe
 		const bool pass = valid && ti != ol.x && cell_may_hit(sc, xyz(od), __float_as_int(od.w), oc.w);
 		if (SAF && valid)
 			atomicMin(&m.saf[o], __float_as_uint(fmaxf(pair_safety(sc), 0.0f)));
-		const uint64_t pm = __ballot(pass);
+		const uint64_t pm = ballot(pass);
 		const int np = (int)__popcll(pm);
 		if (qn + np > 64) {
 			flush();
@@ -1241,7 +1245,7 @@ __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 
 		m.cell[lane] = cell_start(g, start);
 	out_dist = distance;
 	int result = -1;
-	while (__ballot(walk) != 0ull) {
+	while (ballot(walk) != 0ull) {
 		float isect, safety;
 		int target;
 		const int r = walk_round<false>(g, walk, m, cells, safety, isect, target);
@@ -1270,7 +1274,7 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 		walk_start(g, w, start, distance);
 	int result = -1;
 	bool active = walk;
-	while (__ballot(active) != 0ull) {
+	while (ballot(active) != 0ull) {
 		int n = 0, off = 0, target = 0;
 		float isect = 0.0f;
 		if (active) {
@@ -1302,7 +1306,7 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 			}
 			// this lane's pairs within the chunk, lanes [lo, hi)
 			uint64_t todo = 0;
-			const uint64_t can_hit = __ballot(t > 0.0f);
+			const uint64_t can_hit = ballot(t > 0.0f);
 			if (active) {
 				const int lo = max(excl - base, 0), hi = min(incl - base, 64);
 				if (lo < hi) {
@@ -1310,7 +1314,7 @@ __device__ inline int propagate_wave_multi(const Geometry& g, bool walk, F3 star
 					todo = can_hit & upto & ~((1ull << lo) - 1ull);
 				}
 			}
-			while (__ballot(todo != 0ull) != 0ull) {
+			while (ballot(todo != 0ull) != 0ull) {
 				const int src = todo ? (int)__builtin_ctzll(todo) : lane;
 				const float ts = __shfl(t, src);
 				const int tis = __shfl(ti, src);
