@@ -1916,6 +1916,9 @@ struct nbl_geometry {
 	int max_material;   // largest physical material index named by a triangle
 };
 
+// Bytes of score arrays that a driver keeps while scores are off.
+constexpr size_t SCORES_KEPT = (size_t)2 << 30;
+
 struct nbl_material {
 	nbl_device* dev;
 	float* tables[9];   // the seven of the host's, and those of StepMat
@@ -1952,8 +1955,11 @@ struct nbl_driver {
 	uint32_t* perm;         // world grouping: the step launch's indices by world
 	uint32_t next_tag;
 	ScoreMap map;           // map.np == 0: no scores
-	double* sc_mem[4];      // score arrays of buf[0], buf[1], spill, inel
+	// score arrays of buf[0], buf[1], spill, inel, and of the records (det_sc),
+	// and their sizes in words; kept while scores are off, up to SCORES_KEPT
+	double* sc_mem[4];
 	double* det_sc;
+	size_t sc_words[5];
 	std::vector<Material> h_mats;   // host copy of d_mats
 	uint32_t blocks_per_cu = 64;    // k_step grid: blocks of 256 per compute unit
 	uint32_t target = 0;            // particles in flight to aim for
@@ -3269,6 +3275,7 @@ int grow_spill(nbl_driver* d)
 	if (d->map.np) {
 		d->spill.sc = nsc;
 		d->sc_mem[2] = nsc;
+		d->sc_words[2] = (size_t)d->map.np * ncap;
 	}
 	d->spill_cap = ncap;
 	d->spill_growths++;
@@ -3651,22 +3658,42 @@ int nbl_driver_set_score_params(nbl_driver* d, const int32_t* materials, const i
 	if (active_count(*d->h_ctrl, d->spill_cap) != 0 || d->h_ctrl->queue_n != d->h_ctrl->queue_next ||
 		d->h_ctrl->det_ctr != 0)
 		return fail(NBL_ERR_ARG, "scores can only be switched while no particle is in flight or detected");
-	for (double*& p : d->sc_mem) { hipFree(p); p = nullptr; }
-	hipFree(d->det_sc);
-	d->det_sc = nullptr;
 	Bufs* bufs[4] = { &d->buf[0], &d->buf[1], &d->spill, &d->inel };
 	for (Bufs* b : bufs)
 		b->sc = nullptr;
 	d->map.np = 0;
 	d->epoch++;
-	if (n == 0)
+	// A Jacobian switches scores on and off again: allocating their gigabyte
+	// (2^20 particles, 5 parameters) each time took 2 of 36 ms.
+	size_t total = 0;
+	for (size_t w : d->sc_words)
+		total += sizeof(double) * w;
+	auto resize = [&](int k, size_t words) -> int {
+		double*& p = k < 4 ? d->sc_mem[k] : d->det_sc;
+		if (d->sc_words[k] >= words && words)
+			return NBL_OK;
+		hipFree(p);
+		p = nullptr;
+		d->sc_words[k] = 0;
+		if (!words)
+			return NBL_OK;
+		const int e = dev_alloc(&p, words);
+		if (e == NBL_OK)
+			d->sc_words[k] = words;
+		return e;
+	};
+	if (n == 0) {
+		if (total > SCORES_KEPT)
+			for (int k = 0; k < 5; ++k)
+				resize(k, 0);
 		return NBL_OK;
+	}
 	for (int k = 0; k < 4; ++k) {
-		if ((rc = dev_alloc(&d->sc_mem[k], (size_t)n * bufs[k]->sc_stride)))
+		if ((rc = resize(k, (size_t)n * bufs[k]->sc_stride)))
 			return rc;
 		bufs[k]->sc = d->sc_mem[k];
 	}
-	if ((rc = dev_alloc(&d->det_sc, (size_t)n * d->det_cap)))
+	if ((rc = resize(4, (size_t)n * d->det_cap)))
 		return rc;
 	d->map = map;
 	return NBL_OK;
