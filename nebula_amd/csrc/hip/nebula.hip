@@ -1932,12 +1932,11 @@ struct nbl_driver {
 	Material* d_mats;
 	uint32_t capacity, slots, K, det_cap;
 	Bufs buf[2];
-	void* buf_mem[2];
+	void* buf_mem;          // of buf, inel and walk
 	Bufs spill;
 	void* spill_mem;
 	uint32_t spill_cap;
 	Bufs inel;
-	void* inel_mem;
 	char* walk[2];          // unfinished walks of the particles of buf[0] and buf[1], or null
 	Ctrl* ctrl;
 	Ctrl* h_ctrl;
@@ -2571,14 +2570,10 @@ int nbl_driver_destroy(nbl_driver* d)
 	hipStreamSynchronize(d->stream);
 	for (auto& pr : d->ev_used) { hipEventDestroy(pr.first); hipEventDestroy(pr.second); }
 	for (auto& pr : d->ev_free) { hipEventDestroy(pr.first); hipEventDestroy(pr.second); }
-	hipFree(d->buf_mem[0]);
-	hipFree(d->buf_mem[1]);
+	hipFree(d->buf_mem);
 	hipFree(d->spill_mem);
-	hipFree(d->inel_mem);
 	hipFree(d->tally_bin);
 	hipFree(d->tally_counts);
-	hipFree(d->walk[0]);
-	hipFree(d->walk[1]);
 	hipFree(d->ctrl);
 	hipHostFree(d->h_ctrl);
 	hipHostFree(d->h_stage);
@@ -2637,8 +2632,27 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 		delete d;
 		return fail(NBL_ERR_DEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(e));
 	}
-	if ((rc = alloc_bufs(d->buf[0], d->buf_mem[0], d->slots))) return cleanup(rc);
-	if ((rc = alloc_bufs(d->buf[1], d->buf_mem[1], d->slots))) return cleanup(rc);
+	// The two particle buffers, the inelastic queue and the unfinished walks in
+	// one allocation (an allocation costs by the call and by the byte, and a
+	// program may make a driver per scan).  Walks take 24 bytes a slot and
+	// buffer, where a launch may have enough particles to leave some.  Very large
+	// drivers (over 3.2 GB of them) go without: their launches finish every walk.
+	{
+		const size_t b = tile_bytes(d->slots);
+		const bool walks = d->slots >= KEEP_WALKS_MIN && d->slots <= 1u << 26;
+		const size_t w = walks ? WALK_TILE * ((d->slots + 63) / 64) : 0;
+		char* p = nullptr;
+		if (hipMalloc((void**)&p, 3 * b + 2 * w) != hipSuccess)
+			return cleanup(fail(NBL_ERR_ALLOC, "hipMalloc of the particle buffers failed"));
+		d->buf_mem = p;
+		d->buf[0] = { p, nullptr, d->slots };
+		d->buf[1] = { p + b, nullptr, d->slots };
+		d->inel = { p + 2 * b, nullptr, d->slots };
+		if (walks) {
+			d->walk[0] = p + 3 * b;
+			d->walk[1] = p + 3 * b + w;
+		}
+	}
 	// The spill stack starts at eight buffers' worth (60 bytes a slot: 2 GB
 	// at 2^22 slots) and doubles when needed.  A scan of 300 eV primaries
 	// filling 2^22 slots spills more than twice the buffer in its first
@@ -2646,13 +2660,6 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 	// stream idle.
 	d->spill_cap = std::max<uint32_t>(1024u, std::min<uint64_t>(8ull * d->slots, 1ull << 28));
 	if ((rc = alloc_bufs(d->spill, d->spill_mem, d->spill_cap))) return cleanup(rc);
-	if ((rc = alloc_bufs(d->inel, d->inel_mem, d->slots))) return cleanup(rc);
-	// Unfinished walks, 24 bytes a slot and buffer, where a launch may have
-	// enough particles to leave some.  Very large drivers (over 3.2 GB of them)
-	// go without: their launches finish every walk.
-	if (d->slots >= KEEP_WALKS_MIN && d->slots <= 1u << 26)
-		for (char*& w : d->walk)
-			if ((rc = dev_alloc(&w, WALK_TILE * ((d->slots + 63) / 64)))) return cleanup(rc);
 	if ((rc = dev_alloc(&d->ctrl, 1))) return cleanup(rc);
 	if (hipHostMalloc((void**)&d->h_ctrl, sizeof(Ctrl), hipHostMallocDefault) != hipSuccess)
 		return cleanup(fail(NBL_ERR_ALLOC, "hipHostMalloc failed"));
