@@ -6,9 +6,9 @@
 // survivors of the previous launch occupy [0, n_surv) and secondary electrons
 // [slots - n_se, slots).  A launch of k_step moves every particle through up
 // to K steps (init + event each), then appends it to the other buffer:
-// survivors from the front (a wavefront ballot + prefix popcount + one
-// atomic per wave), new secondaries from the back (made by k_inel, one
-// atomic per block).  Dead particles
+// survivors from the front (wavefront ballots + prefix popcounts; one atomic
+// per block, per wave in the general variant), new secondaries from the back (made by k_inel, one atomic per
+// block).  Dead particles
 // are simply not copied, so the next launch reads a dense range.  A
 // one-thread control kernel adopts the output counts and plans the refill of
 // primaries from a device-resident queue; all sizes live in device memory, so
@@ -1993,7 +1993,7 @@ namespace {
 
 // Waves of a k_cascade launch, and the particles in flight up to which a
 // launch is k_cascade's.
-// 16 waves a compute unit are all resident (118 VGPRs); up to 1024 particles
+// 16 waves a compute unit are all resident (at most 125 VGPRs); up to 1024 particles
 // a compute unit they hold every particle (512: 13.3 against 12.9 ms for
 // 96 903 primaries of 500 eV on a grating, 27.0 against 25.8 ms for 160 000
 // of 1 keV on contact holes; 1536, waves taking two turns: 13.7 and 26.0).
