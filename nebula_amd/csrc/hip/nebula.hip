@@ -668,6 +668,55 @@ __device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, co
 	}
 }
 
+// Records of a wave of k_cascade, gathered in LDS and written together: 2048
+// primaries of 1 keV make 3.4 M records, and with an atomic and a look at the
+// counter each turn their launches waited for that one address (23.0 ms of
+// k_cascade, now 3.4).
+struct DepStage {
+	nbl_deposit* at;   // 64 records
+	uint32_t n;
+	bool full;         // the counter has passed the launch's limit
+};
+
+// All lanes together.  `full` leaves 64 records for each of the launch's waves.
+__device__ __forceinline__ void flush_deposits(const StepArgs& a, Ctrl* C, DepStage& st, uint32_t waves)
+{
+	if (st.n == 0u)
+		return;
+	const uint32_t lane = __lane_id();
+	uint32_t base = 0;
+	if (lane == 0u)
+		base = atomicAdd(&C->dep_ctr, st.n);
+	base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+	__builtin_amdgcn_wave_barrier();
+	if (lane < st.n && base + lane < a.dep_cap)
+		a.dep[base + lane] = st.at[lane];
+	__builtin_amdgcn_wave_barrier();
+	st.full = (uint64_t)base + st.n + 64ull * waves > a.dep_cap / 2u;
+	st.n = 0;
+}
+
+__device__ __forceinline__ void stage_deposit(const StepArgs& a, Ctrl* C, DepStage& st, uint32_t waves, bool rec,
+	const F3& pos, float E, uint32_t tag, uint64_t sid, float e0)
+{
+	const uint64_t m = ballot(rec);
+	if (m == 0ull)
+		return;
+	const uint32_t c = (uint32_t)__popcll(m);
+	if (st.n + c > 64u)
+		flush_deposits(a, C, st, waves);
+	if (rec) {
+		nbl_deposit r;
+		r.pos[0] = pos.x; r.pos[1] = pos.y; r.pos[2] = pos.z;
+		r.energy = e0;
+		r.deposit = e0 - E;
+		r.tag = tag;
+		r.sid = sid;
+		st.at[st.n + (uint32_t)__popcll(m & ((1ull << __lane_id()) - 1ull))] = r;
+	}
+	st.n += c;
+}
+
 // WUNI: several worlds, one per wave.  A wave steps the particles of its
 // first lane's world (its geometry and materials are wave-uniform, so the
 // plain kernel's shared walk, walk skip and register budget apply); lanes
@@ -782,15 +831,18 @@ __device__ __forceinline__ uint32_t keep_walk(const StepArgs& a, uint32_t buf, u
 // Returns true in lanes whose step has ended: `oc` ALIVE (with `to_inel`: an
 // inelastic event is to follow), DETECTED or TERMINATED.
 //
-// DEP: energy-deposit records of the elastic events, under `tag`.
+// DEP: `dep_e0` is the energy before an elastic event that deposits some (its
+// record is the caller's: this runs in a part of the wave), 0 without one.
 template <bool SC, bool DEP>
 __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, const StepMat* mats, bool plan,
-	WaveMem& m, uint32_t tag,
+	WaveMem& m, float& dep_e0,
 	InFlight& f, float& rem, ScoreLds& sc, uint32_t& wave_steps, int& oc, bool& to_inel)
 {
 	const uint32_t lane = __lane_id();
 	oc = ALIVE;
 	to_inel = false;
+	if (DEP)
+		dep_e0 = 0.0f;
 	bool ended = false, skip = false;
 	wave_steps += (uint32_t)__popcll(ballot(plan && !f.planned));
 	if (plan) {
@@ -878,8 +930,8 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 			} else {
 				oc = step_event_elastic_or_boundary(W, mats, s, rng, ev, hit, e.y);
 			}
-			if (DEP)
-				deposit(a, a.ctrl, ev == EV_ELASTIC && s.p.E != e0, s.p, tag, m.sid[lane], e0);
+			if (DEP && ev == EV_ELASTIC && s.p.E != e0)
+				dep_e0 = e0;
 		}
 		m.pos[lane] = { s.p.pos.x, s.p.pos.y, s.p.pos.z, s.p.E };
 		m.dir[lane] = { s.p.dir.x, s.p.dir.y, s.p.dir.z, __int_as_float(s.mat) };
@@ -1086,8 +1138,16 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 				break;
 			int oc;
 			bool inel;
-			const bool ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < K, m, DEP ? tag : 0u, f, rem, sc, wave_steps,
+			float dep_e0;
+			const bool ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < K, m, dep_e0, f, rem, sc, wave_steps,
 				oc, inel);
+			if (DEP) {
+				Particle q;
+				const float4 at = m.pos[lane];
+				q.pos = xyz(at);
+				q.E = at.w;
+				deposit(a, C, dep_e0 != 0.0f, q, tag, m.sid[lane], dep_e0);
+			}
 			if (ended) {
 				if (oc == DETECTED) {
 					det = true;
@@ -1401,6 +1461,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 	StepMat* const mats = (StepMat*)s_dyn;
 	if (!MULTI && !WUNI && lane < (uint32_t)W.nmats)
 		load_step_mat(mats[lane], W.mats[lane]);
+	__shared__ nbl_deposit s_dep[DEP ? 64 : 1];
+	DepStage st = { s_dep, 0u, false };
 	const uint64_t below = (1ull << lane) - 1ull;
 	const bool ident = WUNI && a.perm_n[1] != 0u;
 	const uint32_t n_loop = (WUNI && !ident) ? *a.perm_n : n_in;
@@ -1475,9 +1537,20 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			const uint64_t live = ballot(occ && !park);
 			if (live == 0ull)
 				break;
-			// every wave writes at most 64 deposits a step: stop while all of
-			// them still have room in the first half of the buffer
-			if (((MULTI && a.dep) || DEP) && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+			// stop while every wave still has room for 64 records in the first
+			// half of the buffer; what a turn writes beyond them (a particle
+			// can have two events in it) fits the second half
+			// (one world: a wave gathers up to 64 records and learns the
+			// counter's value when it writes them.  It does so before a turn
+			// that may not fit, so once the limit is passed it writes 64
+			// records at most, or those of one turn if it had none.)
+			if (DEP) {
+				if (st.n + 3u * (uint32_t)__popcll(live) > 64u)
+					flush_deposits(a, C, st, waves);
+				if (st.full)
+					break;
+			}
+			if (MULTI && a.dep && (uint64_t)__hip_atomic_load(&C->dep_ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 					+ 64ull * waves > a.dep_cap / 2u)
 				break;
 			if (k < n_steps && pend_share * __popcll(ballot(pend)) >= __popcll(live)) {
@@ -1554,8 +1627,10 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 						occ = true;
 					}
 				}
-				if ((MULTI && a.dep) || DEP)
+				if (MULTI && a.dep)
 					deposit(a, C, pend && done && s.p.E != pre.E, s.p, s.tag, s.sid, pre.E);
+				if (DEP)
+					stage_deposit(a, C, st, waves, pend && done && s.p.E != pre.E, s.p.pos, s.p.E, s.tag, s.sid, pre.E);
 				if (pend) {
 					if (done) {
 						s.step++;
@@ -1617,7 +1692,12 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					}
 				} else {
 					bool inel;
-					ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < n_steps, m, s.tag, f, rem, sc, wave_steps, oc, inel);
+					float dep_e0;
+					ended = step_turn<SC, DEP>(a, W, mats, run && !f.on && k < n_steps, m, dep_e0, f, rem, sc, wave_steps, oc, inel);
+					if (DEP) {
+						const float4 q = m.pos[lane];
+						stage_deposit(a, C, st, waves, dep_e0 != 0.0f, xyz(q), q.w, s.tag, m.sid[lane], dep_e0);
+					}
 					pend = pend || (ended && inel);
 				}
 				if (ended) {
@@ -1668,6 +1748,8 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			if (SC) store_score(out, oslot, np, sc);
 		}
 	}
+	if (DEP)
+		flush_deposits(a, C, st, waves);
 	count_steps(C, my_steps + ((lane == 0) ? wave_steps : 0u));
 }
 
