@@ -308,7 +308,8 @@ int nbl_driver_tally_begin(nbl_driver* d, const int64_t* tag_bin, uint64_t n_tag
 int nbl_driver_tally(nbl_driver* d, double se_cutoff);
 int nbl_driver_tally_read(nbl_driver* d, int64_t* counts, uint32_t* bad);
 
-/* Total particle-steps taken so far (init calls on active particles). */
+/* Total particle-steps taken so far (init calls on active particles; a step
+ * that a launch left on its walk counts when it ends). */
 int nbl_driver_steps(nbl_driver* d, uint64_t* steps);
 
 /* Run until every pushed primary and its cascade has finished, draining

@@ -138,9 +138,12 @@ struct StepArgs {
 	uint32_t same_grid;     // every material has its two mean free path tables as one (imfp2)
 };
 constexpr size_t WALK_TILE = 64 * (16 + 8);
-// Particles in flight from which a launch leaves walks unfinished: with so
-// many some steps end in every launch, which the callers' checks for a run
-// that makes no progress count on.
+// Particles in flight from which a launch leaves walks unfinished (drivers
+// with room for fewer have no memory for walks).  However many: a wave with
+// walks under way goes on until one of its steps has ended, and a step is
+// counted when it ends, so the count of steps rises with every launch that has
+// a particle to move.  The callers' checks for a run without progress rest on
+// that: electrons that start in one point all cross the same cells together.
 constexpr uint32_t KEEP_WALKS_MIN = 65536;
 
 __device__ __forceinline__ State load_state(const Bufs& b, uint32_t i)
@@ -844,7 +847,6 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 	if (DEP)
 		dep_e0 = 0.0f;
 	bool ended = false, skip = false;
-	wave_steps += (uint32_t)__popcll(ballot(plan && !f.planned));
 	if (plan) {
 		State s;
 		const float4 p = m.pos[lane], d = m.dir[lane];
@@ -938,6 +940,7 @@ __device__ __forceinline__ bool step_turn(const StepArgs& a, const World& W, con
 		m.last[lane].x = s.last_tri;
 	}
 	lds_again();
+	wave_steps += (uint32_t)__popcll(ballot(ended));
 	return ended;
 }
 
@@ -1132,8 +1135,9 @@ __device__ __forceinline__ void step_body(const StepArgs& a)
 		// an inelastic event that found no secondary slot earlier
 		bool to_inel = (flags & FL_PEND_INEL) != 0u;
 		bool run = valid && !det && !to_inel, dead = false;
-		// K turns, and if walks are not kept, the walks to their end
-		for (uint32_t k = 0; k < K || (!keep_walks && ballot(f.on) != 0ull); ++k) {
+		// K turns, and the walks to their end if they are not kept, or until a
+		// step has ended
+		for (uint32_t k = 0; k < K || ((!keep_walks || wave_steps == 0u) && ballot(f.on) != 0ull); ++k) {
 			if (ballot(run) == 0ull)
 				break;
 			int oc;
@@ -1231,8 +1235,7 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 			if (run) {
 				rng = step_draws(W.key0, W.key1, s.sid, s.step);
 				oc = step_plan(W, W.mats, s, rng, nd, distance, type, pinfo, planned);
-				if (!planned)
-					++my_steps;
+				++my_steps;
 				planned = false;
 				walk = (oc == ALIVE);
 			}
@@ -1532,8 +1535,10 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 		bool park = false;                            // waits for the next launch
 		s.flags &= FL_WORLD_MASK;
 		float rem = MULTI ? -1.0f : s.safe;
-		// n_steps turns, and if walks are not kept, the walks to their end
-		for (uint32_t k = 0; k < n_steps || (!keep_walks && ballot(f.on) != 0ull); ++k) {
+		// n_steps turns, and the walks to their end if they are not kept, or
+		// until a step has ended
+		const uint32_t steps0 = wave_steps;
+		for (uint32_t k = 0; k < n_steps || ((!keep_walks || wave_steps == steps0) && ballot(f.on) != 0ull); ++k) {
 			const uint64_t live = ballot(occ && !park);
 			if (live == 0ull)
 				break;
@@ -1660,8 +1665,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 					if (run) {
 						rng = step_draws(W.key0, W.key1, s.sid, s.step);
 						oc = step_plan(W, W.mats, s, rng, nd, distance, type, pinfo, f.planned);
-						if (!f.planned)
-							++my_steps;
+						++my_steps;
 						f.planned = false;
 						walk = (oc == ALIVE);
 					}
