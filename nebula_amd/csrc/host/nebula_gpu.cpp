@@ -500,7 +500,11 @@ int run(int argc, char** argv)
 
 	// ----------------------------------------------------------- prescan
 	// Prescan primaries are real work; their detections are written first.
+	// It measures launches of steps_per_launch steps (without set_cascade, a
+	// few launches would take its electrons to their end, and frame_size
+	// would be 1).
 	timer.start();
+	check(nbl_driver_set_cascade(drv, 0), "set_cascade");
 	const uint32_t n_prescan = (uint32_t)std::min<size_t>(prescan_size, N);
 	std::vector<std::pair<uint32_t, uint32_t>> stats;
 	{
@@ -526,6 +530,7 @@ int run(int argc, char** argv)
 		if (stalled >= 64)
 			throw Failure("prescan makes no progress: raise --capacity");
 	}
+	check(nbl_driver_set_cascade(drv, UINT32_MAX), "set_cascade");
 	timer.stop("Prescan");
 	const uint32_t frame_size = 1 + (uint32_t)std::distance(stats.begin(),
 		std::max_element(stats.begin(), stats.end(),

@@ -110,3 +110,35 @@ def test_cli_energy_deposits_equal_oracle(tmp_path):
     assert len(got_dep) > 1000 and len(got_dep) == len(exp_dep)
     assert np.array_equal(_as_sorted_bytes(got_dep), _as_sorted_bytes(exp_dep))
     assert np.array_equal(_as_sorted_bytes(got_det), _as_sorted_bytes(exp_det))
+
+
+@pytest.mark.parametrize("prescan,steps", [(1000, 4), (1000, 6), (50, 4)])
+def test_cli_prescan_follows_the_population(tmp_path, prescan, steps):
+    """The frame size is the number of launches, of `steps` steps a particle,
+    after which the prescan has most particles in flight."""
+    mesh = W.grating_geometry(dy=3.2)
+    pri = W.raster_scan(16, 16, 8, 300.0, -48.0, 48.0, -48.0, 48.0, 37.0, seed=5)
+    W.write_tri(str(tmp_path / "g.tri"), mesh)
+    W.write_pri(str(tmp_path / "s.pri"), pri)
+    A.write_mat_file(str(tmp_path / "si.mat"), material("si"))
+    A.write_mat_file(str(tmp_path / "pmma.mat"), material("pmma"))
+    print(prescan, steps, flush=True)
+    r = subprocess.run([CLI, "--capacity", "65536", "--prescan-size", str(prescan), "--steps-per-launch", str(steps),
+                        "--seed", "7", str(tmp_path / "g.tri"), str(tmp_path / "s.pri"), str(tmp_path / "si.mat"),
+                        str(tmp_path / "pmma.mat")], capture_output=True, timeout=100)
+    err = r.stderr.decode()
+    assert r.returncode == 0, err[-2000:]
+    got = int(err.split("frame_size = ")[1].split()[0])
+    dev = A.Device(0)
+    mats = [A.Material(dev, A.HostMaterial(material(m))) for m in ("si", "pmma")]
+    d = A.Driver(dev, 65536, A.Geometry(dev, mesh), mats, seed=_mt_first(7), steps_per_launch=steps)
+    d.set_cascade(0)
+    d.push(A.prescan_shuffle(pri, prescan)[:prescan])
+    flying = [prescan]
+    while flying[-1] > 0:
+        d.do_iteration(1)
+        running, _, queued = d.counts()
+        flying.append(running + queued)
+    print(got, flying, flush=True)
+    assert got == 1 + int(np.argmax(flying)) > 1
+    d.close()
