@@ -3465,20 +3465,21 @@ int nbl_driver_tally_begin(nbl_driver* d, const int64_t* tag_bin, uint64_t n_tag
 			return rc;
 		d->tally_tags_cap = n_tags;
 	}
-	if (!d->tally_counts || n_bins > d->tally_bins_cap) {
+	// no bins: room for one, so that there is something to clear and to name
+	const uint64_t bins = std::max<uint64_t>(1, n_bins);
+	if (bins > d->tally_bins_cap) {
 		hipFree(d->tally_counts);
 		d->tally_counts = nullptr;
 		d->tally_bins_cap = 0;
-		if ((rc = dev_alloc(&d->tally_counts, 2 * n_bins)))
+		if ((rc = dev_alloc(&d->tally_counts, 2 * bins)))
 			return rc;
-		d->tally_bins_cap = n_bins;
+		d->tally_bins_cap = bins;
 	}
 	// by the null stream, which the driver's own does not wait for: a frame
 	// enqueued before goes on meanwhile
 	if (n_tags)
 		HIP_OK(hipMemcpy(d->tally_bin, tag_bin, sizeof(int64_t) * n_tags, hipMemcpyHostToDevice));
-	HIP_OK(hipMemsetAsync(d->tally_counts, 0, sizeof(unsigned long long) * 2 * std::max<uint64_t>(1, n_bins),
-		d->stream));
+	HIP_OK(hipMemsetAsync(d->tally_counts, 0, sizeof(unsigned long long) * 2 * bins, d->stream));
 	HIP_OK(hipMemsetAsync(&d->ctrl->tally_bad, 0, sizeof(uint32_t), d->stream));
 	d->tally_tags = n_tags;
 	d->tally_bins = n_bins;

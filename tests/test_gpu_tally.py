@@ -65,3 +65,24 @@ def test_tally_refuses_records_without_a_bin(setup, what, error):
     d.flush_detected()
     d.push(pri, tags)
     assert d.run_tally(np.zeros(N, np.int64), 1).sum() == len(rec)
+
+
+def test_tally_of_no_bins():
+    """No bins are enough for a beam of which nothing is detected (on a new
+    driver, whose tally has no memory yet); a detected record has none."""
+    dev = A.Device(0)
+    mats = [A.Material(dev, A.HostMaterial(material(m))) for m in ("si", "pmma")]
+    d = A.Driver(dev, 4096, A.Geometry(dev, grating_tris()), mats, seed=4)
+    pri = W.raster_scan(50, 1, 1, 400.0, -60.0, 60.0, -60.0, 60.0, 37.0, seed=2)
+    tags = np.arange(len(pri), dtype=np.uint32)
+    out = pri.copy()
+    out["pos"][:, 2] = 1e6             # outside the domain: ended by their first step
+    for _ in range(2):
+        d.push(out, tags)
+        assert d.run_tally(np.zeros(len(pri), np.int64), 0).shape == (0, 2)
+    d.push(pri, tags)
+    with pytest.raises(ValueError):
+        d.run_tally(np.zeros(len(pri), np.int64), 0)
+    d.push(pri, tags)
+    assert d.run_tally(np.zeros(len(pri), np.int64), 1).sum() > 0
+    d.close()
