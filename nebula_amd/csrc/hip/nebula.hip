@@ -3142,10 +3142,15 @@ int nbl_driver_autotune(nbl_driver* d, uint32_t iters_per_trial, nbl_tune_result
 	const bool graph = d->use_graph, timing = d->timing;
 	const double step_ms0 = d->step_ms;
 	const uint64_t launches0 = d->step_launches;
+	// neither the steps per launch nor the grid matter to k_cascade, which
+	// would take the trials with few particles
+	const uint32_t few = d->few;
+	d->few = 0;
 	d->use_graph = false;
 	d->timing = true;
 	// the caller's timing totals do not include the trials
 	auto restore = [&]() {
+		d->few = few;
 		d->use_graph = graph;
 		d->timing = timing;
 		d->step_ms = step_ms0;

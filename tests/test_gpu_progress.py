@@ -52,3 +52,19 @@ def test_a_first_flight_of_many_cells_is_progress(world, x, y, tally):
         assert _equal(np.concatenate(rec), ref)
     assert d.steps() == steps
     d.close()
+
+
+def test_the_tuner_measures_short_launches(world):
+    """All electrons fly after the first trial, which ends the search: two
+    trials of one launch of four steps."""
+    dev, mats, geom, oracle = world
+    n = 3000
+    pri = W.raster_scan(n, 1, 1, 300.0, -60.0, 60.0, -60.0, 60.0, 37.0, seed=3)
+    d = A.Driver(dev, 4096, geom, mats, seed=9, steps_per_launch=4)
+    d.push(pri, np.arange(n, dtype=np.uint32))
+    assert d.autotune(iters_per_trial=1)["trials"] == 2
+    assert n <= d.steps() <= 2 * 4 * d.info()["slots"]
+    det = d.run(40 * n)
+    ref, steps = oracle.run_philox(pri, 9, 40 * n, threads=8)
+    assert _equal(det, ref) and d.steps() == steps
+    d.close()
