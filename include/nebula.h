@@ -272,6 +272,11 @@ int nbl_driver_set_launch(nbl_driver* d, uint32_t steps_per_launch, uint32_t blo
  * compute unit; 0: never).  Results do not depend on it. */
 int nbl_driver_set_cascade(nbl_driver* d, uint32_t max_particles);
 
+/* The limit that holds for nbl_driver_iterate(d, n > 1): the one set, or 0
+ * while deposits are on (there only single iterations on a drained buffer
+ * run so).  Frames of many iterations are worth their length above it. */
+int nbl_driver_get_cascade(nbl_driver* d, uint32_t* max_particles);
+
 /* Replay each nbl_driver_iterate(d, n > 1) from a captured hipGraph of n
  * iterations (captured once per n and launch configuration). */
 int nbl_driver_set_graph(nbl_driver* d, int enable);

@@ -152,6 +152,7 @@ _SIGS = {
     "nbl_driver_set_launch": (C.c_int, [C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint32]),
     "nbl_driver_set_graph": (C.c_int, [C.c_void_p, C.c_int]),
     "nbl_driver_set_cascade": (C.c_int, [C.c_void_p, C.c_uint32]),
+    "nbl_driver_get_cascade": (C.c_int, [C.c_void_p, _p(C.c_uint32)]),
     "nbl_driver_autotune": (C.c_int, [C.c_void_p, C.c_uint32, _p(TuneResult)]),
     "nbl_driver_add_world": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, _p(C.c_int32)]),
     "nbl_driver_push_world": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint64,

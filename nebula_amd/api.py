@@ -413,11 +413,6 @@ def to_particles(pri: np.ndarray) -> np.ndarray:
 RECORD_SINK = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint64)
 
 
-# run_tally shortens its frames to two iterations at this many particles:
-# the library then takes them 64 to 1024 steps on in each (k_cascade)
-FEW_PARTICLES = 1 << 18
-
-
 class Driver:
     """gpu_driver<scatter_physics<true>, intersect_t, octree<true>>
     (drivers/gpu/gpu_driver.h:56-178), run by libnebula.so."""
@@ -506,6 +501,12 @@ class Driver:
         """Particles in flight up to which an iteration takes them 64 to 1024
         steps on in their waves (0: never; results do not depend on it)."""
         check(lib().nbl_driver_set_cascade(self._h, max_particles))
+
+    def cascade_limit(self) -> int:
+        """The limit of set_cascade, 0 while deposits are on."""
+        n = C.c_uint32()
+        check(lib().nbl_driver_get_cascade(self._h, C.byref(n)))
+        return n.value
 
     def autotune(self, iters_per_trial: int = 4) -> dict:
         """Measured search over the launch configuration on the queued work;
@@ -620,6 +621,7 @@ class Driver:
         frame_no, direction, probe, pending, before = 0, +1, None, None, None
         steps_prev = self.steps()
         self.k_frames = {}  # frames run at each steps-per-launch value
+        few = self.cascade_limit()
 
         def launch_frame():
             if adapt_k:
@@ -629,7 +631,7 @@ class Driver:
             k_now = self.launch["steps_per_launch"]
             self.k_frames[k_now] = self.k_frames.get(k_now, 0) + 1
             # with few particles left an iteration takes them many steps on
-            self.do_iteration(frame if left > FEW_PARTICLES else min(frame, 2))
+            self.do_iteration(frame if left > few else min(frame, 2))
             return time.perf_counter()
 
         # Each frame's records are tallied on the GPU before the next frame;

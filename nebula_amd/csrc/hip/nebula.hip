@@ -3328,6 +3328,21 @@ int nbl_driver_set_cascade(nbl_driver* d, uint32_t max_particles)
 }
 
 namespace {
+// Particles in flight up to which the iterations of a call of several are
+// k_cascade's: none with deposits (nbl_driver_iterate).
+uint32_t cascade_limit(const nbl_driver* d) { return d->dep ? 0u : d->few; }
+} // namespace
+
+int nbl_driver_get_cascade(nbl_driver* d, uint32_t* max_particles)
+{
+	clear_error();
+	if (!d || !max_particles)
+		return fail(NBL_ERR_ARG, "null argument");
+	*max_particles = cascade_limit(d);
+	return NBL_OK;
+}
+
+namespace {
 // The spill stack holds secondaries that found no room in the particle
 // buffer.  Deep cascades (keV primaries make hundreds of secondaries each)
 // can fill it, and a particle whose secondary finds no room anywhere waits:
@@ -3602,7 +3617,7 @@ int run_loop(nbl_driver* d, bool with_scores, uint32_t frame_iters, const Record
 			}
 			last_steps = total_steps(*d->h_ctrl);
 			if (!frame_iters)
-				frame = running + queued <= d->few ? 2 : std::min<uint32_t>(frame * 2, 32);
+				frame = running + queued <= cascade_limit(d) ? 2 : std::min<uint32_t>(frame * 2, 32);
 			if ((rc = nbl_driver_iterate(d, frame)))
 				return rc;
 		}

@@ -54,6 +54,44 @@ def test_a_first_flight_of_many_cells_is_progress(world, x, y, tally):
     d.close()
 
 
+def _frames(launches, first, most):
+    """The frames of `launches` iterations, of `first` growing to `most`."""
+    out = []
+    while launches > 0:
+        out.append(min(first, most))
+        launches -= out[-1]
+        first *= 2
+    return out if launches == 0 else None
+
+
+@pytest.mark.parametrize("why", ["off", "deposits"])
+@pytest.mark.parametrize("entry", ["tally", "run"])
+def test_frames_stay_long_where_launches_are_short(world, why, entry):
+    """A frame is cut to two iterations where these run many steps each, and
+    not where the caller, or deposits, keep them at steps_per_launch."""
+    dev, mats, geom, _ = world
+    n = 2000
+    pri = W.raster_scan(n, 1, 1, 300.0, -60.0, 60.0, -60.0, 60.0, 37.0, seed=2)
+    print(why, entry, flush=True)
+    d = A.Driver(dev, 4096, geom, mats, seed=8, steps_per_launch=4)
+    d.set_timing(True)
+    if why == "deposits":
+        d.set_deposits(True)
+    else:
+        d.set_cascade(0)
+    d.push(pri, np.arange(n, dtype=np.uint32))
+    if entry == "tally":
+        d.run_tally(np.zeros(n, np.int64), 1, frame=32)
+        launches = d.timing()[1]
+        assert launches == 32 * sum(d.k_frames.values())
+    else:
+        d.run(40 * n)
+        launches = d.timing()[1]
+        assert _frames(launches, 4, 32), launches
+    assert launches > 28
+    d.close()
+
+
 def test_the_tuner_measures_short_launches(world):
     """All electrons fly after the first trial, which ends the search: two
     trials of one launch of four steps."""
