@@ -597,8 +597,8 @@ class Driver:
         counts[bin, 1] = the others (BSE), binned by tag_bin[tag].  The
         detected buffer is tallied after every `frame` iterations (fewer
         once few particles are left), on the GPU (k_tally) unless `tag_bin`
-        is no plain array of integers or far longer than what is to be
-        tracked: then the records are copied out and tallied here.  With
+        is no plain array of integers, far longer than what is to be
+        tracked or too long for the GPU's memory: then the records are copied out and tallied here.  With
         progress_s > 0 a progress line goes to stderr that often.
 
         adapt_k: follow the best steps per launch as the run goes on.  The
@@ -645,7 +645,10 @@ class Driver:
         if on_gpu:
             # while the first frame runs
             bins = np.ascontiguousarray(tag_bin, np.int64)
-            check(lib().nbl_driver_tally_begin(self._h, ptr(bins), len(bins), n_bins))
+            rc = lib().nbl_driver_tally_begin(self._h, ptr(bins), len(bins), n_bins)
+            on_gpu = rc != _lib.NBL_ERR_ALLOC   # no room on the card: the host's
+        if on_gpu:
+            check(rc)
             # a Python number is compared as float32, like the records' energies
             cutoff = float(np.float32(se_cutoff)) if type(se_cutoff) in (int, float) else float(se_cutoff)
             bad = C.c_uint32()

@@ -6,7 +6,7 @@ that name no bin for a record."""
 import numpy as np
 import pytest
 
-from nebula_amd import api as A
+from nebula_amd import _lib, api as A
 from nebula_amd import workloads as W
 from tests.helpers import grating_tris, material
 
@@ -86,3 +86,11 @@ def test_tally_of_no_bins():
     d.push(pri, tags)
     assert d.run_tally(np.zeros(len(pri), np.int64), 1).sum() > 0
     d.close()
+
+
+def test_tally_without_memory_for_it_is_done_on_the_host(setup, monkeypatch):
+    d, pri, tags, rec = setup
+    monkeypatch.setattr(A.lib(), "nbl_driver_tally_begin", lambda *a: _lib.NBL_ERR_ALLOC)
+    table = np.arange(N) % 5
+    d.push(pri, tags)
+    assert np.array_equal(d.run_tally(table, 5), _want(rec, table, 5, 50.0))
