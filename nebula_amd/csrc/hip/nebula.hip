@@ -1994,7 +1994,7 @@ struct nbl_geometry {
 	nbl_device* dev;
 	int* od;
 	float4* tris;
-	float4* scr;
+	ScreenRec* scr;
 	float4* cells;
 	uint32_t* next;
 	uint32_t* start;
@@ -2358,24 +2358,13 @@ int nbl_device_synchronize(nbl_device* d)
 	return NBL_OK;
 }
 
-// |e1|_1 |e2|_1 in the upper 16 bits of a float, rounded up, and the safety
-// bound's factor (pair_safety) in those of another, rounded down; 0, no
-// safety, where it is no ordinary number.
-static float screen_word(float ee, float nx, float ny, float nz)
+// The safety bound's factor (pair_safety); 0, no safety, where it is no
+// ordinary number.
+static float safety_factor(float ee, float nx, float ny, float nz)
 {
-	uint32_t e, r;
-	std::memcpy(&e, &ee, 4);
-	e = (ee == ee && e < 0x7f7f0000u) ? (e + 0xffffu) & 0xffff0000u : 0x7f800000u;
-	std::memcpy(&ee, &e, 4);
 	const double norm = std::sqrt((double)nx * nx + (double)ny * ny + (double)nz * nz);
-	const float rden = (float)(0.9998 / (norm * 1.0001 + 1e-5 * (double)ee));
-	std::memcpy(&r, &rden, 4);
-	if (!(rden > 1e-30f && rden < 1e30f))
-		r = 0;
-	const uint32_t w = e | (r >> 16);
-	float f;
-	std::memcpy(&f, &w, 4);
-	return f;
+	const float rden = (float)(0.9999 / (norm * 1.0001 + 1e-5 * (double)ee));
+	return (rden > 1e-30f && rden < 1e30f) ? rden : 0.0f;
 }
 
 int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const nbl_triangle44* tris,
@@ -2444,7 +2433,7 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 			return fail(NBL_ERR_ARG, "triangle " + std::to_string(i) + ": material id outside the 16-bit range");
 		}
 	if ((rc = dev_alloc(&g->od, (size_t)n_od)) || (rc = dev_alloc(&g->tris, (size_t)ntri * 3))
-		|| (rc = dev_alloc(&g->scr, (size_t)n_od * 2)) || (rc = dev_alloc(&g->cells, cells.rec.size()))
+		|| (rc = dev_alloc(&g->scr, (size_t)n_od)) || (rc = dev_alloc(&g->cells, cells.rec.size()))
 		|| (rc = dev_alloc(&g->next, cells.next.size())) || (rc = dev_alloc(&g->start, cells.start.size()))) {
 		hipFree(g->od);
 		hipFree(g->tris);
@@ -2454,7 +2443,8 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 		delete g;
 		return rc;
 	}
-	std::vector<float4> packed((size_t)ntri * 3), tscr((size_t)ntri * 2);
+	std::vector<float4> packed((size_t)ntri * 3);
+	std::vector<ScreenRec> tscr((size_t)ntri);
 	for (int64_t i = 0; i < ntri; ++i) {
 		const nbl_triangle44& t = tris[i];
 		float ib, ob;
@@ -2471,23 +2461,19 @@ int nbl_geometry_upload(nbl_device* dev, const int32_t* od, int64_t n_od, const 
 		const float l1 = std::fabs(t.e1[0]) + std::fabs(t.e1[1]) + std::fabs(t.e1[2]);
 		const float l2 = std::fabs(t.e2[0]) + std::fabs(t.e2[1]) + std::fabs(t.e2[2]);
 		const uint32_t mats = ((uint32_t)t.material_in & 0xffffu) | ((uint32_t)t.material_out << 16);
-		float mf;
-		std::memcpy(&mf, &mats, 4);
-		tscr[2 * i] = make_float4(t.r0[0], t.r0[1], t.r0[2], screen_word(l1 * l2, nx, ny, nz));
-		tscr[2 * i + 1] = make_float4(nx, ny, nz, mf);
+		tscr[i] = { (int32_t)i, safety_factor(l1 * l2, nx, ny, nz), { t.r0[0], t.r0[1], t.r0[2] }, l1 * l2,
+			{ nx, ny, nz }, mats };
 	}
 	// the screening records in table order: every entry that names a
 	// triangle (list entries; node offsets that happen to be below ntri get a
 	// record nobody reads)
-	std::vector<float4> scr((size_t)n_od * 2, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+	std::vector<ScreenRec> scr((size_t)n_od, ScreenRec{});
 	for (int64_t i = 0; i < n_od; ++i)
-		if (od[i] >= 0 && od[i] < ntri) {
-			scr[2 * i] = tscr[2 * (size_t)od[i]];
-			scr[2 * i + 1] = tscr[2 * (size_t)od[i] + 1];
-		}
+		if (od[i] >= 0 && od[i] < ntri)
+			scr[i] = tscr[od[i]];
 	HIP_OK(hipMemcpy(g->od, od, sizeof(int32_t) * n_od, hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->tris, packed.data(), sizeof(float4) * packed.size(), hipMemcpyHostToDevice));
-	HIP_OK(hipMemcpy(g->scr, scr.data(), sizeof(float4) * scr.size(), hipMemcpyHostToDevice));
+	HIP_OK(hipMemcpy(g->scr, scr.data(), sizeof(ScreenRec) * scr.size(), hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->cells, cells.rec.data(), sizeof(float4) * cells.rec.size(), hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->next, cells.next.data(), sizeof(uint32_t) * cells.next.size(), hipMemcpyHostToDevice));
 	HIP_OK(hipMemcpy(g->start, cells.start.data(), sizeof(uint32_t) * cells.start.size(), hipMemcpyHostToDevice));
