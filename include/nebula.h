@@ -210,8 +210,13 @@ int nbl_material_destroy(nbl_material* m);
 
 /* gpu_driver ctor (drivers/gpu/gpu_driver.inl:51-89).  capacity = target
  * number of particles in flight; steps_per_launch = steps each particle takes
- * per kernel launch (more when few are in flight, nbl_driver_set_cascade).  The driver keeps its own copies of geometry and
- * material descriptors (the objects must outlive it). */
+ * per kernel launch (more when few are in flight, nbl_driver_set_cascade).
+ * The driver keeps its own copies of geometry and material descriptors (the
+ * objects must outlive it).  Device memory for each particle in flight aimed
+ * for: 1408 bytes of particle buffers, queue and spill stack, 96 more for
+ * walks kept between launches (capacities of 2^15 to 2^25), 40 of records.
+ * Drivers with more than 64 materials, in any one world, run kernels that
+ * keep no material on the compute unit and skip no walk. */
 int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* geom,
 	const nbl_material* const* mats, int32_t n_mats, uint32_t physics_flags,
 	float energy_threshold, uint64_t seed, uint32_t steps_per_launch, nbl_driver** out);
@@ -246,9 +251,10 @@ int nbl_driver_iterate(nbl_driver* d, uint32_t n_iter);
  * changes the electron's energy: position after the event, energy before
  * it, energy lost, tag of the primary, stream id of the electron.  Enable
  * before tracking; an iteration can write up to (K + 1) records per
- * particle in flight (half the buffer, if it is the only one since a drain
- * and few particles are in flight), so drain after every nbl_driver_iterate
- * call (a drain that finds records were dropped returns NBL_ERR_CAPACITY). */
+ * particle in flight (half the buffer and what its last steps add, if it is
+ * the only one since a drain and few particles are in flight), so drain after
+ * every nbl_driver_iterate call (a drain that finds records were dropped
+ * returns NBL_ERR_CAPACITY). */
 typedef struct {
 	float pos[3];
 	float energy;
@@ -348,7 +354,7 @@ void* nbl_driver_stream(nbl_driver* d);
  * detection order); *n_detected and *steps (particle-steps) are host
  * outputs.  The library allocates nothing: particle buffers, inelastic
  * queue, spill stack, control block and material descriptors live in one
- * fixed device array of 49 MiB (51 398 656 bytes) per GPU, held until the process ends and
+ * fixed device array of 56 MiB (58 741 248 bytes) per GPU, held until the process ends and
  * shared by every call on that GPU (calls that overlap on one GPU race).
  * Limits: capacity (particles in flight) in [64, 65536], at most 64
  * materials (NBL_ERR_CAPACITY otherwise); the spill stack holds 2^19
@@ -466,7 +472,9 @@ int nbl_driver_get_material_params(nbl_driver* d, int32_t material, float* el_mf
 
 /* Enable scores for n (<= 8) parameters (materials[i], kinds[i]), or
  * disable with n = 0.  Only while nothing is in flight, queued or waiting
- * to be drained (NBL_ERR_ARG otherwise); primaries start with score 0. */
+ * to be drained (NBL_ERR_ARG otherwise); primaries start with score 0.  The
+ * score arrays stay with the driver while scores are off, up to 2 GiB of
+ * them. */
 int nbl_driver_set_score_params(nbl_driver* d, const int32_t* materials, const int32_t* kinds,
 	int32_t n);
 

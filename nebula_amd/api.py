@@ -467,7 +467,9 @@ class Driver:
 
     def run_with_deposits(self, cap: int):
         """Track everything pushed to the end, one iteration at a time,
-        draining deposits after each: (detected, deposits)."""
+        draining deposits after each: (detected, deposits).  The deposits
+        are a part of the array they were gathered in, which may be larger;
+        copy them to let its unused room go."""
         dets = []
         # One array for all deposits, grown by doubling: room that is not used
         # yet is not committed, and joining an array per iteration at the end

@@ -7,12 +7,17 @@
 // [slots - n_se, slots).  A launch of k_step moves every particle through up
 // to K steps (init + event each), then appends it to the other buffer:
 // survivors from the front (wavefront ballots + prefix popcounts; one atomic
-// per block, per wave in the general variant), new secondaries from the back (made by k_inel, one atomic per
-// block).  Dead particles
+// per block, per wave in the general variant), new secondaries from the back
+// (made by k_inel, one atomic per block).  Dead particles
 // are simply not copied, so the next launch reads a dense range.  A
 // one-thread control kernel adopts the output counts and plans the refill of
 // primaries from a device-resident queue; all sizes live in device memory, so
 // an iteration never waits for the host.
+//
+// Times in these files are of one MI355X.  Two times of a case were taken
+// with each other when the choice they stand for was made, with the kernels of
+// that time; "the full image" (6 553 600 primaries of 300 eV on a grating, 2^22
+// in flight, 6 steps a launch) takes 184 ms with the present ones.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,7 +43,7 @@ using namespace nbl::dev;
 // triangle, tag, step, flags; stream id, safety, 4 bytes unused.  A wave's
 // particles are four wide loads or stores within a page or two.  (As an array
 // a field they were 15 narrow ones with an address each, each in a page of its
-// own: of the full image k_inel took 29.3 ms, now 27.8, k_step 205 and 203.)
+// own: of the full image k_inel 29.3 -> 27.8 ms, k_step 205 -> 203.)
 struct Bufs {
 	char* base;
 	double* sc;             // scores, [parameter][entry], or null
@@ -346,7 +351,7 @@ __device__ __forceinline__ uint32_t in_slot(uint32_t i, uint32_t n_surv, uint32_
 // each block's place within its world's range, so the placing pass needs no
 // counting and no atomics in memory.  (With counters in memory, 1024 blocks'
 // atomics on the few of the worlds in flight serialised in L2: the three took
-// 86 us a launch for six scans of 294 720 primaries in all, now 17.)
+// 86 us a launch for six scans of 294 720 primaries in all, these 17.)
 // Worlds beyond NW_LDS are counted and placed with one atomic per world
 // present in a wave instead.
 constexpr uint32_t NW_LDS = 1024, WG_BLOCKS = 256, WG_THREADS = 1024;
@@ -642,9 +647,9 @@ __device__ __forceinline__ bool place_secondary(const StepArgs& a, const Bufs& o
 // particle up to K times, stopping early when it leaves (detected,
 // terminated, inelastic event), and writes it out once: detected record,
 // inelastic queue or survivor buffer, with one ballot per kind and one
-// atomic per wave for the last two together.  The wave steps in lockstep because the octree walk is
-// shared across it (propagate_wave): a lane whose particle has stopped still
-// tests triangles for the others.  (Lanes that took new work after every step
+// atomic per block and counter (emit_block).  The wave steps in lockstep
+// because the octree walk is shared across it (walk_round): a lane whose
+// particle has stopped still tests triangles for the others.  (Lanes that took new work after every step
 // or every few steps were measured slower: the extra ballots and atomics cost
 // more than the idle lanes they saved; so did lanes that kept a stopped
 // particle until half the wave was idle and then refilled together from the
@@ -654,6 +659,11 @@ __device__ __forceinline__ bool place_secondary(const StepArgs& a, const Bufs& o
 // race and boundary choices) and write it with the particle.
 // MULTI: particles belong to different worlds (flags bits 16..31); each lane
 // takes its particle's geometry and materials from the world table.
+// WUNI: several worlds, one per wave, of particles grouped by world
+// (k_world_place): geometry and materials are wave-uniform, so the plain
+// kernel's shared walk, walk skip and register budget apply.
+// DEP: one world, with energy deposits.
+
 // An energy-deposit record (energydeposit_cpu_driver.h:55-66): position
 // after the event, energy before, energy lost; slots by ballot + atomic.
 __device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, const Particle& p, uint32_t tag,
@@ -673,8 +683,8 @@ __device__ __forceinline__ void deposit(const StepArgs& a, Ctrl* C, bool rec, co
 
 // Records of a wave of k_cascade, gathered in LDS and written together: 2048
 // primaries of 1 keV make 3.4 M records, and with an atomic and a look at the
-// counter each turn their launches waited for that one address (23.0 ms of
-// k_cascade, now 3.4).
+// counter each turn their launches waited for that one address (k_cascade
+// 23.0 -> 3.4 ms).
 struct DepStage {
 	nbl_deposit* at;   // 64 records
 	uint32_t n;
@@ -720,12 +730,6 @@ __device__ __forceinline__ void stage_deposit(const StepArgs& a, Ctrl* C, DepSta
 	st.n += c;
 }
 
-// WUNI: several worlds, one per wave.  A wave steps the particles of its
-// first lane's world (its geometry and materials are wave-uniform, so the
-// plain kernel's shared walk, walk skip and register budget apply); lanes
-// holding another world's particle wait, unchanged, for a later launch.
-// Trajectories depend only on each particle's own stream, so which launch
-// steps a particle changes no result.
 __device__ __forceinline__ void store_detected(const StepArgs& a, uint32_t slot, const State& s)
 {
 	nbl_detected r;
@@ -985,8 +989,8 @@ __device__ __forceinline__ void emit(const StepArgs& a, Ctrl* C, uint32_t out_bu
 // (every thread calls).  All atomics of a launch on one counter are served one
 // after the other, beyond the L2s (each XCD has its own), at 12 ns each: with
 // two or three for each of the 67 000 waves of a launch of 4.2 million
-// particles, the counters took most of the launch (the full image 239 ms, now
-// 200; blocks of 2 waves 209, of 8 205).  A wave waits for the block's others,
+// particles, the counters took most of the launch (the full image 239 -> 200
+// ms; blocks of 2 waves 209, of 8 205).  A wave waits for the block's others,
 // which are as long on their way (K turns).
 template <bool SC, uint32_t WAVES>
 __device__ __forceinline__ void emit_block(const StepArgs& a, Ctrl* C, uint32_t out_buf, State& s, const ScoreLds& sc,
@@ -1284,10 +1288,10 @@ __device__ __forceinline__ void step_multi(const StepArgs& a)
 	count_steps(C, my_steps);
 }
 
-// The plain variant runs at 6 waves per SIMD: 74 VGPRs, and 25.9 KB of LDS a
+// The plain variant runs at 6 waves per SIMD: 70 VGPRs, and 25.9 KB of LDS a
 // block with the materials beside it (6 blocks of a compute unit's 160 KB).
 // With its state in registers (93 VGPRs, 5 waves) the full image took 254 ms,
-// 273 at 4 waves and 316 at 3.
+// 273 at 4 waves and 316 at 3; with state and materials in LDS 244 (WaveMem).
 #ifndef NBL_PLAIN_WAVES
 #define NBL_PLAIN_WAVES 5
 #endif
@@ -1321,9 +1325,9 @@ void k_step<false, false, true, false>(StepArgs a)
 // survivor slot surv0 + i with no atomic.  Secondary slots are counted per
 // block (ballot per wave, the counts in LDS, one atomic per block, and one more
 // when some go to the spill stack): atomics on one counter are served one
-// after the other (emit_block).  Blocks of 512: the full image in 191.8 ms,
-// 194.6 with 256, 197.0 with 1024; 201 with 256 and an atomic a wave on the
-// spill stack.  The block loop runs whole blocks, so every thread reaches each
+// after the other (emit_block).  The full image 201 ms with blocks of 256 and an
+// atomic a wave on the spill stack; with one a block 194.6, 191.8 with blocks
+// of 512 and 197.0 with 1024.  The block loop runs whole blocks, so every thread reaches each
 // barrier.
 constexpr uint32_t INEL_THREADS = 512;
 template <bool SC, bool MULTI>
@@ -1542,7 +1546,7 @@ __device__ __forceinline__ void cascade_body(const StepArgs& a)
 			const uint64_t live = ballot(occ && !park);
 			if (live == 0ull)
 				break;
-			// stop while every wave still has room for 64 records in the first
+			// Stop while every wave still has room for 64 records in the first
 			// half of the buffer; what a turn writes beyond them (a particle
 			// can have two events in it) fits the second half
 			// (one world: a wave gathers up to 64 records and learns the
@@ -1795,10 +1799,10 @@ __global__ void k_reset_det(Ctrl* c)
 //
 // Bound by reading the records (40 bytes each) and one atomic a record.  The
 // records' way to the host, through pageable memory with the GPU idle, and the
-// host's count of the last frame took 16 of 271 ms for 6 553 600 primaries of
-// 300 eV (now 255), 0.4 of 10.4 ms for 96 903 of 500 eV.  With few bins (a
-// batch counts one a scan) a launch's atomics would all meet on a few lines of
-// L2, so a block counts in LDS first, as long as the counters fit 16 KB.
+// host's count of the last frame took 16 of 271 ms of the full image, 0.4 of
+// 10.4 ms for 96 903 primaries of 500 eV.  With few bins (a batch counts one a
+// scan) a launch's atomics would all meet on a few lines of L2, so a block
+// counts in LDS first, as long as the counters fit 16 KB.
 constexpr uint32_t TALLY_LDS = 4096;
 __global__ __launch_bounds__(256) void k_tally(Ctrl* c, const nbl_detected* __restrict__ det, uint32_t det_cap,
 	const int64_t* __restrict__ bin, uint64_t n_tags, uint64_t n_bins, double cutoff,
@@ -2079,10 +2083,15 @@ namespace {
 
 // Waves of a k_cascade launch, and the particles in flight up to which a
 // launch is k_cascade's.
-// 16 waves a compute unit are all resident (at most 125 VGPRs); up to 1024 particles
-// a compute unit they hold every particle (512: 13.3 against 12.9 ms for
-// 96 903 primaries of 500 eV on a grating, 27.0 against 25.8 ms for 160 000
-// of 1 keV on contact holes; 1536, waves taking two turns: 13.7 and 26.0).
+// 16 waves a compute unit are all resident (at most 125 VGPRs; the scored
+// kernel's LDS admits 15); up to 1024 particles a compute unit they hold every
+// particle.  A limit of 512 a compute unit, 256 and none: 7.10, 7.30 and 9.3
+// against 6.9 ms for 96 903 primaries of 500 eV on a grating; one world a wave,
+// six scans of 294 720 primaries 19.6, 19.6 and 21.1 against 19.5, of 9 824
+// 3.56, 4.02 and 7.9 against 3.56; with scores, yield and Jacobian of 249 856
+// primaries 33.6, 33.6 and 36.4 against 34.1, of 49 152 10.3, 10.4 and 15.1
+// against 10.4.  (1536, waves taking two turns, in an earlier build: 13.7
+// against 12.9 for the first.)
 uint32_t cascade_waves(const nbl_device* dev) { return 16u * (uint32_t)dev->n_cu; }
 uint32_t cascade_max(const nbl_device* dev) { return 64u * cascade_waves(dev); }
 
@@ -2725,7 +2734,7 @@ int nbl_driver_create(nbl_device* dev, uint32_t capacity, const nbl_geometry* ge
 			d->walk[1] = p + 3 * b + w;
 		}
 	}
-	// The spill stack starts at eight buffers' worth (60 bytes a slot: 2 GB
+	// The spill stack starts at eight buffers' worth (64 bytes a slot: 2 GB
 	// at 2^22 slots) and doubles when needed.  A scan of 300 eV primaries
 	// filling 2^22 slots spills more than twice the buffer in its first
 	// iterations; each doubling costs a copy and a reallocation with the

@@ -76,7 +76,8 @@ constexpr float PF_TWO_OVER_PI = 0x1.45f306p-1f, PF_TAN_PI_8 = 0x1.a8279ap-2f;
 // exponential, phase and table index below and one Philox block a step instead
 // of one more for boundary events, the step kernel issues 18 % fewer VALU
 // instructions: 6 553 600 primaries of 300 eV 288 -> 277 ms, 100 of 1 keV in a
-// slab 1.92 -> 1.75.
+// slab 1.92 -> 1.75.  (What the tests repeat is whole steps, bit for bit, with
+// operands in the ranges and outside them.)
 //
 // 1 / x, |x| in [2^-100, 2^100].
 __device__ __forceinline__ float rcp_mid(float x)
@@ -801,8 +802,8 @@ constexpr int MAX_DEPTH = 21;
 // the centres as the reference does), and a move to the next cell reads one
 // entry.  (With descents of seven levels from the root for every walk and
 // the centre added up again for every further cell: 6 553 600 primaries of
-// 300 eV on a grating 294 ms, now 288; 160 000 of 1 keV on contact holes 21.5
-// and 21.0; 2046 of 300 eV 1.72 and 1.68.)
+// 300 eV on a grating 294 ms, with the tables 288; 160 000 of 1 keV on contact
+// holes 21.5 and 21.0; 2046 of 300 eV 1.72 and 1.68.)
 //
 // cell_start: the cell in which a walk from `p` begins its descent.
 __device__ __forceinline__ uint32_t cell_start(const Geometry& g, F3 p)
@@ -1243,7 +1244,8 @@ __device__ __forceinline__ int walk_round(const Geometry& g, bool active, WaveMe
 }
 
 // The whole walk for the rays of a wave (every lane calls; lanes with walk ==
-// false take part in the shared tests only).
+// false take part in the shared tests only).  The query hook's: the step
+// kernels call walk_round themselves.
 __device__ inline int propagate_wave(const Geometry& g, bool walk, F3 start, F3 dir, float distance,
 	int ignore_tri, int ignore_mat, float& out_dist, WaveMem& m)
 {
