@@ -462,8 +462,8 @@ def main():
     ap.add_argument("--capacity", type=int, default=1 << 22,
                     help="particles in flight (2^22 measured fastest on the scan: 2^21 1.8 %% slower)")
     ap.add_argument("--steps-per-launch", type=int, default=6,
-                    help="steps per particle per launch (the scan takes 191 ms at 5 and "
-                         "6, 193 at 4, 196 at 8)")
+                    help="steps per particle per launch (the scan takes 182 ms at 5, 183 "
+                         "at 6, 184 at 4, 188 at 8)")
     ap.add_argument("--blocks-per-cu", type=int, default=0,
                     help="step-kernel blocks of 256 per compute unit (0: the library's default, 64)")
     ap.add_argument("--pixels", type=int, default=256)
